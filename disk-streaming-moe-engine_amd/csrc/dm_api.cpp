@@ -74,6 +74,7 @@ struct GgufLayer {
   int grid = 0;
   unsigned launches = 0;
   float* rchain = nullptr;  // the router in chain order (dev.rchain)
+  uint8_t* tiles = nullptr; // the experts in matrix-core records (dev.tiles)
 };
 
 void free_glayer(GgufLayer* G) {
@@ -81,6 +82,7 @@ void free_glayer(GgufLayer* G) {
   if (G->buf) (void)hipFree(G->buf);
   if (G->sync) (void)hipFree(G->sync);
   if (G->rchain) (void)hipFree(G->rchain);
+  if (G->tiles) (void)hipFree(G->tiles);
   delete G;
 }
 
@@ -177,6 +179,9 @@ struct dmh_ctx {
   DevBuf<uint16_t> g_xhi, g_xlo;
   DevBuf<uint16_t> g_hr, g_hs;  // bf16 hi parts, then lo parts
   DevBuf<float> g_r, g_rs;
+  // GGUF layers on the matrix cores: exponents and column sums of x and h
+  DevBuf<int32_t> g_ex;
+  DevBuf<uint16_t> g_sums;
   std::vector<GgufLayer*> glayers;
   unsigned long long* status = nullptr;  // [kStatusSlots] first-error keys
   // status_clean[l]: slot l holds no error and nothing has run on it since
@@ -636,7 +641,8 @@ GgufLayer* get_glayer(dmh_ctx* c, int layer) {
 // otherwise router and shared-gate logits (fp32 weights, router_forward's
 // order), selection and gate, then from kGgufGroupMinT tokens on the
 // grouping by expert and the grouped gate/up, down and combine launches
-// (dm::launch_gguf_units), below it gate/up of every (token, slot) and the
+// (dm::launch_gguf_units; from kGgufMmMinT tokens on dm::launch_gguf_mm on
+// layers with matrix-core records), below it gate/up of every (token, slot) and the
 // down projections with moe_aggregate_forward.
 // The grouped several-token form: from 128 tokens on (below, the units hold
 // one or two tokens and the grid sized for the most units there could be
@@ -695,6 +701,24 @@ hipError_t run_gguf_block(dmh_ctx* c, GgufLayer* G, unsigned long long* status, 
     if ((e = dm::launch_group_build(dids, T, L.K, L.E, c->g_off.p, c->g_perm.p, c->g_units.p,
                                     c->g_meta.p, st)) != hipSuccess)
       return e;
+    if (dm::gguf_mm_ok(L, T)) {
+      // prefill: the experts' products on the matrix cores
+      const size_t TK = (size_t)T * L.K, TH = (size_t)T * L.H;
+      const size_t hn = TK * L.I + (size_t)T * L.Ish;
+      const size_t xsum = dm::gguf_mm_sums(L, (int64_t)TH);
+      if ((e = c->g_xhi.ensure(2 * TH)) != hipSuccess) return e;
+      if ((e = c->g_hr.ensure(2 * hn)) != hipSuccess) return e;
+      if ((e = c->g_ex.ensure(T + TK + T)) != hipSuccess) return e;
+      if ((e = c->g_sums.ensure(xsum + dm::gguf_mm_sums(L, (int64_t)hn) + 1)) != hipSuccess)
+        return e;
+      const dm::GgufMmScratch s{c->g_xhi.p,  c->g_hr.p,           c->g_ex.p,
+                                c->g_sums.p, c->g_sums.p + xsum, c->h.p};
+      float* rs = c->g_r.p + TK * L.H;
+      if ((e = dm::launch_gguf_mm(L, dx, T, c->g_off.p, c->g_perm.p, c->g_units.p, c->g_meta.p,
+                                  nu, s, c->g_r.p, rs, status, st)) != hipSuccess)
+        return e;
+      return dm::launch_combine(c->g_r.p, rs, dprobs, dshg, dres, T, L.H, L.K, dy, status, st);
+    }
     return dm::launch_gguf_units(L, dx, T, c->g_off.p, c->g_perm.p, c->g_units.p, c->g_meta.p, nu,
                                  c->h.p, ldh, c->g_r.p, dprobs, dshg, dres, dy, status, st);
   }
@@ -1988,6 +2012,18 @@ static int upload_gguf_body(dmh_ctx* c, int layer, const dmh_moe_dims* d,
         if (G->rchain) (void)hipFree(G->rchain);
         G->rchain = nullptr;
       }
+    }
+  }
+  // the matrix-core form of the experts; without room for it, calls of many
+  // tokens keep the grouped form on the payload
+  if (const size_t nt = dm::gguf_tiles_bytes(G->dev)) {
+    if (hipMalloc(&G->tiles, nt) == hipSuccess &&
+        dm::launch_gguf_tiles(G->dev, G->tiles, st) == hipSuccess &&
+        hipStreamSynchronize(st) == hipSuccess) {
+      G->dev.tiles = G->tiles;
+    } else {
+      if (G->tiles) (void)hipFree(G->tiles);
+      G->tiles = nullptr;
     }
   }
   if (GgufLayer* old = c->glayers[layer]) {

@@ -42,6 +42,7 @@ struct GgufMoeDev {
   const float* shgate; // [H]
   int64_t estride;     // > 0: off[3e + k] = (3e + k) * estride for the routed experts (else 0)
   const float* rchain; // [E + 1][H] router and shared gate in chain order (one-token form), or null
+  const uint8_t* tiles;  // the experts in matrix-core records (launch_gguf_tiles), or null
 };
 
 // h[t][s][i] = SiLU(W_gate x_t)_i * (W_up x_t)_i for slots s < K (expert
@@ -70,6 +71,37 @@ hipError_t launch_gguf_units(const GgufMoeDev& L, const float* x, int T, const i
                              int nunits, float* h, int ldh, float* parts, const float* probs,
                              const float* shg, const float* residual, float* y,
                              unsigned long long* status, hipStream_t st);
+
+// ---- many tokens on the matrix cores (dm_gguf_mm.hip) ------------------------
+// Bytes of the experts' matrix-core records; 0 when the layer has no such
+// form (Q3_K, Q4_K and Q8_0 experts with H, I and Ish multiples of 128, so
+// that 128 columns of a row lie in one block, have it).
+size_t gguf_tiles_bytes(const GgufMoeDev& L);
+// The records of L's experts into out (16-byte aligned).
+hipError_t launch_gguf_tiles(const GgufMoeDev& L, uint8_t* out, hipStream_t st);
+// Fewest tokens of the matrix-core form.  Below, a call gives every token
+// the bits of its own single-token call, whatever it is batched with; from
+// here on the sums run in the matrix cores' order (as exact, other bits).
+constexpr int kGgufMmMinT = 256;
+bool gguf_mm_ok(const GgufMoeDev& L, int T);
+// Elements of the column sums of `elements` activations (0: not needed).
+size_t gguf_mm_sums(const GgufMoeDev& L, int64_t elements);
+struct GgufMmScratch {
+  uint16_t* xs;    // [T][H][2] x in f16 parts
+  uint16_t* hs;    // [T K][I][2], [T][Ish][2] h in f16 parts
+  int32_t* ex;     // [T] exponents of x, [T K + T] of h
+  uint16_t* xsum;  // gguf_mm_sums(T H) column sums of x
+  uint16_t* hsum;  // gguf_mm_sums(T K I + T Ish) of h
+  float* h;        // [T K][I], [T][Ish]
+};
+// The experts' outputs of T tokens grouped by expert (off, perm, units, meta
+// of launch_group_build, nunits = group_units_max): r [T*K][H] by
+// assignment, rs [T][H] of the shared expert, unweighted, with the checks of
+// launch_gguf_units; launch_combine forms y from them.
+hipError_t launch_gguf_mm(const GgufMoeDev& L, const float* x, int T, const int32_t* off,
+                          const int32_t* perm, const int2* units, const int32_t* meta, int nunits,
+                          const GgufMmScratch& s, float* r, float* rs, unsigned long long* status,
+                          hipStream_t st);
 
 // One token in one launch of grid workgroups of 512 threads that must all
 // be resident (gguf_experts_occupancy >= 1 per CU, gguf_one_token_grid_ok):

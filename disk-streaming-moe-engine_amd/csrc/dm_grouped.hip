@@ -954,9 +954,7 @@ static hipError_t big_attrs() {
   return e;
 }
 
-// Persistent big workgroups of this device: its CU count rounded down to a
-// multiple of 8 (0 when it cannot be read).
-static int big_persistent_wgs() {
+int persistent_wgs() {
   static std::atomic<int> cus[64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
@@ -1159,7 +1157,7 @@ hipError_t launch_experts_grouped(const LayerDev& L, const uint16_t* xhi, const 
     // persistent big workgroups: one per CU (150 KB of LDS each), a multiple
     // of 8 so that an item keeps its class; every item needs two stages or
     // more (gate/up: H / 128 of them, down: 2 I / 128)
-    const int pw = L.H >= 256 ? big_persistent_wgs() : 0;
+    const int pw = L.H >= 256 ? persistent_wgs() : 0;
     const int wg_g = pw > 0 && pw < bg ? pw : bg, wg_d = pw > 0 && pw < bd ? pw : bd;
     hipLaunchKernelGGL(k_big<true>, dim3(wg_g + (nsmall * gy + 1) / 2), dim3(kB2Threads), kB2Lds,
                        st, bg, wg_g, meta, units, off, perm, need_lo, g, nsmall, gy);

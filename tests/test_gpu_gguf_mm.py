@@ -1,0 +1,176 @@
+"""GGUF layers with many tokens per call (from 256 on, experts in Q3_K, Q4_K
+or Q8_0 with hidden, inter and inter_sh multiples of 128): the experts'
+products on the matrix cores, integer codes in f16 against activations in
+two f16 parts.
+
+Reference: the reference's composition on the dequantized weights in float64
+(ids and probabilities of the oracle, which must match bit for bit).  Bar: the
+relative 2-norm error of a token's output stays below 2e-6.  The parts hold
+24 bits of an activation (2^-24 each, in x and again in h), the longest chain
+of fp32 additions is 2048 / 64 matrix instructions for each of hi and lo, and
+random rounding over n additions grows as sqrt(n) 2^-24 = 8 * 6e-8 per
+product; gate, up and down together stay under 4 * 5e-7."""
+import json
+
+import numpy as np
+import pytest
+
+from dismoen import DismoenError, gguf, synth
+
+pytestmark = pytest.mark.gpu
+BAR = 2e-6
+
+
+def _upload(block, tmp_path, slot, dims, ty, mutate=None):
+    H, E, K, I, Ish = dims
+    ts = synth.make_gguf_moe_layer(H, E, I, Ish, seed=slot, expert_type=ty)
+    # logits near one, so that several experts carry weight
+    ts[0] = (*ts[0][:3], synth.gguf_payload(np.random.default_rng(slot), 8, E * H, 1.4e-5))
+    p = str(tmp_path / f"mm{slot}.gguf")
+    gguf.write_gguf(p, mutate(ts) if mutate else ts)
+    g = gguf.parse_gguf_index(p)
+    block.upload_layer_gguf(slot, dims, g)
+    return g
+
+
+def _reference(oracle, g, dims, x, ids, probs, shg):
+    """The block without residual in float64 for the given routing."""
+    H, E, K, I, Ish = dims
+
+    def deq(name, rows, cols):
+        t = g.tensors[g.tensor_map["blk.0." + name]]
+        return oracle.dequant_gguf(t.dtype, g.read_raw("blk.0." + name),
+                                   t.num_elements).astype(np.float64).reshape(rows, cols)
+
+    def ffn(v, gate, up, down, n):
+        a, b = v @ deq(gate, n, H).T, v @ deq(up, n, H).T
+        with np.errstate(over="ignore"):
+            return (a / (1.0 + np.exp(-a)) * b) @ deq(down, H, n).T
+
+    x = x.astype(np.float64)
+    y = shg.astype(np.float64)[:, None] * ffn(x, "ffn_shared_gate.weight", "ffn_shared_up.weight",
+                                              "ffn_shared_down.weight", Ish)
+    for e in np.unique(ids):
+        t, k = np.nonzero(ids == e)
+        y[t] += probs[t, k].astype(np.float64)[:, None] * ffn(
+            x[t], *(f"ffn_{w}.{e}.weight" for w in ("gate", "up", "down")), I)
+    return y
+
+
+def _check(block, oracle, g, slot, dims, x):
+    H, E, K, I, Ish = dims
+    T = x.shape[0]
+    res = np.random.default_rng(T).standard_normal((T, H)).astype(np.float32)
+    y, ids, probs, shg = block.forward_port_moe_gguf(x, None, slot, T)
+    yr, ids2, _, _ = block.forward_port_moe_gguf(x, res, slot, T)
+    t = g.tensors[g.tensor_map["blk.0.ffn_gate_exps.weight"]]
+    w = oracle.dequant_gguf(t.dtype, g.read_raw("blk.0.ffn_gate_exps.weight"), t.num_elements)
+    rid, rp = oracle.router_forward(x, w, T, H, E, K, layer=slot)
+    assert np.array_equal(ids, rid) and np.array_equal(ids2, rid)
+    assert np.array_equal(probs.view(np.uint32), rp.view(np.uint32))
+    ref = _reference(oracle, g, dims, x, ids, probs, shg)
+    err = np.linalg.norm(y - ref, axis=1) / np.maximum(np.linalg.norm(ref, axis=1), 1e-300)
+    print(f"T={T} worst token {err.max():.2e}", flush=True)
+    assert err.max() < BAR, (int(err.argmax()), err.max())
+    # the residual is added last
+    assert np.array_equal(yr.view(np.uint32), (y + res).view(np.uint32))
+    return y, ids
+
+
+@pytest.mark.parametrize("ty", [11, 12, 8])
+@pytest.mark.parametrize("slot,dims,T", [
+    (60, (128, 2, 1, 128, 128), 256),     # two stages a product; full 128-token units
+    (61, (640, 9, 3, 384, 128), 257),     # rows of broken 256-weight blocks; partial row blocks
+    (62, (256, 70, 5, 256, 384), 300),    # units of about 21 tokens: one or two small ones
+    (63, (2048, 16, 8, 512, 512), 333),   # the Qwen3.6 shape
+])
+def test_against_float64(block, oracle, tmp_path, ty, slot, dims, T):
+    g = _upload(block, tmp_path, slot, dims, ty)
+    x = np.random.default_rng(T + ty).standard_normal((T, dims[0])).astype(np.float32)
+    _, ids = _check(block, oracle, g, slot, dims, x)
+    n = np.bincount(ids.reshape(-1), minlength=dims[1])
+    print("tokens per expert", n.min(), n.max(), flush=True)
+    block.free_layer_gguf(slot)
+
+
+def test_unit_sizes(block, oracle, tmp_path):
+    """Experts with 1, 15, 16, 17, 32, 33, 48, 65, 81, 97 and 128 + 1 tokens:
+    every number of column tiles and both sides of the small units."""
+    dims = (256, 11, 1, 128, 128)
+    sizes = [1, 15, 16, 17, 32, 33, 48, 65, 81, 97, 129]
+
+    def route(ts):  # expert e's logit is x[e]
+        blocks = np.zeros((11, 8, 34), np.uint8)
+        blocks[:, :, 0:2] = np.array([1.0], np.float16).view(np.uint8)
+        for e in range(11):
+            blocks[e, 0, 2 + e] = 1
+        return [(*ts[0][:3], blocks.tobytes())] + ts[1:]
+
+    g = _upload(block, tmp_path, 64, dims, 11, route)
+    rng = np.random.default_rng(5)
+    owner = rng.permutation(np.repeat(np.arange(11), sizes))
+    x = rng.standard_normal((owner.size, 256)).astype(np.float32)
+    x[np.arange(owner.size), owner] = 6.0
+    x[:, :11] = np.minimum(x[:, :11], 6.0)
+    _, ids = _check(block, oracle, g, 64, dims, x)
+    assert np.array_equal(np.bincount(ids.reshape(-1), minlength=11), sizes)
+    block.free_layer_gguf(64)
+
+
+@pytest.mark.parametrize("ty", [11, 12])
+def test_rows_of_any_scale(block, oracle, tmp_path, ty):
+    """Rows whose values lie near 1e-30, 1e-4 and 1e4 and rows that hold one
+    large value among small ones: each row has its own power of two.  (The
+    tiny rows' h is below fp32's range in the reference too; the bar is on
+    the others and a zero row gives zeros.)"""
+    dims = (256, 12, 4, 128, 256)
+    g = _upload(block, tmp_path, 65, dims, ty)
+    rng = np.random.default_rng(9)
+    x = rng.standard_normal((264, 256)).astype(np.float32)
+    x[0:40] *= np.float32(1e-4)
+    x[40:80] *= np.float32(1e4)
+    x[80:120, 3] = 3e4
+    x[120:160] *= rng.choice(np.float32([1e-6, 1.0, 1e3]), (40, 256))
+    y, _ = _check(block, oracle, g, 65, dims, x)
+    x[5] = 0.0
+    x[6] *= np.float32(1e-26)
+    y2, _, _, _ = block.forward_port_moe_gguf(x, None, 65, 264)
+    assert not y2[5].any() and np.isfinite(y2).all()
+    keep = np.arange(264) // 2 != 3
+    keep[5] = False
+    assert np.array_equal(y[keep], y2[keep])
+    block.free_layer_gguf(65)
+
+
+def test_errors(block, tmp_path):
+    """The texts of the other forms: a non-finite activation, an infinite
+    super-scale in a shared and in a routed expert."""
+    dims, T = (256, 8, 2, 128, 128), 300
+    x = np.random.default_rng(1).standard_normal((T, 256)).astype(np.float32)
+    _upload(block, tmp_path, 66, dims, 11)
+    bad = x.copy()
+    bad[299, 7] = np.inf
+    with pytest.raises(DismoenError) as ei:
+        block.forward_port_moe_gguf(bad, None, 66, T)
+    assert json.loads(str(ei.value))["error_type"] == "ACT_LOAD_FAILED"
+    block.forward_port_moe_gguf(x, None, 66, T)  # and recovers
+
+    def inf_scale(name):
+        def f(ts):
+            i = [k for k, t in enumerate(ts) if t[0] == "blk.0." + name][0]
+            raw = bytearray(ts[i][3])
+            raw[112:114] = b"\x00\x7c"
+            return ts[:i] + [(*ts[i][:3], bytes(raw))] + ts[i + 1:]
+        return f
+
+    for name, detail in (("ffn_shared_up.weight", "non-finite in up projection"),
+                         ("ffn_shared_down.weight", "non-finite in down projection"),
+                         ("ffn_gate.3.weight", "non-finite in gate projection")):
+        _upload(block, tmp_path, 66, dims, 11, inf_scale(name))
+        texts = []
+        for n in (T, 255):  # the matrix-core form and the form below it
+            with pytest.raises(DismoenError) as ei:
+                block.forward_port_moe_gguf(x[:n], None, 66, n)
+            texts.append(str(ei.value))
+        assert texts[0] == texts[1] and json.loads(texts[0])["detail"] == detail
+    block.free_layer_gguf(66)
