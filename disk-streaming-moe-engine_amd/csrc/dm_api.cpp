@@ -639,17 +639,13 @@ GgufLayer* get_glayer(dmh_ctx* c, int layer) {
 // persistent grids could hold CUs the launch waits for) and the
 // stream is not being captured (a replay would repeat the launch count);
 // otherwise router and shared-gate logits (fp32 weights, router_forward's
-// order), selection and gate, then from kGgufGroupMinT tokens on the
-// grouping by expert and the grouped gate/up, down and combine launches
-// (dm::launch_gguf_units; from kGgufMmMinT tokens on dm::launch_gguf_mm on
-// layers with matrix-core records), below it gate/up of every (token, slot) and the
-// down projections with moe_aggregate_forward.
-// The grouped several-token form: from 128 tokens on (below, the units hold
-// one or two tokens and the grid sized for the most units there could be
-// costs more than the rows it saves: Qwen3.6 shape, Q3_K, per call 851
-// against 957 us at 128 tokens, 404 against 258 at 32), for at most 4096
-// experts (the grouping's LDS holds two ints per expert).
-constexpr int kGgufGroupMinT = 128;
+// order), selection and gate, then, where the call holds enough work
+// (dm::gguf_units_pay), the grouping by expert and the grouped gate/up, down
+// and combine launches (dm::launch_gguf_units; from kGgufMmMinT tokens on
+// dm::launch_gguf_mm on layers with matrix-core records), below it gate/up of
+// every (token, slot) and the down projections with moe_aggregate_forward.
+// The grouped forms take at most 4096 experts (the grouping's LDS holds two
+// ints per expert).
 constexpr int kGgufGroupMaxE = 4096;
 
 hipError_t run_gguf_block(dmh_ctx* c, GgufLayer* G, unsigned long long* status, const float* dx,
@@ -690,18 +686,21 @@ hipError_t run_gguf_block(dmh_ctx* c, GgufLayer* G, unsigned long long* status, 
   if ((e = dm::launch_router_select(c->z.p, L.E + 1, T, L.E, L.K, 1, dids, dprobs, dshg, status,
                                     st)) != hipSuccess)
     return e;
-  if (T >= kGgufGroupMinT && L.E <= kGgufGroupMaxE) {
+  if (T > 1 && L.E <= kGgufGroupMaxE && (dm::gguf_units_pay(L, T) || dm::gguf_mm_ok(L, T))) {
     // several tokens: grouped by expert, each expert row read once per unit
-    const int nu = dm::group_units_max(T, L.K, L.E);
+    const bool mm = dm::gguf_mm_ok(L, T);
+    const int tok = mm ? 0 : dm::gguf_unit_tokens(L, T);
+    const int nu = mm ? dm::group_units_max(T, L.K, L.E)
+                      : dm::group_small_units_max(T, L.K, L.E, tok);
     if ((e = c->g_off.ensure(L.E + 1)) != hipSuccess) return e;
     if ((e = c->g_perm.ensure((size_t)T * L.K)) != hipSuccess) return e;
     if ((e = c->g_meta.ensure(2)) != hipSuccess) return e;
     if ((e = c->g_units.ensure(nu)) != hipSuccess) return e;
     if ((e = c->g_r.ensure((size_t)T * (L.K + 1) * L.H)) != hipSuccess) return e;
     if ((e = dm::launch_group_build(dids, T, L.K, L.E, c->g_off.p, c->g_perm.p, c->g_units.p,
-                                    c->g_meta.p, st)) != hipSuccess)
+                                    c->g_meta.p, st, tok)) != hipSuccess)
       return e;
-    if (dm::gguf_mm_ok(L, T)) {
+    if (mm) {
       // prefill: the experts' products on the matrix cores
       const size_t TK = (size_t)T * L.K, TH = (size_t)T * L.H;
       const size_t hn = TK * L.I + (size_t)T * L.Ish;

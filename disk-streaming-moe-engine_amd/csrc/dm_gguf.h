@@ -59,10 +59,15 @@ hipError_t launch_gguf_down_combine(const GgufMoeDev& L, const float* h, int ldh
                                     const float* residual, float* y, unsigned long long* status,
                                     hipStream_t st);
 
+// Whether T tokens of L run faster grouped (launch_gguf_units) than token by
+// token (launch_gguf_gateup, launch_gguf_down_combine).
+bool gguf_units_pay(const GgufMoeDev& L, int T);
+// Tokens per unit of launch_gguf_units.
+int gguf_unit_tokens(const GgufMoeDev& L, int T);
 // The same outputs for T tokens grouped by expert (off, perm, units, meta
-// of launch_group_build on ids; nunits = group_units_max(T, K, E)): each
-// expert row is read once per unit of up to 128 tokens instead of once per
-// (token, slot).  Three launches: gate/up into h as launch_gguf_gateup, the
+// of launch_group_build on ids with tok = gguf_unit_tokens; nunits =
+// group_small_units_max): each expert row is read and decoded once per unit
+// instead of once per (token, slot).  Three launches: gate/up into h as launch_gguf_gateup, the
 // down projections into parts [T][K+1][H], then moe_aggregate_forward's
 // combine.  Every token's sums are formed by the same helpers in the same
 // order as launch_gguf_gateup / launch_gguf_down_combine: the same bits.

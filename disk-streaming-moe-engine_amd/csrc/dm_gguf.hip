@@ -14,6 +14,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "dm_device.h"
 #include "dm_gguf.h"
 #include "dm_grouped.h"
@@ -432,21 +434,20 @@ __global__ __launch_bounds__(256) void k_gguf_down_combine(
 }
 
 // ---- several tokens grouped by expert --------------------------------------
-// The units of launch_group_build: an expert's row is read once per unit (up
-// to 128 tokens) and its weights decoded once per pass of kGgufUnitTok
-// tokens.  Each token's lane sums and wave reductions are those of
-// k_gguf_gateup / k_gguf_down_combine (the same helpers, the same order), so
-// a token's outputs do not depend on the form that computed them.
+// The units of launch_group_build (up to four or eight tokens of an expert):
+// an expert's row is read and decoded once per unit.  Each token's lane sums
+// and wave reductions are those of k_gguf_gateup / k_gguf_down_combine (the
+// same helpers or the same arithmetic, the same order), so a token's outputs
+// do not depend on the form that computed them.
 constexpr int kGgufUnitTok = 8;
 
 struct GgufUnit {
   int e, p0, n;  // expert (E: shared), first position (shared: first token), tokens
   bool sh;
 };
-__device__ __forceinline__ GgufUnit gguf_unit(const int2* units, const int32_t* meta,
-                                              const int32_t* off, int u, int E, int T) {
+__device__ __forceinline__ GgufUnit gguf_unit(const int2* units, const int32_t* off, int u, int size,
+                                              int E, int T) {
   const int2 v = units[u];
-  const int size = u < meta[1] ? kUnitBig : kUnitSmall;
   GgufUnit r;
   r.sh = v.x >= E;
   r.e = r.sh ? E : v.x;
@@ -474,10 +475,10 @@ __global__ __launch_bounds__(256) void k_gguf_gateup_units(
     GgufMoeDev L, const float* __restrict__ x, const int32_t* __restrict__ off,
     const int32_t* __restrict__ perm, const int2* __restrict__ units,
     const int32_t* __restrict__ meta, int ntok, float* __restrict__ h, int ldh,
-    unsigned long long* status, int u0) {
+    unsigned long long* status, int u0, int usz) {
   const int u = u0 + (int)blockIdx.y;
   if (u >= meta[0]) return;
-  const GgufUnit ut = gguf_unit(units, meta, off, u, L.E, ntok);
+  const GgufUnit ut = gguf_unit(units, off, u, usz, L.E, ntok);
   const int rows = ut.sh ? L.Ish : L.I;
   const int r = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (r >= rows || ut.n <= 0) return;
@@ -542,10 +543,10 @@ __global__ __launch_bounds__(256) void k_gguf_down_units(
     GgufMoeDev L, const float* __restrict__ h, int ldh, const int32_t* __restrict__ off,
     const int32_t* __restrict__ perm, const int2* __restrict__ units,
     const int32_t* __restrict__ meta, int ntok, float* __restrict__ parts,
-    unsigned long long* status, int u0) {
+    unsigned long long* status, int u0, int usz) {
   const int u = u0 + (int)blockIdx.y;
   if (u >= meta[0]) return;
-  const GgufUnit ut = gguf_unit(units, meta, off, u, L.E, ntok);
+  const GgufUnit ut = gguf_unit(units, off, u, usz, L.E, ntok);
   const int d = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (d >= L.H || ut.n <= 0) return;
   const int lane = threadIdx.x & 63;
@@ -588,201 +589,371 @@ __global__ __launch_bounds__(256) void k_gguf_down_units(
   }
 }
 
-// Blocked forms (the common shapes): a wave keeps the activations of
-// kGgufBlkTok tokens in registers (its lane's chunks, at most kGgufBlkCh of
-// them) across rpw rows (1 .. kGgufBlkRowsMax, more when the units hold
-// more tokens), so that a row costs its weights and the
-// products, not another read of every token's x (or h) from the caches.
-// The lane sums run over the same chunks in the same order as above.
-constexpr int kGgufBlkTok = 4, kGgufBlkCh = 2, kGgufBlkRowsMax = 8;
+// Blocked forms (the common shapes): a workgroup of 4 waves stages the
+// activations of its unit in LDS and each wave takes rpw rows, all the unit's
+// tokens (TN: 1, 2, 4 or 8) per row: its weights are decoded once and the
+// next row's bytes requested as soon as a chunk is decoded.  Bound by the
+// vector units (a weight costs its decode, 2.5 operations for Q4_K, and a
+// multiply-add per token) and, in the down rows of few tokens, by the block
+// headers' decode, so the loads are as wide as the blocks allow (Q4_K: header
+// and codes 16 bytes each) and four sums are reduced together (wave_sum4),
+// which costs half of reducing them one after another and leaves their
+// epilogues to four lanes at once.  The lane sums run over the same chunks in
+// the same order as above: the same bits.  24 tokens of Q4_K at 2048 / 512:
+// gate/up 283 -> 74 us, down 189 -> 49 us against the token-by-token kernels.
+constexpr int kGgufBlkCh = 2;         // chunks of a lane and row at most
+constexpr int kGgufBlkThreads = 256;  // 4 waves
 
-// gate/up, sixteen weights per lane (gu_dot16), H <= 64 * 16 * kGgufBlkCh
-template <int T>
-__global__ __launch_bounds__(256) void k_gguf_gateup_units_blk(
-    GgufMoeDev L, const float* __restrict__ x, const int32_t* __restrict__ off,
-    const int32_t* __restrict__ perm, const int2* __restrict__ units,
-    const int32_t* __restrict__ meta, int ntok, float* __restrict__ h, int ldh,
-    unsigned long long* status, int u0, int rpw) {
-  const int u = u0 + (int)blockIdx.y;
-  if (u >= meta[0]) return;
-  const GgufUnit ut = gguf_unit(units, meta, off, u, L.E, ntok);
-  const int rows = ut.sh ? L.Ish : L.I;
-  const int row0 = ((int)blockIdx.x * 4 + (threadIdx.x >> 6)) * rpw;
-  if (row0 >= rows || ut.n <= 0) return;
-  const int lane = threadIdx.x & 63;
-  const uint8_t* wg = L.raw + L.off[(size_t)ut.e * 3 + 0];
-  const uint8_t* wu = L.raw + L.off[(size_t)ut.e * 3 + 1];
-  for (int i0 = 0; i0 < ut.n; i0 += kGgufBlkTok) {
-    const int nk = min(kGgufBlkTok, ut.n - i0);
-    int tt[kGgufBlkTok], sl[kGgufBlkTok];
-    f32x4 xv[kGgufBlkTok][kGgufBlkCh][4];
+// wave_sum_dpp of four values, value lane & 3 valid in lanes 60 .. 63: two
+// exchange steps that halve the values each lane carries, then the same
+// binary tree (additions commute, so the bits are wave_sum_dpp's).
+__device__ __forceinline__ float wave_sum4(float v0, float v1, float v2, float v3, int lane) {
+  const bool o1 = lane & 1, o2 = lane & 2;
+  const float a = (o1 ? v1 : v0) + dpp_f<0xB1, 0xF>(o1 ? v0 : v1);  // quad_perm 1 0 3 2
+  const float b = (o1 ? v3 : v2) + dpp_f<0xB1, 0xF>(o1 ? v2 : v3);
+  float s = (o2 ? b : a) + dpp_f<0x4E, 0xF>(o2 ? a : b);  // quad_perm 2 3 0 1
+  s = s + dpp_f<0x124, 0xF>(s);  // row_ror:4: quads 3 + 2 and 1 + 0
+  s = s + dpp_f<0x128, 0xF>(s);  // row_ror:8
+  auto p = __builtin_amdgcn_permlane16_swap(f2u(s), f2u(s), false, false);
+  s = u2f(p[0]) + u2f(p[1]);  // rows 0 + 1, rows 2 + 3
+  p = __builtin_amdgcn_permlane32_swap(f2u(s), f2u(s), false, false);
+  return u2f(p[0]) + u2f(p[1]);
+}
+
+__device__ __forceinline__ uint32_t load_u32(const uint8_t* p) {  // at any address
+  uint32_t v;
+  __builtin_memcpy(&v, p, 4);
+  return v;
+}
+
+// The bytes of W (8 or 16) consecutive weights at element e0, a multiple of
+// W, and the values valuesW forms from them (Q3_K, W = 16: see q3_dot16).
+// (F32 and BF16 rows: the address, read when decoded.)
+template <int T, int W>
+struct WRaw {
+  const uint8_t* raw;
+  int64_t e0;
+  __device__ __forceinline__ void load(const uint8_t* r, int64_t e) {
+    raw = r;
+    e0 = e;
+  }
+  __device__ __forceinline__ void decode(int layout, f32x4 (&v)[W / 4]) const {
+    valuesW<T, W>(raw, e0, layout, v);
+  }
+};
+template <int W>
+struct WRaw<kGgmlQ3_K, W> {
+  Q3Raw<W> q;
+  __device__ __forceinline__ void load(const uint8_t* raw, int64_t e0) {
+    const uint8_t* blk = raw + (e0 >> 8) * 114;
+    const int e = (int)(e0 & 255);
+    const uint16_t* h = reinterpret_cast<const uint16_t*>(blk);
+    if constexpr (W == 16) {
+      const uint32_t c = load_u32(blk + 32 + (e >> 2));
+      q.hm = h[e >> 4];
+      q.q0 = c & 0xFFFFu;
+      q.q1 = c >> 16;
+    } else {
+      q.hm = blk[e >> 3];
+      q.q0 = h[16 + (e >> 3)];
+      q.q1 = 0;
+    }
+    q.sc = blk[96 + (e >> 4)];
+    q.d = h[56];
+  }
+  __device__ __forceinline__ void decode(int, f32x4 (&v)[W / 4]) const { q3_decode<W>(q, v); }
+};
+template <int W>
+struct WRaw<kGgmlQ4_K, W> {
+  uint4 hd;
+  uint32_t c[W / 4];
+  int j, sh;  // sub-block, code shift
+  __device__ __forceinline__ void load(const uint8_t* raw, int64_t e0) {
+    const uint8_t* blk = raw + (e0 >> 8) * 144;  // 16-byte aligned, as the tensors are
+    const int e = (int)(e0 & 255);
+    j = e >> 5;
+    sh = (e & 16) >> 2;
+    hd = *reinterpret_cast<const uint4*>(blk);
+    const uint8_t* p = blk + 16 + 16 * j + (e & 15);
+    if constexpr (W == 16) {
+      const uint4 v = *reinterpret_cast<const uint4*>(p);
+      c[0] = v.x;
+      c[1] = v.y;
+      c[2] = v.z;
+      c[3] = v.w;
+    } else {
+      const uint2 v = *reinterpret_cast<const uint2*>(p);
+      c[0] = v.x;
+      c[1] = v.y;
+    }
+  }
+  __device__ __forceinline__ void decode(int layout, f32x4 (&v)[W / 4]) const {
+    // packed bytes j & 3, 4 + (j & 3), 8 + (j & 3) (the words of values4)
+    const int s8 = 8 * (j & 3);
+    const uint32_t b0 = hd.y >> s8, b1 = hd.z >> s8, b2 = hd.w >> s8;
+    uint32_t sc, mn;
+    if (j < 4) {
+      sc = b0 & 63;
+      mn = b1 & 63;
+    } else {
+      const uint32_t lo = layout ? b2 : b1;
+      sc = (lo & 15) | ((b0 & 0xC0) >> 2);
+      mn = ((lo >> 4) & 15) | ((b1 & 0xC0) >> 2);
+    }
+    const float fs = (float)sc * h2f(hd.x & 0xFFFF), fm = (float)mn * h2f(hd.x >> 16);
+    // fs q (17 + 4 bits) is exact, so one rounding gives values4's fs q - fm
 #pragma unroll
-    for (int k = 0; k < kGgufBlkTok; ++k) {
-      gguf_unit_pos(ut, perm, L.K, min(i0 + k, ut.n - 1), tt[k], sl[k]);
-      const float* xt = x + (size_t)tt[k] * L.H;
+    for (int i = 0; i < W / 4; ++i) {
+      const uint32_t q = (c[i] >> sh) & 0x0F0F0F0Fu;
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        v[i][k] = __builtin_fmaf(fs, (float)((q >> (8 * k)) & 0xFF), -fm);
+    }
+  }
+};
+template <int W>
+struct WRaw<kGgmlQ8_0, W> {
+  uint32_t d, c[W / 4];
+  __device__ __forceinline__ void load(const uint8_t* raw, int64_t e0) {
+    const uint8_t* blk = raw + (e0 >> 5) * 34;
+    d = *reinterpret_cast<const uint16_t*>(blk);
+#pragma unroll
+    for (int i = 0; i < W / 4; ++i) c[i] = load_u32(blk + 2 + (int)(e0 & 31) + 4 * i);
+  }
+  __device__ __forceinline__ void decode(int, f32x4 (&v)[W / 4]) const {
+    const float fd = h2f(d);
+#pragma unroll
+    for (int i = 0; i < W / 4; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[i][k] = fd * (float)(int8_t)((c[i] >> (8 * k)) & 0xFF);
+  }
+};
+
+// acc + the products of a chunk's sixteen gate or up weights (gu_dot16's)
+template <int T>
+struct GuW {
+  f32x4 w[4];
+  float fs;
+  __device__ __forceinline__ void set(const WRaw<T, 16>& r, int layout) {
+    if constexpr (T == kGgmlQ3_K) {
+      uint32_t qw[4];
+      q3_codes(r.q.q0 | (r.q.q1 << 16), r.q.hm, qw);
+      fs = (float)((int)r.q.sc - 32) * h2f(r.q.d);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) w[i >> 2][i & 3] = q3_code(qw, i);
+    } else {
+      r.decode(layout, w);
+      fs = 0.0f;
+    }
+  }
+  __device__ __forceinline__ float dot(const f32x4 (&x)[4], float xs, float acc) const {
+    if constexpr (T == kGgmlQ3_K) {
+      float t = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) t = dot4(w[i], x[i], t);
+      return __builtin_fmaf(fs, __builtin_fmaf(-4.0f, xs, t), acc);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc = dot4(w[i], x[i], acc);
+      return acc;
+    }
+  }
+};
+
+// Rows row0 .. rend - 1 of a gate / up pair against TN staged tokens (nk of
+// them real).  xl: [token][chunk][4][64 lanes] float4, xs: [token][chunk]
+// [64] chunk sums (Q3_K), pos: [token] (token, slot).
+template <int T, int TN>
+__device__ __forceinline__ void gu_rows(const GgufMoeDev& L, const uint8_t* wg, const uint8_t* wu,
+                                        const f32x4* xl, const float* xs, const int2* pos, bool sh,
+                                        int nk, int row0, int rend, float* __restrict__ h, int ldh,
+                                        unsigned long long* status) {
+  constexpr int R = TN >= 4 ? 1 : 4 / TN;  // rows whose sums are reduced together
+  const int lane = threadIdx.x & 63, H = L.H, nch = (H + 1023) >> 10;
+  WRaw<T, 16> pg[kGgufBlkCh], pu[kGgufBlkCh];
+  auto fetch = [&](int r, int ch) {
+    const int64_t e0 = (int64_t)r * H + min(lane * 16 + 1024 * ch, H - 16);
+    pg[ch].load(wg, e0);
+    pu[ch].load(wu, e0);
+  };
+#pragma unroll
+  for (int ch = 0; ch < kGgufBlkCh; ++ch)
+    if (ch < nch) fetch(row0, ch);
+  for (int r0 = row0; r0 < rend; r0 += R) {
+    float ag[R * TN], au[R * TN];
+#pragma unroll
+    for (int v = 0; v < R * TN; ++v) ag[v] = au[v] = 0.0f;
+#pragma unroll
+    for (int rr = 0; rr < R; ++rr) {  // (rows from rend on: row rend - 1 again, not stored)
 #pragma unroll
       for (int ch = 0; ch < kGgufBlkCh; ++ch) {
-        const int c = lane * 16 + 1024 * ch;
+        if (ch >= nch) break;  // uniform
+        GuW<T> g, u;
+        g.set(pg[ch], L.layout);
+        u.set(pu[ch], L.layout);
+        fetch(min(r0 + rr + 1, rend - 1), ch);
+        if (lane * 16 + 1024 * ch < H) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          xv[k][ch][j] = c < L.H ? *reinterpret_cast<const f32x4*>(xt + c + 4 * j)
-                                 : f32x4{0, 0, 0, 0};
+          for (int k = 0; k < TN; ++k) {
+            f32x4 x[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = xl[((k * nch + ch) * 4 + i) * 64 + lane];
+            const float s = T == kGgmlQ3_K ? xs[(k * nch + ch) * 64 + lane] : 0.0f;
+            ag[rr * TN + k] = g.dot(x, s, ag[rr * TN + k]);
+            au[rr * TN + k] = u.dot(x, s, au[rr * TN + k]);
+          }
+        }
       }
     }
-    // Q3_K: the next row's bytes are requested before this row's products
-    // (q3_dot16 on them is gu_dot16's arithmetic)
-    Q3Raw<16> pg[kGgufBlkCh], pu[kGgufBlkCh];
-    auto q3_fetch = [&](int r) {
 #pragma unroll
-      for (int ch = 0; ch < kGgufBlkCh; ++ch) {
-        const int c = min(lane * 16 + 1024 * ch, L.H - 16);
-        pg[ch] = q3_load<16>(wg, (int64_t)r * L.H + c);
-        pu[ch] = q3_load<16>(wu, (int64_t)r * L.H + c);
-      }
-    };
-    if constexpr (T == kGgmlQ3_K) q3_fetch(row0);
-    for (int rr = 0; rr < rpw; ++rr) {
-      const int r = row0 + rr;
-      if (r >= rows) break;  // uniform per wave
-      const int64_t base = (int64_t)r * L.H;
-      float ag[kGgufBlkTok], au[kGgufBlkTok];
-#pragma unroll
-      for (int k = 0; k < kGgufBlkTok; ++k) ag[k] = au[k] = 0.0f;
-      if constexpr (T == kGgmlQ3_K) {
-        Q3Raw<16> cg[kGgufBlkCh], cu[kGgufBlkCh];
-#pragma unroll
-        for (int ch = 0; ch < kGgufBlkCh; ++ch) {
-          cg[ch] = pg[ch];
-          cu[ch] = pu[ch];
-        }
-        if (rr + 1 < rpw && r + 1 < rows) q3_fetch(r + 1);
-#pragma unroll
-        for (int ch = 0; ch < kGgufBlkCh; ++ch) {
-          const int c = lane * 16 + 1024 * ch;
-          if (c < L.H) {
-#pragma unroll
-            for (int k = 0; k < kGgufBlkTok; ++k)
-              if (k < nk) {
-                const float xs = xsum16(xv[k][ch]);
-                ag[k] = q3_dot16(cg[ch], xv[k][ch], xs, ag[k]);
-                au[k] = q3_dot16(cu[ch], xv[k][ch], xs, au[k]);
-              }
-          }
-        }
-      } else {
-#pragma unroll
-        for (int ch = 0; ch < kGgufBlkCh; ++ch) {
-          const int c = lane * 16 + 1024 * ch;
-          if (c < L.H) {
-#pragma unroll
-            for (int k = 0; k < kGgufBlkTok; ++k)
-              if (k < nk) gu_dot16<T>(wg, wu, base + c, L.layout, xv[k][ch], ag[k], au[k]);
-          }
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < kGgufBlkTok; ++k) {
-        if (k >= nk) break;  // uniform per wave
-        const float g = wave_sum_dpp(ag[k]), uu = wave_sum_dpp(au[k]);
-        if (lane == 0) {
-          const int t = tt[k], slot = sl[k];
-          const float hv = dm_silu(g) * uu;
-          const uint32_t ph = ut.sh ? kPhShared : kPhExpert, sp = ut.sh ? 0 : (uint32_t)slot;
-          if (!finite_f(g)) record_err(status, err_key(ph, t, sp, r, kEkGate));
-          if (!finite_f(uu)) record_err(status, err_key(ph, t, sp, r, kEkUp));
-          if (!finite_f(hv)) record_err(status, err_key(ph, t, sp, r, kEkH));
-          h[((size_t)t * (L.K + 1) + slot) * ldh + r] = hv;
-        }
+    for (int v0 = 0; v0 < R * TN; v0 += 4) {
+      const float g = wave_sum4(ag[v0], ag[v0 + 1], ag[v0 + 2], ag[v0 + 3], lane);
+      const float u = wave_sum4(au[v0], au[v0 + 1], au[v0 + 2], au[v0 + 3], lane);
+      const int v = v0 + (lane & 3), r = r0 + v / TN, k = v % TN;
+      if (lane >= 60 && r < rend && k < nk) {
+        const int t = pos[k].x, slot = pos[k].y;
+        const float hv = dm_silu(g) * u;
+        const uint32_t ph = sh ? kPhShared : kPhExpert, sp = sh ? 0 : (uint32_t)slot;
+        if (!finite_f(g)) record_err(status, err_key(ph, t, sp, r, kEkGate));
+        if (!finite_f(u)) record_err(status, err_key(ph, t, sp, r, kEkUp));
+        if (!finite_f(hv)) record_err(status, err_key(ph, t, sp, r, kEkH));
+        h[((size_t)t * (L.K + 1) + slot) * ldh + r] = hv;
       }
     }
   }
 }
 
-// down, eight weights per lane, I and Ish <= 64 * 8 * kGgufBlkCh
-template <int T>
-__global__ __launch_bounds__(256) void k_gguf_down_units_blk(
+// Workgroup (rb, u): 8 rpw rows of unit u0 + u.  Sixteen weights per lane
+// (gu_dot16), H <= 64 * 16 * kGgufBlkCh.
+template <int T, int TM>
+__global__ __launch_bounds__(kGgufBlkThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_gguf_gateup_units_blk(
+    GgufMoeDev L, const float* __restrict__ x, const int32_t* __restrict__ off,
+    const int32_t* __restrict__ perm, const int2* __restrict__ units,
+    const int32_t* __restrict__ meta, int ntok, float* __restrict__ h, int ldh,
+    unsigned long long* status, int u0, int rpw) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char ldsg[];
+  __shared__ int2 pos[TM];
+  const int u = u0 + (int)blockIdx.y;
+  if (u >= meta[0]) return;
+  const GgufUnit ut = gguf_unit(units, off, u, TM, L.E, ntok);
+  const int rows = ut.sh ? L.Ish : L.I, nch = (L.H + 1023) >> 10;
+  if ((int)blockIdx.x * 4 * rpw >= rows || ut.n <= 0) return;  // uniform per workgroup
+  const int row0 = ((int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * rpw;
+  const int rend = min(row0 + rpw, rows);
+  const uint8_t* wg = L.raw + L.off[(size_t)ut.e * 3 + 0];
+  const uint8_t* wu = L.raw + L.off[(size_t)ut.e * 3 + 1];
+  f32x4* xl = reinterpret_cast<f32x4*>(ldsg);
+  float* xs = reinterpret_cast<float*>(xl + TM * nch * 256);
+  const int nk = ut.n;
+  for (int i = threadIdx.x; i < nk * nch * 64; i += kGgufBlkThreads) {
+    const int l = i & 63, kc = i >> 6, k = kc / nch, c = l * 16 + 1024 * (kc - k * nch);
+    int t, slot;
+    gguf_unit_pos(ut, perm, L.K, k, t, slot);
+    f32x4 v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      v[j] = c < L.H ? *reinterpret_cast<const f32x4*>(x + (size_t)t * L.H + c + 4 * j)
+                     : f32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) xl[(kc * 4 + j) * 64 + l] = v[j];
+    if (T == kGgmlQ3_K) xs[kc * 64 + l] = xsum16(v);
+    if (c == 0) pos[k] = make_int2(t, slot);
+  }
+  __syncthreads();
+  if (row0 >= rows) return;
+  if (nk == 1) gu_rows<T, 1>(L, wg, wu, xl, xs, pos, ut.sh, nk, row0, rend, h, ldh, status);
+  else if (nk == 2) gu_rows<T, 2>(L, wg, wu, xl, xs, pos, ut.sh, nk, row0, rend, h, ldh, status);
+  else if (nk <= 4) gu_rows<T, 4>(L, wg, wu, xl, xs, pos, ut.sh, nk, row0, rend, h, ldh, status);
+  else gu_rows<T, TM>(L, wg, wu, xl, xs, pos, ut.sh, nk, row0, rend, h, ldh, status);
+}
+
+// Output rows d0 .. dend - 1 of a down projection against TN staged tokens'
+// h (hl: [token][chunk][2][64 lanes] float4).
+template <int T, int TN>
+__device__ __forceinline__ void down_rows(const GgufMoeDev& L, const uint8_t* wd, int n,
+                                          const f32x4* hl, const int2* pos, bool sh, int nk, int d0,
+                                          int dend, float* __restrict__ parts,
+                                          unsigned long long* status) {
+  constexpr int R = TN >= 4 ? 1 : 4 / TN;
+  const int lane = threadIdx.x & 63, nch = (n + 511) >> 9;
+  WRaw<T, 8> p[kGgufBlkCh];
+  auto fetch = [&](int d, int ch) {
+    p[ch].load(wd, (int64_t)d * n + min(lane * 8 + 512 * ch, n - 8));
+  };
+#pragma unroll
+  for (int ch = 0; ch < kGgufBlkCh; ++ch)
+    if (ch < nch) fetch(d0, ch);
+  for (int r0 = d0; r0 < dend; r0 += R) {
+    float a[R * TN];
+#pragma unroll
+    for (int v = 0; v < R * TN; ++v) a[v] = 0.0f;
+#pragma unroll
+    for (int rr = 0; rr < R; ++rr) {
+#pragma unroll
+      for (int ch = 0; ch < kGgufBlkCh; ++ch) {
+        if (ch >= nch) break;  // uniform
+        f32x4 w[2];
+        p[ch].decode(L.layout, w);
+        fetch(min(r0 + rr + 1, dend - 1), ch);
+        if (lane * 8 + 512 * ch < n) {
+#pragma unroll
+          for (int k = 0; k < TN; ++k)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+              a[rr * TN + k] = dot4(w[j], hl[((k * nch + ch) * 2 + j) * 64 + lane], a[rr * TN + k]);
+        }
+      }
+    }
+#pragma unroll
+    for (int v0 = 0; v0 < R * TN; v0 += 4) {
+      const float s = wave_sum4(a[v0], a[v0 + 1], a[v0 + 2], a[v0 + 3], lane);
+      const int v = v0 + (lane & 3), d = r0 + v / TN, k = v % TN;
+      if (lane >= 60 && d < dend && k < nk) {
+        const int t = pos[k].x, slot = pos[k].y;
+        if (!finite_f(s))
+          record_err(status, err_key(sh ? kPhShared : kPhExpert, t, sh ? 0 : slot, n + d, kEkDown));
+        parts[((size_t)t * (L.K + 1) + slot) * L.H + d] = s;
+      }
+    }
+  }
+}
+
+// Eight weights per lane, I and Ish <= 64 * 8 * kGgufBlkCh.
+template <int T, int TM>
+__global__ __launch_bounds__(kGgufBlkThreads) void k_gguf_down_units_blk(
     GgufMoeDev L, const float* __restrict__ h, int ldh, const int32_t* __restrict__ off,
     const int32_t* __restrict__ perm, const int2* __restrict__ units,
     const int32_t* __restrict__ meta, int ntok, float* __restrict__ parts,
     unsigned long long* status, int u0, int rpw) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char ldsg[];
+  __shared__ int2 pos[TM];
   const int u = u0 + (int)blockIdx.y;
   if (u >= meta[0]) return;
-  const GgufUnit ut = gguf_unit(units, meta, off, u, L.E, ntok);
-  const int d0 = ((int)blockIdx.x * 4 + (threadIdx.x >> 6)) * rpw;
-  if (d0 >= L.H || ut.n <= 0) return;
-  const int lane = threadIdx.x & 63;
-  const int n = ut.sh ? L.Ish : L.I;
+  const GgufUnit ut = gguf_unit(units, off, u, TM, L.E, ntok);
+  if ((int)blockIdx.x * 4 * rpw >= L.H || ut.n <= 0) return;  // uniform per workgroup
+  const int d0 = ((int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * rpw;
+  const int dend = min(d0 + rpw, L.H);
+  const int n = ut.sh ? L.Ish : L.I, nch = (n + 511) >> 9;
   const uint8_t* wd = L.raw + L.off[(size_t)ut.e * 3 + 2];
-  for (int i0 = 0; i0 < ut.n; i0 += kGgufBlkTok) {
-    const int nk = min(kGgufBlkTok, ut.n - i0);
-    int tt[kGgufBlkTok], sl[kGgufBlkTok];
-    f32x4 hv[kGgufBlkTok][kGgufBlkCh][2];
+  f32x4* hl = reinterpret_cast<f32x4*>(ldsg);
+  const int nk = ut.n;
+  for (int i = threadIdx.x; i < nk * nch * 64; i += kGgufBlkThreads) {
+    const int l = i & 63, kc = i >> 6, k = kc / nch, c = l * 8 + 512 * (kc - k * nch);
+    int t, slot;
+    gguf_unit_pos(ut, perm, L.K, k, t, slot);
+    const float* ht = h + ((size_t)t * (L.K + 1) + slot) * ldh;
 #pragma unroll
-    for (int k = 0; k < kGgufBlkTok; ++k) {
-      gguf_unit_pos(ut, perm, L.K, min(i0 + k, ut.n - 1), tt[k], sl[k]);
-      const float* ht = h + ((size_t)tt[k] * (L.K + 1) + sl[k]) * ldh;
-#pragma unroll
-      for (int ch = 0; ch < kGgufBlkCh; ++ch) {
-        const int c = lane * 8 + 512 * ch;
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          hv[k][ch][j] = c < n ? *reinterpret_cast<const f32x4*>(ht + c + 4 * j)
-                               : f32x4{0, 0, 0, 0};
-      }
-    }
-    // Q3_K: the next row's bytes are requested before this row's products
-    // (q3_decode on them forms valuesW's values)
-    Q3Raw<8> pd[kGgufBlkCh];
-    auto q3_fetch = [&](int d) {
-#pragma unroll
-      for (int ch = 0; ch < kGgufBlkCh; ++ch)
-        pd[ch] = q3_load<8>(wd, (int64_t)d * n + min(lane * 8 + 512 * ch, n - 8));
-    };
-    if constexpr (T == kGgmlQ3_K) q3_fetch(d0);
-    for (int rr = 0; rr < rpw; ++rr) {
-      const int d = d0 + rr;
-      if (d >= L.H) break;  // uniform per wave
-      const int64_t base = (int64_t)d * n;
-      float a[kGgufBlkTok];
-#pragma unroll
-      for (int k = 0; k < kGgufBlkTok; ++k) a[k] = 0.0f;
-      Q3Raw<8> cd[kGgufBlkCh];
-      if constexpr (T == kGgmlQ3_K) {
-#pragma unroll
-        for (int ch = 0; ch < kGgufBlkCh; ++ch) cd[ch] = pd[ch];
-        if (rr + 1 < rpw && d + 1 < L.H) q3_fetch(d + 1);
-      }
-#pragma unroll
-      for (int ch = 0; ch < kGgufBlkCh; ++ch) {
-        const int c = lane * 8 + 512 * ch;
-        if (c < n) {
-          f32x4 w4[2];
-          if constexpr (T == kGgmlQ3_K)
-            q3_decode<8>(cd[ch], w4);
-          else
-            valuesW<T, 8>(wd, base + c, L.layout, w4);
-#pragma unroll
-          for (int k = 0; k < kGgufBlkTok; ++k)
-            if (k < nk) {
-#pragma unroll
-              for (int j = 0; j < 2; ++j) a[k] = dot4(w4[j], hv[k][ch][j], a[k]);
-            }
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < kGgufBlkTok; ++k) {
-        if (k >= nk) break;  // uniform per wave
-        const float v = wave_sum_dpp(a[k]);
-        if (lane == 0) {
-          const int t = tt[k], slot = sl[k];
-          if (!finite_f(v))
-            record_err(status, err_key(ut.sh ? kPhShared : kPhExpert, t, ut.sh ? 0 : slot,
-                                       n + d, kEkDown));
-          parts[((size_t)t * (L.K + 1) + slot) * L.H + d] = v;
-        }
-      }
-    }
+    for (int j = 0; j < 2; ++j)
+      hl[(kc * 2 + j) * 64 + l] =
+          c < n ? *reinterpret_cast<const f32x4*>(ht + c + 4 * j) : f32x4{0, 0, 0, 0};
+    if (c == 0) pos[k] = make_int2(t, slot);
   }
+  __syncthreads();
+  if (d0 >= L.H) return;
+  if (nk == 1) down_rows<T, 1>(L, wd, n, hl, pos, ut.sh, nk, d0, dend, parts, status);
+  else if (nk == 2) down_rows<T, 2>(L, wd, n, hl, pos, ut.sh, nk, d0, dend, parts, status);
+  else if (nk <= 4) down_rows<T, 4>(L, wd, n, hl, pos, ut.sh, nk, d0, dend, parts, status);
+  else down_rows<T, TM>(L, wd, n, hl, pos, ut.sh, nk, d0, dend, parts, status);
 }
 
 // y[t][d] from parts[t][0..K][d]: k_gguf_down_combine's combine, thread per (t, d).
@@ -1484,15 +1655,23 @@ hipError_t launch_dequant_gguf(int t, const uint8_t* raw, int64_t n, int layout,
     case kGgmlF32: KERNEL<kGgmlF32, W><<<GRID, 256, 0, st>>>(__VA_ARGS__); break;         \
     default: return hipErrorInvalidValue;                                                 \
   }
-#define DM_GGUF_DISPATCH_T(KERNEL, GRID, ...)                                             \
+#define DM_GGUF_DISPATCH_BLK(KERNEL, GRID, LDS, ...)                                      \
+  if (tm8) {                                                                              \
+    DM_GGUF_DISPATCH_TM(KERNEL, 8, GRID, LDS, __VA_ARGS__)                                \
+  } else {                                                                                \
+    DM_GGUF_DISPATCH_TM(KERNEL, 4, GRID, LDS, __VA_ARGS__)                                \
+  }
+#define DM_GGUF_DISPATCH_TM(KERNEL, TM, GRID, LDS, ...)                                   \
   switch (L.type) {                                                                       \
-    case kGgmlQ8_0: KERNEL<kGgmlQ8_0><<<GRID, 256, 0, st>>>(__VA_ARGS__); break;          \
-    case kGgmlQ4_K: KERNEL<kGgmlQ4_K><<<GRID, 256, 0, st>>>(__VA_ARGS__); break;          \
-    case kGgmlQ3_K: KERNEL<kGgmlQ3_K><<<GRID, 256, 0, st>>>(__VA_ARGS__); break;          \
-    case kGgmlBF16: KERNEL<kGgmlBF16><<<GRID, 256, 0, st>>>(__VA_ARGS__); break;          \
-    case kGgmlF32: KERNEL<kGgmlF32><<<GRID, 256, 0, st>>>(__VA_ARGS__); break;            \
+    case kGgmlQ8_0: DM_GGUF_BLK(KERNEL, kGgmlQ8_0, TM, GRID, LDS, __VA_ARGS__) break;     \
+    case kGgmlQ4_K: DM_GGUF_BLK(KERNEL, kGgmlQ4_K, TM, GRID, LDS, __VA_ARGS__) break;     \
+    case kGgmlQ3_K: DM_GGUF_BLK(KERNEL, kGgmlQ3_K, TM, GRID, LDS, __VA_ARGS__) break;     \
+    case kGgmlBF16: DM_GGUF_BLK(KERNEL, kGgmlBF16, TM, GRID, LDS, __VA_ARGS__) break;     \
+    case kGgmlF32: DM_GGUF_BLK(KERNEL, kGgmlF32, TM, GRID, LDS, __VA_ARGS__) break;       \
     default: return hipErrorInvalidValue;                                                 \
   }
+#define DM_GGUF_BLK(KERNEL, T_, TM, GRID, LDS, ...) \
+  KERNEL<T_, TM><<<GRID, kGgufBlkThreads, LDS, st>>>(__VA_ARGS__);
 #define DM_GGUF_DISPATCH(KERNEL, GRID, ...)                                               \
   if (L.H % 8 == 0 && L.I % 8 == 0 && L.Ish % 8 == 0) {                                   \
     DM_GGUF_DISPATCH_W(KERNEL, 8, GRID, __VA_ARGS__)                                      \
@@ -1531,6 +1710,64 @@ hipError_t launch_gguf_down_combine(const GgufMoeDev& L, const float* h, int ldh
   }
   return hipGetLastError();
 }
+// Eight tokens of more than 1024 activations are more LDS (68 KB) than a
+// launch may take by default: raised once per device.
+template <int T>
+static hipError_t gguf_blk_attr() {
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(k_gguf_gateup_units_blk<T, 8>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                             8 * kGgufBlkCh * (4096 + 256));
+}
+static hipError_t gguf_blk_attrs() {
+  static std::atomic<uint64_t> done{0};
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  const uint64_t bit = dev < 64 ? 1ull << dev : 0;
+  if (bit && (done.load() & bit)) return hipSuccess;
+  if ((e = gguf_blk_attr<kGgmlQ8_0>()) != hipSuccess) return e;
+  if ((e = gguf_blk_attr<kGgmlQ4_K>()) != hipSuccess) return e;
+  if ((e = gguf_blk_attr<kGgmlQ3_K>()) != hipSuccess) return e;
+  if ((e = gguf_blk_attr<kGgmlBF16>()) != hipSuccess) return e;
+  if ((e = gguf_blk_attr<kGgmlF32>()) != hipSuccess) return e;
+  done.fetch_or(bit);
+  return hipSuccess;
+}
+
+// The shapes of the blocked kernels.
+static bool gguf_blk_gateup(const GgufMoeDev& L) {
+  return L.H % 16 == 0 && L.H <= 64 * 16 * kGgufBlkCh;  // as launch_gguf_gateup: W = 16
+}
+static bool gguf_blk_down(const GgufMoeDev& L) {  // as launch_gguf_down_combine: W = 8
+  return L.H % 8 == 0 && L.I % 8 == 0 && L.Ish % 8 == 0 &&
+         (L.I > L.Ish ? L.I : L.Ish) <= 64 * 8 * kGgufBlkCh;
+}
+
+// The grouped form's grouping, two more launches and staging cost about 25 us;
+// what it saves grows with the row chunks (a row's share of one wave pass: 1024
+// weights of a gate or up row, 512 of a down row) that the token-by-token form
+// decodes again for every token, and with the cost of a type's decode there.
+// Measured over 2 .. 200 tokens at hidden / inter 2048 / 512, 1024 / 256 and
+// 256 / 128 (us per call, token by token against grouped, 2048 / 512: Q4_K 59 /
+// 46 at 2 tokens, 470 / 136 at 24, 2826 / 330 at 128; Q3_K 46 / 48 at 4, 74 / 66
+// at 8, 177 / 121 at 24; Q8_0 53 / 45 at 3, 319 / 163 at 24; 256 / 128: Q4_K 29 /
+// 30 at 12, Q3_K 37 / 36 at 48, Q8_0 30 / 31 at 32; 1280 / 128, Q8_0 at 10 tokens:
+// 37 / 40), the limits lie where the grouped form was the faster in all of them.
+// Shapes without the blocked kernels: from 128 tokens.
+bool gguf_units_pay(const GgufMoeDev& L, int T) {
+  if (!gguf_blk_gateup(L) || !gguf_blk_down(L)) return T >= 128;
+  const int64_t gu = 2 * ((int64_t)L.K * L.I + L.Ish) * ((L.H + 1023) / 1024);
+  const int64_t dn = (int64_t)L.H * ((int64_t)L.K * ((L.I + 511) / 512) + (L.Ish + 511) / 512);
+  const int64_t least = L.type == kGgmlQ4_K ? 56000 : L.type == kGgmlQ3_K ? 200000 : 120000;
+  return T * (gu + dn) >= least;
+}
+
+// Eight once the experts hold four or more each; four before, so that more
+// workgroups share a CU.
+int gguf_unit_tokens(const GgufMoeDev& L, int T) {
+  return (int64_t)T * L.K > 4 * (int64_t)L.E ? 8 : 4;
+}
+
 hipError_t launch_gguf_units(const GgufMoeDev& L, const float* x, int T, const int32_t* off,
                              const int32_t* perm, const int2* units, const int32_t* meta,
                              int nunits, float* h, int ldh, float* parts, const float* probs,
@@ -1540,36 +1777,45 @@ hipError_t launch_gguf_units(const GgufMoeDev& L, const float* x, int T, const i
       ldh < L.I || ldh < L.Ish)
     return hipErrorInvalidValue;
   const int rows = L.I > L.Ish ? L.I : L.Ish;
-  // rows per wave of the blocked forms: one for few tokens (the units hold
-  // one or two, and more waves hide more latency), up to eight as the units fill
-  const int rpw = T >= 512 ? kGgufBlkRowsMax : T >= 128 ? 4 : T >= 32 ? 2 : 1;  // (T >= 128 in use)
+  // Blocked forms: tokens staged at a time (four while the units hold few
+  // more, so that more workgroups share a CU) and rows per wave.
+  const int usz = gguf_unit_tokens(L, T);
+  const bool tm8 = usz == 8;
+  // rows per wave: enough waves for the device first, then fewer of them
+  const auto rpw_of = [&](int64_t n) { return n >= 49152 ? 16 : n >= 24576 ? 8 : 4; };
+  const int rpw_g = rpw_of((int64_t)nunits * rows), rpw_d = rpw_of((int64_t)nunits * L.H / 2);
+  if (tm8 && L.H > 1024) {
+    const hipError_t e = gguf_blk_attrs();
+    if (e != hipSuccess) return e;
+  }
+  const auto blocks = [](int n, int rpw) { return (unsigned)((n + 4 * rpw - 1) / (4 * rpw)); };
   for (int u0 = 0; u0 < nunits; u0 += 65535) {
     const int n = nunits - u0 < 65535 ? nunits - u0 : 65535;
     const dim3 grid((unsigned)((rows + 3) / 4), (unsigned)n);
-    if (L.H % 16 == 0 && L.H <= 64 * 16 * kGgufBlkCh) {  // as launch_gguf_gateup: W = 16
-      const dim3 gb((unsigned)((rows + 4 * rpw - 1) / (4 * rpw)), (unsigned)n);
-      DM_GGUF_DISPATCH_T(k_gguf_gateup_units_blk, gb, L, x, off, perm, units, meta, T, h, ldh,
-                         status, u0, rpw)
+    if (gguf_blk_gateup(L)) {
+      const dim3 gb(blocks(rows, rpw_g), (unsigned)n);
+      const size_t lds = (size_t)(tm8 ? 8 : 4) * ((L.H + 1023) / 1024) * (4096 + 256);
+      DM_GGUF_DISPATCH_BLK(k_gguf_gateup_units_blk, gb, lds, L, x, off, perm, units, meta, T, h,
+                           ldh, status, u0, rpw_g)
     } else if (L.H % 16 == 0) {
       DM_GGUF_DISPATCH_W(k_gguf_gateup_units, 16, grid, L, x, off, perm, units, meta, T, h, ldh,
-                         status, u0)
+                         status, u0, usz)
     } else {
       DM_GGUF_DISPATCH(k_gguf_gateup_units, grid, L, x, off, perm, units, meta, T, h, ldh, status,
-                       u0)
+                       u0, usz)
     }
   }
   for (int u0 = 0; u0 < nunits; u0 += 65535) {
     const int n = nunits - u0 < 65535 ? nunits - u0 : 65535;
     const dim3 grid((unsigned)((L.H + 3) / 4), (unsigned)n);
-    const int nmax = L.I > L.Ish ? L.I : L.Ish;
-    if (L.H % 8 == 0 && L.I % 8 == 0 && L.Ish % 8 == 0 && nmax <= 64 * 8 * kGgufBlkCh) {
-      // as launch_gguf_down_combine: W = 8
-      const dim3 gb((unsigned)((L.H + 4 * rpw - 1) / (4 * rpw)), (unsigned)n);
-      DM_GGUF_DISPATCH_T(k_gguf_down_units_blk, gb, L, h, ldh, off, perm, units, meta, T, parts,
-                         status, u0, rpw)
+    if (gguf_blk_down(L)) {
+      const dim3 gb(blocks(L.H, rpw_d), (unsigned)n);
+      const size_t lds = (size_t)(tm8 ? 8 : 4) * ((rows + 511) / 512) * 2048;
+      DM_GGUF_DISPATCH_BLK(k_gguf_down_units_blk, gb, lds, L, h, ldh, off, perm, units, meta, T,
+                           parts, status, u0, rpw_d)
     } else {
       DM_GGUF_DISPATCH(k_gguf_down_units, grid, L, h, ldh, off, perm, units, meta, T, parts,
-                       status, u0)
+                       status, u0, usz)
     }
   }
   const int64_t nt = (int64_t)T * L.H;
@@ -1579,7 +1825,9 @@ hipError_t launch_gguf_units(const GgufMoeDev& L, const float* x, int T, const i
 }
 #undef DM_GGUF_DISPATCH
 #undef DM_GGUF_DISPATCH_W
-#undef DM_GGUF_DISPATCH_T
+#undef DM_GGUF_DISPATCH_BLK
+#undef DM_GGUF_DISPATCH_TM
+#undef DM_GGUF_BLK
 
 bool gguf_one_token_supported(const GgufMoeDev& L) {
   return L.H % 64 == 0 && L.H <= kFrontMaxH && L.I % 16 == 0 && L.I <= 512 && L.Ish % 8 == 0 &&

@@ -13,6 +13,8 @@ int persistent_wgs();
 
 // Upper bound of the work units for T tokens (size of the units buffer).
 int group_units_max(int T, int K, int E);
+// The same when every unit is a small one of up to tok tokens.
+int group_small_units_max(int T, int K, int E, int tok);
 
 // Tokens per work unit of launch_group_build: units[0 .. meta[1]) hold up to
 // kUnitBig of their expert's positions, units[meta[1] .. meta[0]) up to
@@ -21,9 +23,11 @@ int group_units_max(int T, int K, int E);
 constexpr int kUnitBig = 128;
 constexpr int kUnitSmall = 16;
 
-// Group the T*K assignments by expert: off [E+1], perm [T*K], units, meta[0].
+// Group the T*K assignments by expert: off [E+1], perm [T*K], units, meta.
+// With tok != 0 every unit is a small one of up to tok tokens (meta[1] = 0).
 hipError_t launch_group_build(const int32_t* ids, int T, int K, int E, int32_t* off,
-                              int32_t* perm, int2* units, int32_t* meta, hipStream_t st);
+                              int32_t* perm, int2* units, int32_t* meta, hipStream_t st,
+                              int tok = 0);
 
 // The front end of a small batch in one launch: x -> bf16 hi / lo rows and
 // need-lo (flags[0]), router logits z [T][E+1] in the layer order, softmax /

@@ -49,9 +49,15 @@ constexpr int kGThreads = 256;
 // big units.  An expert's c tokens form c / 128 full big units; a remainder
 // r > 32 is one more big unit, a remainder r <= 32 becomes ceil(r / 16) small
 // units.  Order: full routed units, full shared units, partial big routed
-// units, a partial big shared unit, then the small routed and shared units,
-// so that the costly workgroups start first.
-__device__ __forceinline__ void unit_split(int c, int& nf, int& pb, int& ps) {
+// units, a partial big shared unit, then the small shared units (the fuller
+// ones of a small batch) and the small routed ones, so that the costly
+// workgroups start first.  With tok != 0 every unit is a small one, of up to tok tokens.
+__device__ __forceinline__ void unit_split(int c, int tok, int& nf, int& pb, int& ps) {
+  if (tok) {
+    nf = pb = 0;
+    ps = (c + tok - 1) / tok;
+    return;
+  }
   const int r = c % kMT;
   nf = c / kMT;
   pb = r > 2 * kSmallMax;
@@ -62,7 +68,7 @@ __device__ __forceinline__ void unit_split(int c, int& nf, int& pb, int& ps) {
 // COH: ids are read with agent-scope loads (written in the same launch).
 template <bool COH>
 __device__ __forceinline__ void group_build_wg(const int32_t* __restrict__ ids, int T, int K, int E,
-                                               int32_t* __restrict__ off,
+                                               int tok, int32_t* __restrict__ off,
                                                int32_t* __restrict__ perm,
                                                int2* __restrict__ units,
                                                int32_t* __restrict__ meta, int* lds) {
@@ -71,7 +77,7 @@ __device__ __forceinline__ void group_build_wg(const int32_t* __restrict__ ids, 
   int* cnt = lds;
   int* cur = lds + E;
   int* sc = lds + 2 * E;
-  const int tid = threadIdx.x, TK = T * K;
+  const int tid = threadIdx.x, TK = T * K, small = tok ? tok : kSmallMax;
   for (int e = tid; e < E; e += 1024) cnt[e] = 0;
   __syncthreads();
   // the first kCache expert ids of this thread stay in registers for the
@@ -97,7 +103,7 @@ __device__ __forceinline__ void group_build_wg(const int32_t* __restrict__ ids, 
   int v[4] = {0, 0, 0, 0};
   for (int e = e0; e < e1; ++e) {
     int nf, pb, ps;
-    unit_split(cnt[e], nf, pb, ps);
+    unit_split(cnt[e], tok, nf, pb, ps);
     v[0] += cnt[e];
     v[1] += nf;
     v[2] += pb;
@@ -134,17 +140,17 @@ __device__ __forceinline__ void group_build_wg(const int32_t* __restrict__ ids, 
   }
   const int nf = tot[1], npb = tot[2], nps = tot[3];
   int snf, spb, sps;
-  unit_split(T, snf, spb, sps);
+  unit_split(T, tok, snf, spb, sps);
   const int pb0 = nf + snf, s0 = pb0 + npb + spb;
-  int base = pre[0], fb = pre[1], pb = pb0 + pre[2], ps = s0 + pre[3];
+  int base = pre[0], fb = pre[1], pb = pb0 + pre[2], ps = s0 + sps + pre[3];
   for (int e = e0; e < e1; ++e) {
     int nfe, pbe, pse;
-    unit_split(cnt[e], nfe, pbe, pse);
+    unit_split(cnt[e], tok, nfe, pbe, pse);
     off[e] = base;
     cur[e] = base;
     for (int i = 0; i < nfe; ++i) units[fb + i] = make_int2(e, kMT * i);
     if (pbe) units[pb++] = make_int2(e, kMT * nfe);
-    for (int i = 0; i < pse; ++i) units[ps++] = make_int2(e, kMT * nfe + kSmallMax * i);
+    for (int i = 0; i < pse; ++i) units[ps++] = make_int2(e, kMT * nfe + small * i);
     base += cnt[e];
     fb += nfe;
   }
@@ -160,28 +166,28 @@ __device__ __forceinline__ void group_build_wg(const int32_t* __restrict__ ids, 
     perm[atomicAdd(&cur[e], 1)] = a;
   }
   for (int i = tid; i < snf; i += 1024) units[nf + i] = make_int2(E, kMT * i);
+  for (int i = tid; i < sps; i += 1024) units[s0 + i] = make_int2(E, kMT * snf + small * i);
   if (tid == 0) {
     if (spb) units[pb0 + npb] = make_int2(E, kMT * snf);
-    for (int i = 0; i < sps; ++i) units[s0 + nps + i] = make_int2(E, kMT * snf + kSmallMax * i);
     meta[0] = s0 + nps + sps;
     meta[1] = s0;
   }
 }
 
 __global__ __launch_bounds__(1024) void k_group_build(const int32_t* __restrict__ ids, int T, int K,
-                                                      int E, int32_t* __restrict__ off,
+                                                      int E, int tok, int32_t* __restrict__ off,
                                                       int32_t* __restrict__ perm,
                                                       int2* __restrict__ units,
                                                       int32_t* __restrict__ meta) {
   extern __shared__ int lds[];
-  group_build_wg<false>(ids, T, K, E, off, perm, units, meta, lds);
+  group_build_wg<false>(ids, T, K, E, tok, off, perm, units, meta, lds);
 }
 
 hipError_t launch_group_build(const int32_t* ids, int T, int K, int E, int32_t* off,
-                              int32_t* perm, int2* units, int32_t* meta, hipStream_t st) {
+                              int32_t* perm, int2* units, int32_t* meta, hipStream_t st, int tok) {
   const size_t lds = (size_t)(2 * E + 64) * sizeof(int);
-  hipLaunchKernelGGL(k_group_build, dim3(1), dim3(1024), lds, st, ids, T, K, E, off, perm, units,
-                     meta);
+  hipLaunchKernelGGL(k_group_build, dim3(1), dim3(1024), lds, st, ids, T, K, E, tok, off,
+                     perm, units, meta);
   return hipGetLastError();
 }
 
@@ -366,7 +372,7 @@ __global__ __launch_bounds__(1024) void k_front(const float* __restrict__ x,
   __syncthreads();
   if (!last_tok) return;
   if (tid == 0) atomicExch(&flags[1], 0);
-  group_build_wg<true>(ids, T, L.K, E, off, perm, units, meta, reinterpret_cast<int*>(fl));
+  group_build_wg<true>(ids, T, L.K, E, 0, off, perm, units, meta, reinterpret_cast<int*>(fl));
 }
 
 bool front_supported(const LayerDev& L, int T) {
@@ -395,6 +401,12 @@ hipError_t launch_front(const LayerDev& L, const float* x, int T, float* z, uint
   else DM_FRONT(8);
 #undef DM_FRONT
   return hipGetLastError();
+}
+
+int group_small_units_max(int T, int K, int E, int tok) {
+  // an expert of c tokens has ceil(c / tok): at most c, and at most c / tok + 1
+  const long tk = (long)T * K, n = tk / tok + (tk < E ? tk : E);
+  return (int)(tk < n ? tk : n) + (T + tok - 1) / tok;
 }
 
 int group_units_max(int T, int K, int E) {
