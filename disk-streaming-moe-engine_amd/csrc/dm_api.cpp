@@ -377,7 +377,7 @@ struct BlockScratch {
   int32_t* needlo = nullptr;  // [kFlagInts] zero on entry: the need-lo flag (the combine
                               // clears it again) and the front-end arrival counters
                               // (reset by the front-end kernel itself)
-  int2* units = nullptr;      // [group_units_max(T, K, E)]
+  int2* units = nullptr;      // [group_units_max(T, K, E, unit_tok(T))]
   uint16_t* xhi = nullptr;    // [T][H] bf16 hi parts of x
   uint16_t* xlo = nullptr;    // [T][H] bf16 lo parts
   uint16_t* hr = nullptr;     // [2][T*K][I] routed h, hi then lo
@@ -406,7 +406,7 @@ size_t scratch_carve(const LayerDev& L, int T, bool norm, uint8_t* base, BlockSc
     t.perm = (int32_t*)take(TK * 4);
     t.meta = (int32_t*)take(2 * 4);
     t.needlo = (int32_t*)take(kFlagInts * 4);
-    t.units = (int2*)take((size_t)dm::group_units_max(T, L.K, L.E) * sizeof(int2));
+    t.units = (int2*)take((size_t)dm::group_units_max(T, L.K, L.E, dm::unit_tok(T)) * sizeof(int2));
     t.xhi = (uint16_t*)take(TH * 2);
     t.xlo = (uint16_t*)take(TH * 2);
     t.hr = (uint16_t*)take(2 * TK * L.I * 2);
@@ -442,7 +442,7 @@ hipError_t ctx_scratch(dmh_ctx* ctx, const LayerDev& L, int T, bool norm, BlockS
   if (ctx->g_needlo.cap != nl_cap &&
       (e = hipMemsetAsync(ctx->g_needlo.p, 0, kFlagInts * sizeof(int), ctx->cur)) != hipSuccess)
     return e;
-  if ((e = ctx->g_units.ensure(dm::group_units_max(T, L.K, L.E))) != hipSuccess) return e;
+  if ((e = ctx->g_units.ensure(dm::group_units_max(T, L.K, L.E, dm::unit_tok(T)))) != hipSuccess) return e;
   if ((e = ctx->g_xhi.ensure(TH)) != hipSuccess) return e;
   if ((e = ctx->g_xlo.ensure(TH)) != hipSuccess) return e;
   if ((e = ctx->g_hr.ensure(2 * TK * L.I)) != hipSuccess) return e;
@@ -561,8 +561,8 @@ hipError_t run_block(dmh_ctx* ctx, Layer* Ly, int layer, const float* dx, const 
     if ((e = dm::launch_router_select(sc->z, L.E + 1, T, L.E, L.K, 1, dids, dprobs, dshg,
                                       status, st)) != hipSuccess)
       return e;
-    if ((e = dm::launch_group_build(dids, T, L.K, L.E, sc->off, sc->perm, sc->units, sc->meta,
-                                    st)) != hipSuccess)
+    if ((e = dm::launch_group_build(dids, T, L.K, L.E, dm::unit_tok(T), sc->off, sc->perm, sc->units,
+                                    sc->meta, st)) != hipSuccess)
       return e;
     if ((e = dm::launch_experts_grouped(L, sc->xhi, sc->xlo, sc->needlo, sc->off, sc->perm,
                                         sc->units, sc->meta, T, sc->hr, sc->hr + TK * L.I, sc->hs,
@@ -689,16 +689,15 @@ hipError_t run_gguf_block(dmh_ctx* c, GgufLayer* G, unsigned long long* status, 
   if (T > 1 && L.E <= kGgufGroupMaxE && (dm::gguf_units_pay(L, T) || dm::gguf_mm_ok(L, T))) {
     // several tokens: grouped by expert, each expert row read once per unit
     const bool mm = dm::gguf_mm_ok(L, T);
-    const int tok = mm ? 0 : dm::gguf_unit_tokens(L, T);
-    const int nu = mm ? dm::group_units_max(T, L.K, L.E)
-                      : dm::group_small_units_max(T, L.K, L.E, tok);
+    const int tok = mm ? dm::kGgufMmTok : dm::gguf_unit_tokens(L, T);
+    const int nu = dm::group_units_max(T, L.K, L.E, tok);
     if ((e = c->g_off.ensure(L.E + 1)) != hipSuccess) return e;
     if ((e = c->g_perm.ensure((size_t)T * L.K)) != hipSuccess) return e;
     if ((e = c->g_meta.ensure(2)) != hipSuccess) return e;
     if ((e = c->g_units.ensure(nu)) != hipSuccess) return e;
     if ((e = c->g_r.ensure((size_t)T * (L.K + 1) * L.H)) != hipSuccess) return e;
-    if ((e = dm::launch_group_build(dids, T, L.K, L.E, c->g_off.p, c->g_perm.p, c->g_units.p,
-                                    c->g_meta.p, st, tok)) != hipSuccess)
+    if ((e = dm::launch_group_build(dids, T, L.K, L.E, tok, c->g_off.p, c->g_perm.p, c->g_units.p,
+                                    c->g_meta.p, st)) != hipSuccess)
       return e;
     if (mm) {
       // prefill: the experts' products on the matrix cores
@@ -1716,7 +1715,7 @@ int dmh_experts_forward(dmh_ctx* c, int layer, const float* x, int T, const int3
   HIP_TRY(c->g_perm.ensure(TK));
   HIP_TRY(c->g_meta.ensure(2));
   HIP_TRY(c->g_needlo.ensure(1));
-  HIP_TRY(c->g_units.ensure(dm::group_units_max(T, K, L.E)));
+  HIP_TRY(c->g_units.ensure(dm::group_units_max(T, K, L.E, dm::unit_tok(T))));
   HIP_TRY(c->g_xhi.ensure(TH));
   HIP_TRY(c->g_xlo.ensure(TH));
   HIP_TRY(c->g_hr.ensure(2 * TK * L.I));
@@ -1726,8 +1725,8 @@ int dmh_experts_forward(dmh_ctx* c, int layer, const float* x, int T, const int3
   HIP_TRY(c->g_rs.ensure(TH));
   HIP_TRY(hipMemsetAsync(c->g_needlo.p, 0, sizeof(int), st));
   HIP_TRY(dm::launch_split_rows(dx, (int64_t)TH, c->g_xhi.p, c->g_xlo.p, c->g_needlo.p, st));
-  HIP_TRY(dm::launch_group_build(c->uids.p, T, K, L.E, c->g_off.p, c->g_perm.p, c->g_units.p,
-                                 c->g_meta.p, st));
+  HIP_TRY(dm::launch_group_build(c->uids.p, T, K, L.E, dm::unit_tok(T), c->g_off.p, c->g_perm.p,
+                                 c->g_units.p, c->g_meta.p, st));
   float* drs = (dev && shared_out) ? shared_out : c->g_rs.p;
   HIP_TRY(dm::launch_experts_grouped(Lk, c->g_xhi.p, c->g_xlo.p, c->g_needlo.p, c->g_off.p,
                                      c->g_perm.p, c->g_units.p, c->g_meta.p, T, c->g_hr.p,

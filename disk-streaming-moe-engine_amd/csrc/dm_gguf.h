@@ -66,7 +66,7 @@ bool gguf_units_pay(const GgufMoeDev& L, int T);
 int gguf_unit_tokens(const GgufMoeDev& L, int T);
 // The same outputs for T tokens grouped by expert (off, perm, units, meta
 // of launch_group_build on ids with tok = gguf_unit_tokens; nunits =
-// group_small_units_max): each expert row is read and decoded once per unit
+// group_units_max): each expert row is read and decoded once per unit
 // instead of once per (token, slot).  Three launches: gate/up into h as launch_gguf_gateup, the
 // down projections into parts [T][K+1][H], then moe_aggregate_forward's
 // combine.  Every token's sums are formed by the same helpers in the same
@@ -88,6 +88,7 @@ hipError_t launch_gguf_tiles(const GgufMoeDev& L, uint8_t* out, hipStream_t st);
 // the bits of its own single-token call, whatever it is batched with; from
 // here on the sums run in the matrix cores' order (as exact, other bits).
 constexpr int kGgufMmMinT = 256;
+constexpr int kGgufMmTok = 128;  // tokens per unit
 bool gguf_mm_ok(const GgufMoeDev& L, int T);
 // Elements of the column sums of `elements` activations (0: not needed).
 size_t gguf_mm_sums(const GgufMoeDev& L, int64_t elements);
@@ -100,7 +101,7 @@ struct GgufMmScratch {
   float* h;        // [T K][I], [T][Ish]
 };
 // The experts' outputs of T tokens grouped by expert (off, perm, units, meta
-// of launch_group_build, nunits = group_units_max): r [T*K][H] by
+// of launch_group_build with tok = kGgufMmTok, nunits = group_units_max): r [T*K][H] by
 // assignment, rs [T][H] of the shared expert, unweighted, with the checks of
 // launch_gguf_units; launch_combine forms y from them.
 hipError_t launch_gguf_mm(const GgufMoeDev& L, const float* x, int T, const int32_t* off,

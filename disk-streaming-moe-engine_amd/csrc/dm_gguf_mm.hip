@@ -39,7 +39,7 @@ constexpr int kMmCols = 64;                   // columns of a record and of a st
 constexpr int kMmThreads = 512;               // 8 waves
 constexpr int kMmStages = 3;                  // stages in flight
 constexpr int kMmRowBytes = kMmCols * 2 * 2;  // a token row's hi and lo parts of a stage
-constexpr int kMmBBytes = kUnitBig * kMmRowBytes;
+constexpr int kMmBBytes = kGgufMmTok * kMmRowBytes;
 
 // Bytes of a record: the codes (lane l of a wave: row l & 15, columns
 // 8 (l >> 4) .. + 7 of each 32), then the scales.
@@ -52,7 +52,7 @@ struct Rec {
   static constexpr int kCodes = TY == kGgmlQ8_0 ? 1024 : 512;
   static constexpr int kRest = TY == kGgmlQ3_K ? 192 : TY == kGgmlQ4_K ? 256 : 128;
   static constexpr int kBytes = kCodes + kRest;
-  static constexpr int kSums = TY == kGgmlQ4_K ? kUnitBig * 16 : 0;  // column sums of a stage
+  static constexpr int kSums = TY == kGgmlQ4_K ? kGgufMmTok * 16 : 0;  // column sums of a stage
   static constexpr int kStage = kMmBBytes + 16 * kBytes + kSums;
   // direct-to-LDS loads per wave and stage, besides those of the token rows
   static constexpr int kDma = kCodes / 512 + 1 + (kSums ? 1 : 0);
@@ -281,31 +281,22 @@ __device__ __forceinline__ int mm_row(const MmArgs& g, const MmItem& it, int r) 
   return GU && !it.shared ? g.perm[p] / g.L.K : p;
 }
 
-// Item idx: the big units first, in 8 classes (idx % 8 is the XCD the
-// dispatcher places the workgroup on: a unit's row blocks share that XCD's L2
-// for its token rows, as in k_big), then the small ones.
+// Item idx, in 8 classes (idx % 8 is the XCD the dispatcher places the
+// workgroup on: a unit's row blocks share that XCD's L2 for its token rows,
+// as in k_experts).
 template <int TY, bool GU>
 __device__ __forceinline__ MmItem mm_item(const MmArgs& g, int idx, int nblk, int w, int lane) {
   MmItem it;
   it.valid = false;
-  const int nall = g.meta[0], nbig = g.meta[1], span = (nbig + 7) >> 3, nb = 8 * span * nblk;
-  int u, f;
-  if (idx < nb) {
-    const int i = idx >> 3, ul = i / nblk;
-    u = (idx & 7) * span + ul;
-    f = i - ul * nblk;
-    if (u >= nbig) return it;
-  } else {
-    u = nbig + (idx - nb) / nblk;
-    f = (idx - nb) % nblk;
-    if (u >= nall) return it;
-  }
+  const int nall = g.meta[0], span = (nall + 7) >> 3, i = idx >> 3, ul = i / nblk;
+  const int u = (idx & 7) * span + ul, f = i - ul * nblk;
+  if (ul >= span || u >= nall) return it;
   const GgufMoeDev& L = g.L;
   const int2 v = g.units[u];
   it.shared = v.x >= L.E;
   it.e = it.shared ? L.E : v.x;
   it.p0 = it.shared ? v.y : g.off[v.x] + v.y;
-  it.n = min(u < nbig ? kUnitBig : kUnitSmall, (it.shared ? g.T : g.off[v.x + 1]) - it.p0);
+  it.n = min(kGgufMmTok, (it.shared ? g.T : g.off[v.x + 1]) - it.p0);
   it.rows = it.shared ? L.Ish : L.I;
   it.fb = f;
   if (GU && f * 128 >= it.rows) return it;
@@ -337,7 +328,7 @@ __device__ __forceinline__ MmItem mm_item(const MmArgs& g, int idx, int nblk, in
     it.sums = g.sums + before / 16;
     it.srow = (uint32_t)mm_row<GU>(g, it, 16 * w + (lane & 15)) * (uint32_t)(it.KD / 16);
   }
-  if (threadIdx.x < kUnitBig) {
+  if (threadIdx.x < kGgufMmTok) {
     const int p = it.p0 + min((int)threadIdx.x, it.n - 1);
     const int a = it.shared ? p : g.perm[p];
     it.info = make_int2(a, g.ex[GU ? (it.shared ? p : a / L.K) : (it.shared ? g.T * L.K + p : p)]);
@@ -623,8 +614,8 @@ __device__ __forceinline__ void mm_run(const MmArgs& g, const unsigned char* lds
     // ... and after the barrier every wave's have, and nobody reads stage
     // ps - 1 any more, whose buffer stage ps + 2 takes
     __builtin_amdgcn_s_barrier();
-    if (ps == 0 && nxt.valid && threadIdx.x < kUnitBig)
-      const_cast<int2*>(info)[(par ^ 1) * kUnitBig + threadIdx.x] = nxt.info;
+    if (ps == 0 && nxt.valid && threadIdx.x < kGgufMmTok)
+      const_cast<int2*>(info)[(par ^ 1) * kGgufMmTok + threadIdx.x] = nxt.info;
     const uint32_t st = l0 + (uint32_t)((gb + ps + 2) % kMmStages * R::kStage);
     if (ps + 2 < cur.nst)
       mm_issue<TY>(cur, ps + 2, st, w, lane);
@@ -643,7 +634,7 @@ __device__ __forceinline__ void mm_run(const MmArgs& g, const unsigned char* lds
   for (int ct = 0; ct < NCT; ++ct) {
     const int c = 16 * ct + j;
     if (c < cur.n) {
-      const int2 in = info[par * kUnitBig + c];
+      const int2 in = info[par * kGgufMmTok + c];
       const int p = cur.p0 + c, a = in.x, ex = in.y;
       const uint32_t ph = cur.shared ? kPhShared : kPhExpert;
       if (GU) {
@@ -707,7 +698,7 @@ void k_gguf_mm(const int32_t* meta, const int2* units, const int32_t* off, const
   g.perm = perm;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int nblk = GU ? ((g.L.I > g.L.Ish ? g.L.I : g.L.Ish) + 127) / 128 : (g.L.H + 255) / 256;
-  const int items = (8 * ((meta[1] + 7) >> 3) + meta[0] - meta[1]) * nblk;
+  const int items = 8 * ((meta[0] + 7) >> 3) * nblk;
   const int step = gridDim.x;
   int idx = blockIdx.x;
   MmItem cur = mm_next<TY, GU>(g, idx, step, items, nblk, w, lane);
@@ -715,7 +706,7 @@ void k_gguf_mm(const int32_t* meta, const int2* units, const int32_t* off, const
   const uint32_t l0 = lds_u32(ldsm);
   mm_issue<TY>(cur, 0, l0, w, lane);
   mm_issue<TY>(cur, 1, l0 + Rec<TY>::kStage, w, lane);
-  if (threadIdx.x < kUnitBig)
+  if (threadIdx.x < kGgufMmTok)
     reinterpret_cast<int2*>(ldsm + kMmStages * Rec<TY>::kStage)[threadIdx.x] = cur.info;
   int gb = 0, par = 0;
   while (true) {
@@ -736,7 +727,7 @@ void k_gguf_mm(const int32_t* meta, const int2* units, const int32_t* off, const
 
 template <int TY>
 constexpr int mm_lds() {
-  return kMmStages * Rec<TY>::kStage + 2 * kUnitBig * (int)sizeof(int2);
+  return kMmStages * Rec<TY>::kStage + 2 * kGgufMmTok * (int)sizeof(int2);
 }
 template <int TY>
 hipError_t mm_attrs() {

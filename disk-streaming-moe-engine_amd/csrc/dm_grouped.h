@@ -11,23 +11,21 @@ namespace dm {
 // CU count rounded down to a multiple of 8 (0 when it cannot be read).
 int persistent_wgs();
 
-// Upper bound of the work units for T tokens (size of the units buffer).
-int group_units_max(int T, int K, int E);
-// The same when every unit is a small one of up to tok tokens.
-int group_small_units_max(int T, int K, int E, int tok);
+// Upper bound of the work units of up to tok tokens (size of the units buffer).
+int group_units_max(int T, int K, int E, int tok);
 
-// Tokens per work unit of launch_group_build: units[0 .. meta[1]) hold up to
-// kUnitBig of their expert's positions, units[meta[1] .. meta[0]) up to
-// kUnitSmall.  A unit is (expert, first position within the expert); the
-// expert E is the shared one, whose positions are the tokens.
-constexpr int kUnitBig = 128;
+// Tokens per work unit of launch_experts_grouped for calls of T tokens.  A
+// unit is (expert, first position within the expert); the expert E is the
+// shared one, whose positions are the tokens.
+constexpr int kUnitTok = 64;
 constexpr int kUnitSmall = 16;
+constexpr int kSmallMaxT = 32;
+constexpr int unit_tok(int T) { return T <= kSmallMaxT ? kUnitSmall : kUnitTok; }
 
-// Group the T*K assignments by expert: off [E+1], perm [T*K], units, meta.
-// With tok != 0 every unit is a small one of up to tok tokens (meta[1] = 0).
-hipError_t launch_group_build(const int32_t* ids, int T, int K, int E, int32_t* off,
-                              int32_t* perm, int2* units, int32_t* meta, hipStream_t st,
-                              int tok = 0);
+// Group the T*K assignments by expert: off [E+1], perm [T*K], units of up to
+// tok positions, meta[0] = number of units.
+hipError_t launch_group_build(const int32_t* ids, int T, int K, int E, int tok, int32_t* off,
+                              int32_t* perm, int2* units, int32_t* meta, hipStream_t st);
 
 // The front end of a small batch in one launch: x -> bf16 hi / lo rows and
 // need-lo (flags[0]), router logits z [T][E+1] in the layer order, softmax /

@@ -11,17 +11,15 @@
 //                   (matrix cores for bf16 activations), softmax, top-k
 //   k_group_build   one workgroup: count assignments per expert, scan,
 //                   scatter them into expert order, emit the work units
-//                   (expert, tile of up to 128 tokens); the shared expert is
-//                   expert E over all tokens.  Units of more than 16 tokens
-//                   ("big") come first, then the small ones.
+//                   (expert, up to 64 or 16 of its tokens); the shared expert is
+//                   expert E over all tokens
 //   k_split_rows    activations -> bf16 hi / lo rows
-//   k_big<true>     h = SiLU(W_g x) * (W_u x) for big units: token rows,
-//                   4-bit weights and scales all staged in LDS by
-//                   direct-to-LDS loads, three stages in flight, weights
+//   k_experts<true>  h = SiLU(W_g x) * (W_u x): token rows, 4-bit weights and
+//                   scales all staged in LDS by direct-to-LDS loads, weights
 //                   dequantised from LDS (16 features x 32 k per MFMA)
-//   k_gu_small      the same for units of <= 16 tokens: B fragments straight
-//                   from memory, no LDS and no barriers, deeper prefetch
-//   k_big<false> / k_down_small   r = W_d h, B = h as bf16 hi + lo parts
+//   k_experts<false> r = W_d h, B = h as bf16 hi + lo parts
+//   k_gu_small, k_down_small  the same for calls of a few tokens: operands
+//                   straight from memory, no LDS and no barriers
 //   k_combine       y = sum_k p_k r_k + g r_sh (+ residual), reference order
 //
 // Each token's outputs depend only on its own column of the MFMA tiles, so
@@ -36,35 +34,16 @@
 
 namespace dm {
 
-constexpr int kMT = 128;       // tokens per big work unit (8 MFMA column tiles of 16)
-constexpr int kNCT = kMT / 16;
-constexpr int kSmallMax = 16;  // units of at most this many tokens are small
 constexpr int kGThreads = 256;
 
 // ---------------------------------------------------------------------------
 // One workgroup of 1024 threads.  ids [T*K] in the reference order (slot k of
 // token t at t*K + k).  Outputs: off [E+1] expert offsets into perm, perm
-// [T*K] assignment indices grouped by expert, units [nmax] = (expert, first
-// position within the expert), meta[0] = number of units, meta[1] = number of
-// big units.  An expert's c tokens form c / 128 full big units; a remainder
-// r > 32 is one more big unit, a remainder r <= 32 becomes ceil(r / 16) small
-// units.  Order: full routed units, full shared units, partial big routed
-// units, a partial big shared unit, then the small shared units (the fuller
-// ones of a small batch) and the small routed ones, so that the costly
-// workgroups start first.  With tok != 0 every unit is a small one, of up to tok tokens.
-__device__ __forceinline__ void unit_split(int c, int tok, int& nf, int& pb, int& ps) {
-  if (tok) {
-    nf = pb = 0;
-    ps = (c + tok - 1) / tok;
-    return;
-  }
-  const int r = c % kMT;
-  nf = c / kMT;
-  pb = r > 2 * kSmallMax;
-  ps = (r > 0 && r <= 2 * kSmallMax) ? (r + kSmallMax - 1) / kSmallMax : 0;
-}
-
-// The grouping on one workgroup of 1024 threads, lds: (2 E + 64) ints.
+// [T*K] assignment indices grouped by expert, units = (expert, first position
+// within the expert) of up to tok positions each, meta[0] = number of units:
+// the shared expert's first (they are full), then the routed ones in expert
+// order.
+// The grouping on one workgroup of 1024 threads, lds: (2 E + 32) ints.
 // COH: ids are read with agent-scope loads (written in the same launch).
 template <bool COH>
 __device__ __forceinline__ void group_build_wg(const int32_t* __restrict__ ids, int T, int K, int E,
@@ -72,12 +51,11 @@ __device__ __forceinline__ void group_build_wg(const int32_t* __restrict__ ids, 
                                                int32_t* __restrict__ perm,
                                                int2* __restrict__ units,
                                                int32_t* __restrict__ meta, int* lds) {
-  // cnt[E] | cur[E] | wave totals of the 4 scans (counts, full units,
-  // partial big, small units), 16 waves each
+  // cnt[E] | cur[E] | wave totals of the 2 scans (counts, units), 16 waves each
   int* cnt = lds;
   int* cur = lds + E;
   int* sc = lds + 2 * E;
-  const int tid = threadIdx.x, TK = T * K, small = tok ? tok : kSmallMax;
+  const int tid = threadIdx.x, TK = T * K;
   for (int e = tid; e < E; e += 1024) cnt[e] = 0;
   __syncthreads();
   // the first kCache expert ids of this thread stay in registers for the
@@ -100,21 +78,17 @@ __device__ __forceinline__ void group_build_wg(const int32_t* __restrict__ ids, 
   __syncthreads();
   // thread tid owns experts [e0, e1)
   const int per = (E + 1023) / 1024, e0 = min(tid * per, E), e1 = min(e0 + per, E);
-  int v[4] = {0, 0, 0, 0};
+  int v[2] = {0, 0};
   for (int e = e0; e < e1; ++e) {
-    int nf, pb, ps;
-    unit_split(cnt[e], tok, nf, pb, ps);
     v[0] += cnt[e];
-    v[1] += nf;
-    v[2] += pb;
-    v[3] += ps;
+    v[1] += (cnt[e] + tok - 1) / tok;
   }
-  // exclusive prefix sums of the four counts over the threads: inclusive
+  // exclusive prefix sums of the two counts over the threads: inclusive
   // scans inside each wave (shuffles), then the 16 wave totals from LDS
   const int lane = tid & 63, wv = tid >> 6;
-  int incl[4];
+  int incl[2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < 2; ++i) {
     int a = v[i];
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -125,9 +99,9 @@ __device__ __forceinline__ void group_build_wg(const int32_t* __restrict__ ids, 
     if (lane == 63) sc[i * 16 + wv] = a;
   }
   __syncthreads();
-  int pre[4], tot[4];
+  int pre[2], tot[2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < 2; ++i) {
     int p = 0, t = 0;
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
@@ -138,21 +112,13 @@ __device__ __forceinline__ void group_build_wg(const int32_t* __restrict__ ids, 
     pre[i] = p + incl[i] - v[i];
     tot[i] = t;
   }
-  const int nf = tot[1], npb = tot[2], nps = tot[3];
-  int snf, spb, sps;
-  unit_split(T, tok, snf, spb, sps);
-  const int pb0 = nf + snf, s0 = pb0 + npb + spb;
-  int base = pre[0], fb = pre[1], pb = pb0 + pre[2], ps = s0 + sps + pre[3];
+  const int nsh = (T + tok - 1) / tok;
+  int base = pre[0], un = nsh + pre[1];
   for (int e = e0; e < e1; ++e) {
-    int nfe, pbe, pse;
-    unit_split(cnt[e], tok, nfe, pbe, pse);
     off[e] = base;
     cur[e] = base;
-    for (int i = 0; i < nfe; ++i) units[fb + i] = make_int2(e, kMT * i);
-    if (pbe) units[pb++] = make_int2(e, kMT * nfe);
-    for (int i = 0; i < pse; ++i) units[ps++] = make_int2(e, kMT * nfe + small * i);
+    for (int i = 0; i < cnt[e]; i += tok) units[un++] = make_int2(e, i);
     base += cnt[e];
-    fb += nfe;
   }
   if (tid == 0) off[E] = TK;
   __syncthreads();
@@ -165,13 +131,8 @@ __device__ __forceinline__ void group_build_wg(const int32_t* __restrict__ ids, 
     const int e = min(max((int)(COH ? ld_coh_i32(ids + a) : ids[a]), 0), E - 1);
     perm[atomicAdd(&cur[e], 1)] = a;
   }
-  for (int i = tid; i < snf; i += 1024) units[nf + i] = make_int2(E, kMT * i);
-  for (int i = tid; i < sps; i += 1024) units[s0 + i] = make_int2(E, kMT * snf + small * i);
-  if (tid == 0) {
-    if (spb) units[pb0 + npb] = make_int2(E, kMT * snf);
-    meta[0] = s0 + nps + sps;
-    meta[1] = s0;
-  }
+  for (int i = tid; i < nsh; i += 1024) units[i] = make_int2(E, tok * i);
+  if (tid == 0) meta[0] = nsh + tot[1];
 }
 
 __global__ __launch_bounds__(1024) void k_group_build(const int32_t* __restrict__ ids, int T, int K,
@@ -183,9 +144,9 @@ __global__ __launch_bounds__(1024) void k_group_build(const int32_t* __restrict_
   group_build_wg<false>(ids, T, K, E, tok, off, perm, units, meta, lds);
 }
 
-hipError_t launch_group_build(const int32_t* ids, int T, int K, int E, int32_t* off,
-                              int32_t* perm, int2* units, int32_t* meta, hipStream_t st, int tok) {
-  const size_t lds = (size_t)(2 * E + 64) * sizeof(int);
+hipError_t launch_group_build(const int32_t* ids, int T, int K, int E, int tok, int32_t* off,
+                              int32_t* perm, int2* units, int32_t* meta, hipStream_t st) {
+  const size_t lds = (size_t)(2 * E + 32) * sizeof(int);
   hipLaunchKernelGGL(k_group_build, dim3(1), dim3(1024), lds, st, ids, T, K, E, tok, off,
                      perm, units, meta);
   return hipGetLastError();
@@ -372,7 +333,7 @@ __global__ __launch_bounds__(1024) void k_front(const float* __restrict__ x,
   __syncthreads();
   if (!last_tok) return;
   if (tid == 0) atomicExch(&flags[1], 0);
-  group_build_wg<true>(ids, T, L.K, E, 0, off, perm, units, meta, reinterpret_cast<int*>(fl));
+  group_build_wg<true>(ids, T, L.K, E, unit_tok(T), off, perm, units, meta, reinterpret_cast<int*>(fl));
 }
 
 bool front_supported(const LayerDev& L, int T) {
@@ -385,7 +346,7 @@ hipError_t launch_front(const LayerDev& L, const float* x, int T, float* z, uint
                         unsigned long long* status, hipStream_t st) {
   if (!front_supported(L, T)) return hipErrorInvalidValue;
   const size_t sel = (size_t)(((L.E + 3) & ~3) + 8) * sizeof(float);
-  const size_t bld = (size_t)(2 * L.E + 64) * sizeof(int);
+  const size_t bld = (size_t)(2 * L.E + 32) * sizeof(int);
   const size_t xs = (size_t)L.H * sizeof(float);
   const size_t lds = sel > bld ? (sel > xs ? sel : xs) : (bld > xs ? bld : xs);
   const dim3 grid((L.E + 1 + 63) / 64, T);
@@ -403,31 +364,10 @@ hipError_t launch_front(const LayerDev& L, const float* x, int T, float* z, uint
   return hipGetLastError();
 }
 
-int group_small_units_max(int T, int K, int E, int tok) {
+int group_units_max(int T, int K, int E, int tok) {
   // an expert of c tokens has ceil(c / tok): at most c, and at most c / tok + 1
   const long tk = (long)T * K, n = tk / tok + (tk < E ? tk : E);
   return (int)(tk < n ? tk : n) + (T + tok - 1) / tok;
-}
-
-int group_units_max(int T, int K, int E) {
-  // per expert at most c / 128 + 2 units (two small units of a remainder <= 32)
-  return 2 * E + (T * K + kMT - 1) / kMT + (T + kMT - 1) / kMT + 2;
-}
-
-// Bounds of the two unit kinds, for the launch grids (the exact counts are
-// known on the device only).  Small units: each holds at least one
-// assignment and an expert has at most two (its remainder <= 32), the
-// shared expert at most two as well.  Big units: the full ones of all
-// assignments (routed and shared), plus at most one partial per expert with
-// more than 32 tokens in its remainder, and the shared expert's.
-static int small_units_max(int T, int K, int E) {
-  const long tk = (long)T * K;
-  return (int)(tk < 2L * E ? tk : 2L * E) + 2;
-}
-static int big_units_max(int T, int K, int E) {
-  const long tk = (long)T * K;
-  const long partial = tk / (2 * kSmallMax + 1);
-  return (int)(tk / kMT + T / kMT + (partial < E ? partial : E) + 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -463,8 +403,7 @@ hipError_t launch_split_rows(const float* x, int64_t n, uint16_t* hi, uint16_t* 
 // ---------------------------------------------------------------------------
 // Token rows of a unit (e, start): row r is position p = off[e] + start + r
 // of the expert order, i.e. assignment a = perm[p] of token a / K; for the
-// shared expert (e == E) row r is token start + r itself.  Big units hold up
-// to kMT rows, small units up to kSmallMax.
+// shared expert (e == E) row r is token start + r itself.
 struct UnitTokens {
   int e, p0, n;   // expert, first position, tokens in this unit
   bool shared;
@@ -644,324 +583,289 @@ __device__ __forceinline__ void down_epilogue(const GroupArgs& g, const UnitToke
 }
 
 // ---------------------------------------------------------------------------
-// Big-unit workgroups come in classes b % 8, and the dispatcher places all
-// workgroups of a class on one XCD (it hands a launch's workgroups to the
-// XCDs in rotation).  The big units are cut into 8 contiguous ranges (the
-// units of one expert are adjacent in the unit list) and range c runs in
-// class c with each unit's feature blocks next to each other: the blocks of
-// a unit share that XCD's L2 for the unit's token rows, and the units of an
-// expert share it for the expert's weights.  Item (unit u, block f) of
-// workgroup b; false when b has no item.
-__device__ __forceinline__ bool big_item(int b, int nbig, int nblk, int& u, int& f) {
-  const int c = b & 7, idx = b >> 3;
-  const int span = (nbig + 7) >> 3;
-  const int ul = idx / nblk;
-  u = c * span + ul;
-  f = idx - ul * nblk;
-  return ul < span && u < nbig;
-}
-static int big_grid(int nbig, int nblk) { return 8 * ((nbig + 7) / 8) * nblk; }
-
-// ---------------------------------------------------------------------------
-// Big units (17..128 tokens): k_big<GU>.  A workgroup of 8 waves takes one
-// unit and 128 features (gate/up: gate and up tiles rb0 + w of wave w, so
-// that h = SiLU(g) * u is formed in its registers) or 256 output rows (down:
-// tiles rb0 + 2w, rb0 + 2w + 1 of wave w), all 8 column tiles of the unit
-// (columns past its tokens are never stored).  Every operand is staged in
-// LDS by direct-to-LDS loads (global_load_lds_dwordx4: 16 bytes per lane
-// land in LDS without passing through registers), three stages in flight:
-//   - B rows: 128 rows x 256 bytes per k-step, segment sigma of row r stored
-//     at position sigma ^ (r & 15) of its row, so that the 16 rows of one
-//     MFMA B operand read distinct LDS banks;
-//   - A: the step's 16 A16 chunks (2 per wave) as they lie in memory, and
-//     their scales.
-// B rows are bf16 hi parts, and when the activations are not all bf16
-// values (h always; x when the need-lo flag is set) the lo parts too: then
-// a k-step is two stages, hi then lo, with the same A (read twice, the
-// second time from L2) and both products summed into the accumulators.
-// One barrier per stage: after it, stage s is complete everywhere and the
-// buffer of stage s - 1 is free for stage s + 2.
-constexpr int kB2Threads = 512;
-constexpr int kB2Stages = 3;
-constexpr int kB2RowBytes = kQuadCols * 2;                // one token row of a k-step
-constexpr int kB2BBytes = kMT * kB2RowBytes;               // 32 KB
-constexpr int kB2ABytes = 16 * 1024;                       // 16 A16 chunks
-constexpr int kB2SBytes = 16 * 128;                        // their scales
-constexpr int kB2Stage = kB2BBytes + kB2ABytes + kB2SBytes;  // 51200 bytes
-constexpr size_t kB2Lds = (size_t)kB2Stages * kB2Stage;    // 153600 bytes
-constexpr int kB2DmaPerStage = 7;                          // DMA instructions per wave and stage
-
-// 16 bytes per lane from p to LDS at byte address m + 16 * lane (m uniform
-// per wave): dma16_lds, inline assembly.  The compiler, which cannot tell the
-// stages of one LDS array apart, would otherwise wait for every load in
-// flight before any LDS read.  The kernel counts these loads itself
-// (s_waitcnt vmcnt); a load the compiler tracks is only ever waited for longer
-// because of them.  LDS addresses are 32-bit offsets from lds_u32 of the
-// array: arithmetic on a generic pointer into LDS makes the compiler build
-// the 64-bit address, which it cannot always lower.
-// The B fragments of 8 column tiles (rows 16 ct + j of a staged k-step,
-// 16 * 256 bytes apart) as 8 LDS reads in flight together.  Inline assembly
-// again: the compiler would otherwise sink each read next to its first use,
-// leaving two in flight.  Their registers are not valid before lds_wait8.
-__device__ __forceinline__ void lds_read8(uint32_t a, bf16x8 (&b)[kNCT]) {
-  static_assert(kNCT == 8 && 16 * kB2RowBytes == 4096, "offsets below");
-  asm volatile(
-      "ds_read_b128 %0, %8\n\tds_read_b128 %1, %8 offset:4096\n\t"
-      "ds_read_b128 %2, %8 offset:8192\n\tds_read_b128 %3, %8 offset:12288\n\t"
-      "ds_read_b128 %4, %8 offset:16384\n\tds_read_b128 %5, %8 offset:20480\n\t"
-      "ds_read_b128 %6, %8 offset:24576\n\tds_read_b128 %7, %8 offset:28672"
-      : "=&v"(b[0]), "=&v"(b[1]), "=&v"(b[2]), "=&v"(b[3]), "=&v"(b[4]), "=&v"(b[5]),
-        "=&v"(b[6]), "=&v"(b[7])
-      : "v"(a));
-}
-// Wait until at most N LDS operations are in flight (LDS operations complete
-// in order, so every read issued before the last N has landed); b's
-// registers are tied to the wait, so no use of them moves above it.
-template <int N>
-__device__ __forceinline__ void lds_wait8(bf16x8 (&b)[kNCT]) {
-  asm volatile("s_waitcnt lgkmcnt(%8)"
-               : "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]), "+v"(b[4]), "+v"(b[5]),
-                 "+v"(b[6]), "+v"(b[7])
-               : "n"(N));
-}
-
-__device__ __forceinline__ void gu_small_part(const GroupArgs& g, int bx, int by, int w);
-__device__ __forceinline__ void down_small_part(const GroupArgs& g, int bx, int by, int w);
-
-// One big item (unit ui, feature / row block fb) as seen by one lane: what
-// the DMA of its stages needs (its A views and tiles, its B rows) and what
-// its epilogue needs.
-struct BigItem {
-  bool valid;
-  UnitTokens ut;
-  int I, fb, nst, nGQ, KD, t0, t1, st_;
-  bool lo;
-  ExpertView v0, v1;
-  const uint16_t* bhi;
-  const uint16_t* blo;
-  uint32_t rowo[4];  // this lane's B row offsets (elements) of the four DMA rows
+// k_experts<GU>: a workgroup of 8 waves takes one unit (up to 64 tokens) and
+// 128 features (gate/up: gate and up tile 8 f + w of wave w, so that h =
+// SiLU(g) * u is formed in its registers) or 256 output rows (down: tiles
+// 16 f + 2w, 16 f + 2w + 1 of wave w).  A unit of n tokens runs with the
+// column tiles it needs (NCT: 1, 2 or 4 of 16 tokens).  Every operand is
+// staged in LDS by direct-to-LDS loads (global_load_lds_dwordx4: 16 bytes per
+// lane land in LDS without passing through registers), D stages ahead:
+//   - B rows: 256 bytes per token and stage, segment sigma of row r stored at
+//     position sigma ^ (r & 15) of its row, so that the 16 rows of one MFMA B
+//     operand read distinct LDS banks;
+//   - A: a k-step's 16 A16 chunks (16 rows x 128 columns, 2 per wave) as they
+//     lie in memory, and their scales.
+// A stage is 128 columns of the bf16 hi parts, or, when the activations are
+// not all bf16 values (LO: h always; x when the need-lo flag is set), 64
+// columns of the hi and of the lo parts: then a chunk serves two stages, its
+// weights dequantised once for both parts.  One barrier per stage: after it,
+// stage s is complete everywhere and the buffer of stage s - 1 is free.
+//
+// At most 128 registers and 78 KB of LDS, so that two workgroups share a CU:
+// one's matrix instructions run while the other waits for its stage or its
+// first loads (one workgroup per CU on 128-token units waited for a third of
+// its time and lost a quarter of the launch to the last round of items).
+// Workgroups are dispatched as others end; they come in classes b % 8, which
+// the dispatcher places on one XCD each (it hands a launch's workgroups to the
+// XCDs in rotation).  The units are cut into 8 contiguous ranges (the units of
+// an expert are adjacent) and range c runs in class c with each unit's blocks
+// next to each other: they share that XCD's L2 for the unit's token rows, and
+// the units of an expert for its weights.
+//
+// Bound by the matrix and vector units together from some 32 tokens a unit
+// (every weight is rounded to bf16 on the way, 1.75 operations), below by the
+// weights' bytes.  Against that former kernel, at hidden 2048, inter 512, 256
+// experts: 1533 fp32 tokens, gate/up 291 -> 168 us and down 166 + 13 -> 95; 2048
+// bf16 tokens (Zipf) 152 -> 134 and 125 + 24 -> 108; 131 tokens 91 -> 70 and 23 + 47
+// -> 45 (290 MB of weights in the 70: 4.1 TB/s; a copy reaches 5.1).
+constexpr int kExThreads = 512;
+constexpr int kExRowBytes = 256;                        // a token row of a stage
+constexpr int kExChunks = 16 * 1024;                    // 16 A16 chunks
+constexpr int kExABytes = kExChunks + 16 * 128;         // and their scales
+constexpr int kExADma = 3;                              // loads of a chunk pair per wave
+template <int NCT>
+struct ExStages {
+  static constexpr int kAhead = NCT == 4 ? 1 : 2;       // stages in flight
+  static constexpr int kBufs = kAhead + 1;
+  static constexpr int kB = 16 * NCT * kExRowBytes;
+  static constexpr int kBuf = kB + kExABytes;
+  static constexpr int kRowLoads = NCT == 4 ? 2 : 1;    // of 32 rows over the 8 waves
 };
+constexpr int cmax(int a, int b) { return a > b ? a : b; }
+constexpr int kExLds = cmax(ExStages<4>::kBufs * ExStages<4>::kBuf,
+                            cmax(ExStages<2>::kBufs * ExStages<2>::kBuf,
+                                 ExStages<1>::kBufs * ExStages<1>::kBuf));
+static_assert(2 * kExLds <= 160 * 1024, "two workgroups per CU");
 
-template <bool GU>
-__device__ __forceinline__ BigItem big_item_state(const GroupArgs& g, int idx, int items,
-                                                  int nblk, int w, int lane) {
-  BigItem it;
-  it.valid = false;
-  int ui, fb;
-  if (idx >= items || !big_item(idx, g.meta[1], nblk, ui, fb)) return it;
-  const LayerDev& L = g.L;
-  const int H = L.H, K = L.K;
-  it.ut = unit_tokens(g.units[ui], g.off, L.E, g.T, kMT);
-  it.I = it.ut.shared ? L.Ish : L.I;
-  it.fb = fb;
-  if (GU && fb * 128 >= it.I) return it;  // uniform per workgroup
-  it.KD = GU ? H : it.I;  // reduction length
-  it.nGQ = it.KD / kQuadCols;
-  it.lo = GU ? g.need_lo[0] != 0 : true;
-  it.nst = it.lo ? 2 * it.nGQ : it.nGQ;
-  if (GU) {
-    const size_t mat = (size_t)it.I * H;
-    it.v0 = it.ut.shared ? ExpertView{L.sgu_nib, L.sgu_sc, it.I, H}
-                         : ExpertView{L.gu_nib + (size_t)it.ut.e * mat,
-                                      L.gu_sc + (size_t)it.ut.e * 2 * (mat / kGroup), it.I, H};
-    it.v1 = {it.v0.nib + mat / 2, it.v0.sc + mat / kGroup, it.I, H};
-    it.t0 = it.t1 = fb * 8 + w;
-  } else {
-    const size_t mat = (size_t)H * it.I;
-    it.v0 = it.ut.shared ? ExpertView{L.sd_nib, L.sd_sc, H, it.I}
-                         : ExpertView{L.d_nib + (size_t)it.ut.e * (mat / 2),
-                                      L.d_sc + (size_t)it.ut.e * (mat / kGroup), H, it.I};
-    it.v1 = it.v0;
-    // H is a multiple of 128, so the last block may hold 128 rows: waves
-    // past H load tiles 0 and 1 (their share of the B rows is still needed)
-    // and store nothing
-    it.t0 = fb * 256 + 32 * w < H ? fb * 16 + 2 * w : 0;
-    it.t1 = it.t0 + 1;
-  }
-  it.bhi = GU ? g.xhi : (it.ut.shared ? g.hsh : g.hrh);
-  it.blo = GU ? g.xlo : (it.ut.shared ? g.hsl : g.hrl);
-  // B rows: instructions i = w + 8 m (m < 4) carry rows 4i..4i+3, lane L
-  // row 4i + L/16, stored segment L % 16 = global segment (L % 16) ^ (row & 15)
+// The B fragments of N column tiles (rows 16 ct + j of a stage, 16 * 256 bytes
+// apart) as N LDS reads in flight together.  Inline assembly: the compiler
+// would otherwise sink each read next to its first use.  Their registers are
+// not valid before lds_wait.
+template <int N>
+__device__ __forceinline__ void lds_read(uint32_t a, bf16x8 (&b)[N]) {
 #pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    const int r = 4 * (w + 8 * m) + (lane >> 4);
-    const int p = it.ut.p0 + min(r, it.ut.n - 1);
-    const int sg = (lane & 15) ^ (r & 15);
-    const int row = !GU ? p : it.ut.shared ? p : g.perm[p] / K;  // h rows by position, x by token
-    it.rowo[m] = (uint32_t)row * (uint32_t)it.KD + sg * 8;
-  }
-  it.st_ = lane < 8 ? it.t0 : it.t1;
-  it.valid = true;
-  return it;
+  for (int ct = 0; ct < N; ++ct)
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(b[ct]) : "v"(a), "n"(ct * 16 * kExRowBytes));
+}
+// Wait until at most M LDS operations are in flight (LDS operations complete
+// in order, so every read issued before the last M has landed); b's
+// registers are tied to the wait, so no use of them moves above it.
+template <int M, int N>
+__device__ __forceinline__ void lds_wait(bf16x8 (&b)[N]) {
+  if constexpr (N == 4)
+    asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]) : "n"(M));
+  else if constexpr (N == 2)
+    asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(b[0]), "+v"(b[1]) : "n"(M));
+  else
+    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(b[0]) : "n"(M));
+}
+// Until at most n of this wave's memory operations are in flight (uniform).
+__device__ __forceinline__ void vm_wait(int n) {
+  static_assert(kExADma == 3, "0, a stage's row load, a chunk pair, or both");
+  if (n == 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+  else if (n == 3) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
+  else if (n == 1) asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
+  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-// The first valid item at idx, idx + step, ... (idx advanced past it).
-template <bool GU>
-__device__ __forceinline__ BigItem big_next_item(const GroupArgs& g, int& idx, int step, int items,
-                                                 int nblk, int w, int lane) {
-  BigItem it;
-  it.valid = false;
-  while (idx < items) {
-    it = big_item_state<GU>(g, idx, items, nblk, w, lane);
-    idx += step;
-    if (it.valid) break;
-  }
-  return it;
-}
+// One unit's block on NCT column tiles.
+template <bool GU, bool LO, int NCT>
+struct ExRun {
+  using S = ExStages<NCT>;
+  const uint8_t* a0;  // this wave's two tiles
+  const uint8_t* a1;
+  const uint8_t* sc;  // this lane's 16 bytes of their scales (lanes 0 .. 15)
+  const uint16_t* b[S::kRowLoads];  // this lane's 8 columns of its token rows
+  uint32_t l0;
+  int w, lane, nst, nrow;           // stages; row loads of this wave and stage
+  uint4 c0, c1;
+  uint2 s0, s1;
+  f32x4 acc[2][NCT];
 
-// Workgroups 0 .. big_wgs - 1 are persistent: workgroup b takes the big
-// items (big_item index space 0 .. items - 1) b, b + big_wgs, ...; with
-// big_wgs a multiple of 8, every item of b is of class b % 8, on b's XCD.
-// The stage pipeline runs on across items: the first two stages of the
-// next item are requested during the last two stages of the current one,
-// so they land while its epilogue runs (the start latency of a workgroup,
-// ~3.4 us, is paid once per workgroup instead of once per item).
-// Workgroups from big_wgs on run the small units of the same stage (sx x sy
-// four-wave parts, two per workgroup): dispatched after every big one, they
-// fill the CUs the big items' last round leaves idle.
-// (The grouping's arrays lead the arguments, preloaded at dispatch: they
-// start each workgroup's chain of dependent loads.)
-template <bool GU>
-__global__ __launch_bounds__(kB2Threads) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void k_big(int items, int big_wgs, const int32_t* meta, const int2* units, const int32_t* off,
-           const int32_t* perm, const int* need_lo, GroupArgs gk, int sx, int sy) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char lds2[];
-  GroupArgs g = gk;
-  g.meta = meta;
-  g.units = units;
-  g.off = off;
-  g.perm = perm;
-  g.need_lo = need_lo;
-  if ((int)blockIdx.x >= big_wgs) {
-    const int w = gwave_id();
-    const int s = 2 * ((int)blockIdx.x - big_wgs) + (w >> 2);
-    if (s < sx * sy) {
-      if (GU)
-        gu_small_part(g, s % sx, s / sx, w & 3);
-      else
-        down_small_part(g, s % sx, s / sx, w & 3);
+  __device__ __forceinline__ void issue_b(int s) {
+    const uint32_t st = l0 + (uint32_t)(s % S::kBufs * S::kBuf);
+    if (NCT > 1 || nrow) {  // uniform
+#pragma unroll
+      for (int m = 0; m < S::kRowLoads; ++m)
+        dma16_lds(b[m] + s * (LO ? 64 : 128), st + (uint32_t)((w + 8 * m) * 1024));
     }
-    return;
   }
-  const LayerDev& L = g.L;
-  const int H = L.H;
-  const int nblk = GU ? ((L.I > L.Ish ? L.I : L.Ish) + 127) / 128 : (H + 255) / 256;
-  const int tid = threadIdx.x, w = gwave_id(), lane = tid & 63, q = lane >> 4, j = lane & 15;
-  int idx = blockIdx.x;
-  BigItem cur = big_next_item<GU>(g, idx, big_wgs, items, nblk, w, lane);
-  if (!cur.valid) return;  // uniform per workgroup
-  // this lane's part of the DMA of a stage:
-  //   B rows: 4 instructions of 4 rows (rowo)
-  //   A: chunk 2w (tile t0) and chunk 2w + 1 (tile t1)
-  //   scales: lanes 0..15 carry the 2 x 128 bytes of the same two chunks
-  auto issue = [&](const BigItem& it, int ps, int buf) {
-    const int s = it.lo ? ps >> 1 : ps;
-    const uint16_t* src = (it.lo && (ps & 1)) ? it.blo : it.bhi;
-    const uint32_t st = lds_u32(lds2) + (uint32_t)(buf * kB2Stage);
+  __device__ __forceinline__ void issue_a(int c) {
+    const uint32_t st = l0 + (uint32_t)(c % S::kBufs * S::kBuf + S::kB);
+    dma16_lds(a0 + (c * 64 + lane) * 16, st + (uint32_t)(2 * w * 1024));
+    dma16_lds(a1 + (c * 64 + lane) * 16, st + (uint32_t)((2 * w + 1) * 1024));
+    // scales of the two chunks: 128 bytes each, lanes 0..7 and 8..15
+    if (lane < 16) dma16_lds(sc + c * 128, st + (uint32_t)(kExChunks + w * 256));
+  }
+
+  // Stage s (LO: ODD: the second one of its chunk).  The B fragments of step
+  // z + 1 (a group of 32 columns; LO: of its hi, then its lo part) are read
+  // while step z multiplies.
+  template <bool ODD>
+  __device__ __forceinline__ void stage(int s, const unsigned char* lds) {
+    // this wave's loads of stage s have landed; in flight may be those of
+    // stage s + 1 (where two are ahead) and, at the odd stage of a chunk, the
+    // next chunk's
+    const bool more = s + 1 < nst;
+    int n = S::kAhead > 1 && more ? nrow : 0;
+    if (LO ? ODD && more : S::kAhead > 1 && more) n += kExADma;
+    vm_wait(n);
+    // ... and after the barrier every wave's, and nobody reads stage s - 1
+    __builtin_amdgcn_s_barrier();
+    if (s + S::kAhead < nst) {
+      issue_b(s + S::kAhead);
+      if (!LO) issue_a(s + S::kAhead);
+    }
+    const int c = LO ? s >> 1 : s;
+    if (LO && !ODD && s + 2 < nst) issue_a(c + 1);
+    const int q = lane >> 4, j = lane & 15;
+    if (!LO || !ODD) {
+      const unsigned char* a = lds + c % S::kBufs * S::kBuf + S::kB;
+      c0 = *reinterpret_cast<const uint4*>(a + 2 * w * 1024 + lane * 16);
+      c1 = *reinterpret_cast<const uint4*>(a + (2 * w + 1) * 1024 + lane * 16);
+      s0 = *reinterpret_cast<const uint2*>(a + kExChunks + w * 256 + j * 8);
+      s1 = *reinterpret_cast<const uint2*>(a + kExChunks + w * 256 + 128 + j * 8);
+    }
+    const uint32_t bp = l0 + (uint32_t)(s % S::kBufs * S::kBuf + j * kExRowBytes);
+    auto seg = [&](int z) { return (uint32_t)(((LO ? 8 * (z & 1) + 4 * (z >> 1) : 4 * z) + q) ^ j) * 16; };
+    bf16x8 bb[2][NCT], d0, d1;
+    lds_read<NCT>(bp + seg(0), bb[0]);
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
-      dma16_lds(src + it.rowo[m] + s * kQuadCols, st + (uint32_t)((w + 8 * m) * 1024));
-    dma16_lds(it.v0.nib + a16_nib_offset(it.nGQ, it.t0, s, lane), st + (uint32_t)(kB2BBytes + 2 * w * 1024));
-    dma16_lds(it.v1.nib + a16_nib_offset(it.nGQ, it.t1, s, lane),
-              st + (uint32_t)(kB2BBytes + (2 * w + 1) * 1024));
-    // scales of the two chunks: 128 bytes each, lanes 0..7 and 8..15 (only
-    // 16 lanes write: 256 bytes at the wave's own place)
-    if (lane < 16)
-      dma16_lds(reinterpret_cast<const unsigned char*>((lane < 8 ? it.v0 : it.v1).sc +
-                                                       a16_sc_offset(it.nGQ, it.st_, s, 0)) +
-                    (lane & 7) * 16,
-                st + (uint32_t)(kB2BBytes + kB2ABytes + w * 256));
-  };
-  issue(cur, 0, 0);
-  issue(cur, 1, 1);  // every item has at least two stages (checked at launch)
-  int gb = 0;        // stage count of the items before cur (buffer of its stage ps: (gb + ps) % 3)
-  while (true) {
-    // the next item's state (its loads wait, at the latest, for cur's first
-    // two stages, which stage 0 waits for anyway)
-    const BigItem nxt = big_next_item<GU>(g, idx, big_wgs, items, nblk, w, lane);
-    // the epilogue's assignments, requested now: a load issued after the next
-    // item's first stages would wait for them
-    int aa[kNCT];
-    unit_assignments<kNCT>(g, cur.ut, j, aa);
-    f32x4 acc[2][kNCT];
+    for (int z = 0; z < 4; ++z) {
+      if (z < 3) lds_read<NCT>(bp + seg(z + 1), bb[(z + 1) & 1]);
+      if (!LO || !(z & 1)) {
+        const int kk = LO ? (ODD ? 2 : 0) + (z >> 1) : z;
+        d0 = dequant8(word_of(c0, kk), scale_of(s0, kk));
+        d1 = dequant8(word_of(c1, kk), scale_of(s1, kk));
+      }
+      if (z < 3)
+        lds_wait<NCT>(bb[z & 1]);
+      else
+        lds_wait<0>(bb[z & 1]);
+#pragma unroll
+      for (int ct = 0; ct < NCT; ++ct) {
+        acc[0][ct] = mfma16(d0, bb[z & 1][ct], acc[0][ct]);
+        acc[1][ct] = mfma16(d1, bb[z & 1][ct], acc[1][ct]);
+      }
+    }
+  }
+
+  __device__ __forceinline__ void run(const GroupArgs& g, const UnitTokens& ut, int I, int fb,
+                                      const unsigned char* lds) {
+    const LayerDev& L = g.L;
+    const int H = L.H, K = L.K;
+    w = gwave_id();
+    lane = threadIdx.x & 63;
+    l0 = lds_u32(lds);
+    const int q = lane >> 4, j = lane & 15;
+    const int KD = GU ? H : I, nGQ = KD / kQuadCols;  // reduction length, chunks
+    nst = LO ? 2 * nGQ : nGQ;
+    const size_t mat = (size_t)I * H;
+    const uint8_t* nib;
+    const uint16_t* scl;
+    int t0, t1;
+    if (GU) {
+      nib = ut.shared ? L.sgu_nib : L.gu_nib + (size_t)ut.e * mat;
+      scl = ut.shared ? L.sgu_sc : L.gu_sc + (size_t)ut.e * 2 * (mat / kGroup);
+      t0 = fb * 8 + w;
+      t1 = I / kTileRows + t0;  // the up matrix follows the gate's tiles
+    } else {
+      nib = ut.shared ? L.sd_nib : L.d_nib + (size_t)ut.e * (mat / 2);
+      scl = ut.shared ? L.sd_sc : L.d_sc + (size_t)ut.e * (mat / kGroup);
+      // H is a multiple of 128, so the last block may hold 128 rows: waves
+      // past H load tiles 0 and 1 (their share of the B rows is still needed)
+      // and store nothing
+      t0 = fb * 256 + 32 * w < H ? fb * 16 + 2 * w : 0;
+      t1 = t0 + 1;
+    }
+    a0 = nib + a16_nib_offset(nGQ, t0, 0, 0);
+    a1 = nib + a16_nib_offset(nGQ, t1, 0, 0);
+    sc = reinterpret_cast<const uint8_t*>(scl + a16_sc_offset(nGQ, lane < 8 ? t0 : t1, 0, 0)) +
+         (lane & 7) * 16;
+    // B rows: load m of wave w carries rows 4 (w + 8m) .. + 3, lane l row
+    // 4 (w + 8m) + l / 16, stored segment l % 16 = segment (l % 16) ^ (row & 15)
+    // (of 16: 128 hi columns; LO: 64 hi, then 64 lo columns)
+    nrow = NCT > 1 || w < 4 ? S::kRowLoads : 0;
+    const int sg = (lane & 15) ^ ((4 * w + q) & 15);
+    const uint16_t* hi = GU ? g.xhi : (ut.shared ? g.hsh : g.hrh);
+    const uint16_t* lo = GU ? g.xlo : (ut.shared ? g.hsl : g.hrl);
+    const uint16_t* src = LO ? (sg < 8 ? hi : lo) + (sg & 7) * 8 : hi + sg * 8;
+#pragma unroll
+    for (int m = 0; m < S::kRowLoads; ++m) {
+      const int p = ut.p0 + min(4 * (w + 8 * m) + q, ut.n - 1);
+      const int row = !GU || ut.shared ? p : g.perm[p] / K;  // h rows by position, x by token
+      b[m] = src + (size_t)row * KD;
+    }
+    issue_b(0);
+    issue_a(0);
+    if (S::kAhead > 1 && nst > 1) {
+      issue_b(1);
+      if (!LO) issue_a(1);
+    }
+    int aa[NCT];
+    unit_assignments<NCT>(g, ut, j, aa);
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int ct = 0; ct < kNCT; ++ct) acc[t][ct] = f32x4{0, 0, 0, 0};
-    for (int ps = 0; ps < cur.nst; ++ps) {
-      // this wave's loads of stage ps have landed (one later stage may be in flight)
-      // (the first stage of an item after the first: everything, since the
-      // previous epilogue's stores were issued after this stage's loads and
-      // a count of outstanding operations cannot tell them apart)
-      static_assert(kB2DmaPerStage == 7, "the wait below counts one stage of 7 loads");
-      if ((ps + 1 < cur.nst || nxt.valid) && !(ps == 0 && gb > 0))
-        asm volatile("s_waitcnt vmcnt(7)" ::: "memory");
-      else
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      // every wave's loads of stage ps have landed, and every wave has finished
-      // reading stage ps - 1 (whose buffer the next issue overwrites)
-      __builtin_amdgcn_s_barrier();
-      const int gs = gb + ps;
-      if (ps + 2 < cur.nst)
-        issue(cur, ps + 2, (gs + 2) % kB2Stages);
-      else if (nxt.valid)
-        issue(nxt, ps + 2 - cur.nst, (gs + 2) % kB2Stages);
-      const unsigned char* st = lds2 + (gs % kB2Stages) * kB2Stage;
-      const uint4 c0 = *reinterpret_cast<const uint4*>(st + kB2BBytes + 2 * w * 1024 + lane * 16);
-      const uint4 c1 =
-          *reinterpret_cast<const uint4*>(st + kB2BBytes + (2 * w + 1) * 1024 + lane * 16);
-      const uint2 s0 =
-          *reinterpret_cast<const uint2*>(st + kB2BBytes + kB2ABytes + w * 256 + j * 8);
-      const uint2 s1 =
-          *reinterpret_cast<const uint2*>(st + kB2BBytes + kB2ABytes + w * 256 + 128 + j * 8);
-      // The 8 B fragments of k-group kk + 1 are read while kk computes.
-      bf16x8 bc[kNCT], bn[kNCT];
-      const uint32_t bp = lds_u32(lds2) + (uint32_t)((gs % kB2Stages) * kB2Stage + j * kB2RowBytes);
-      lds_read8(bp + (q ^ j) * 16, bc);
-#pragma unroll
-      for (int kk = 0; kk < kGroupsPerQuad; ++kk) {
-        if (kk + 1 < kGroupsPerQuad) lds_read8(bp + ((4 * (kk + 1) + q) ^ j) * 16, bn);
-        const bf16x8 a0 = dequant8(word_of(c0, kk), scale_of(s0, kk));
-        const bf16x8 a1 = dequant8(word_of(c1, kk), scale_of(s1, kk));
-        if (kk + 1 < kGroupsPerQuad)
-          lds_wait8<kNCT>(bc);
-        else
-          lds_wait8<0>(bc);
-#pragma unroll
-        for (int ct = 0; ct < kNCT; ++ct) {
-          acc[0][ct] = mfma16(a0, bc[ct], acc[0][ct]);
-          acc[1][ct] = mfma16(a1, bc[ct], acc[1][ct]);
-        }
-        if (kk + 1 < kGroupsPerQuad) {
-#pragma unroll
-          for (int ct = 0; ct < kNCT; ++ct) bc[ct] = bn[ct];
-        }
+      for (int ct = 0; ct < NCT; ++ct) acc[t][ct] = f32x4{0, 0, 0, 0};
+    if (LO) {
+      for (int s = 0; s < nst; s += 2) {
+        stage<false>(s, lds);
+        stage<true>(s + 1, lds);
       }
+    } else {
+      for (int s = 0; s < nst; ++s) stage<false>(s, lds);
     }
     if (GU)
-      gu_epilogue<2, kNCT>(g, cur.ut, cur.I, cur.fb * 128 + 16 * w, q, j, acc, aa);
-    else if (cur.fb * 256 + 32 * w < H)
-      down_epilogue<2, kNCT>(g, cur.ut, cur.I, cur.fb * 256 + 32 * w, q, j, acc, aa);
-    if (!nxt.valid) break;  // uniform
-    gb += cur.nst;
-    cur = nxt;
+      gu_epilogue<2, NCT>(g, ut, I, fb * 128 + 16 * w, q, j, acc, aa);
+    else if (fb * 256 + 32 * w < H)
+      down_epilogue<2, NCT>(g, ut, I, fb * 256 + 32 * w, q, j, acc, aa);
   }
+};
+
+template <bool GU, bool LO>
+__device__ __forceinline__ void ex_unit(const GroupArgs& g, const UnitTokens& ut, int I, int fb,
+                                        const unsigned char* lds) {
+  if (ut.n <= 16) ExRun<GU, LO, 1>().run(g, ut, I, fb, lds);
+  else if (ut.n <= 32) ExRun<GU, LO, 2>().run(g, ut, I, fb, lds);
+  else ExRun<GU, LO, 4>().run(g, ut, I, fb, lds);
 }
 
-// k_big's LDS (150 KB) is above the default limit of a launch: raised once
-// per device.
-static hipError_t big_attrs() {
+// (The grouping's arrays lead the arguments, preloaded at dispatch: they
+// start each workgroup's chain of dependent loads.)
+template <bool GU>
+__global__ __launch_bounds__(kExThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void k_experts(const int32_t* meta, const int2* units, const int32_t* off, const int32_t* perm,
+               const int* need_lo, int nblk, GroupArgs gk) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds2[];
+  GroupArgs g = gk;
+  g.perm = perm;
+  const int nall = meta[0], span = (nall + 7) >> 3, idx = (int)blockIdx.x >> 3;
+  const int ul = idx / nblk, fb = idx - ul * nblk, u = ((int)blockIdx.x & 7) * span + ul;
+  if (ul >= span || u >= nall) return;
+  const UnitTokens ut = unit_tokens(units[u], off, g.L.E, g.T, kUnitTok);
+  const int I = ut.shared ? g.L.Ish : g.L.I;
+  if (GU && fb * 128 >= I) return;  // uniform per workgroup
+  if (!GU || need_lo[0] != 0)
+    ex_unit<GU, true>(g, ut, I, fb, lds2);
+  else
+    ex_unit<GU, false>(g, ut, I, fb, lds2);
+}
+
+// k_experts' LDS is above the default limit of a launch: raised once per
+// device.
+static hipError_t ex_attrs() {
   static std::atomic<uint64_t> done{0};
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   const uint64_t bit = dev < 64 ? 1ull << dev : 0;
   if (bit && (done.load() & bit)) return hipSuccess;
-  e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_big<true>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kB2Lds);
+  e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_experts<true>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, kExLds);
   if (e == hipSuccess)
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_big<false>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kB2Lds);
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_experts<false>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kExLds);
   if (e == hipSuccess) done.fetch_or(bit);
   return e;
 }
@@ -980,12 +884,18 @@ int persistent_wgs() {
 }
 
 // ---------------------------------------------------------------------------
-// Small units (<= 16 tokens): one column tile.  Waves are independent (no
-// LDS, no barrier): each wave owns 2 A tiles (gate/up: 16 features, gate and
-// up tile; down: 32 output rows) and reads its B fragments (lane (q, j):
-// token j, columns 8q..8q+7 of each group) straight from memory into the
-// same prefetch ring as the A chunks, P k-steps ahead.  At most 168 registers
-// per lane, so that three waves share a SIMD and their loads overlap.
+// Calls of at most kSmallMaxT tokens: units of up to 16, one column tile.
+// Their few workgroups are bound by the latency of their stages, so waves are
+// independent (no LDS, no barrier): each wave owns 2 A tiles (gate/up: 16
+// features, gate and up tile; down: 32 output rows) and reads its B fragments
+// (lane (q, j): token j, columns 8q..8q+7 of each group) straight from memory
+// into the same prefetch ring as the A chunks, P k-steps ahead.  At most 168
+// registers per lane, so that three waves share a SIMD and their loads
+// overlap.  Through k_experts instead, weights from HBM: 2 tokens 46 us per
+// call against 37, 12 tokens 68 against 63, 24 tokens 91 against 83 (fp32
+// activations 112 against 110), 32 tokens 94 against 90 (115 against 121); at 48
+// tokens, where the shared expert fills three units, it is 112 against the 139 of
+// one workgroup per CU on 128-token units beside these kernels.
 constexpr int kSmallTiles = 2;
 
 template <bool LO>
@@ -1052,17 +962,14 @@ __device__ __forceinline__ void small_loop(const ExpertView& v0, const ExpertVie
     if (s0 + u < ns) small_step<LO>(ring[u], acc);
 }
 
-static_assert(kMT == kUnitBig && kSmallMax == kUnitSmall, "unit sizes of dm_grouped.h");
 constexpr int kSmallGuCols = 4 * 16;   // features per small gate/up workgroup
 constexpr int kSmallDnRows = 4 * 32;   // output rows per small down workgroup
 
-// Small gate/up unit bx (of those after the big ones), features by * 64 ..,
-// on wave w of four; no barriers, so that four waves of a larger workgroup
-// can run it too.
+// Gate/up of unit bx, features by * 64 .., on wave w of four.
 __device__ __forceinline__ void gu_small_part(const GroupArgs& g, int bx, int by, int w) {
-  const int ui = g.meta[1] + bx;
+  const int ui = bx;
   if (ui >= g.meta[0]) return;
-  const UnitTokens ut = unit_tokens(g.units[ui], g.off, g.L.E, g.T, kSmallMax);
+  const UnitTokens ut = unit_tokens(g.units[ui], g.off, g.L.E, g.T, kUnitSmall);
   const LayerDev& L = g.L;
   const int H = L.H, K = L.K, I = ut.shared ? L.Ish : L.I;
   const int lane = threadIdx.x & 63, q = lane >> 4, j = lane & 15;
@@ -1087,11 +994,11 @@ __device__ __forceinline__ void gu_small_part(const GroupArgs& g, int bx, int by
   gu_epilogue<kSmallTiles, 1>(g, ut, I, f0, q, j, acc, aa);
 }
 
-// Small down unit bx, output rows by * 128 .., on wave w of four.
+// Down of unit bx, output rows by * 128 .., on wave w of four.
 __device__ __forceinline__ void down_small_part(const GroupArgs& g, int bx, int by, int w) {
-  const int ui = g.meta[1] + bx;
+  const int ui = bx;
   if (ui >= g.meta[0]) return;
-  const UnitTokens ut = unit_tokens(g.units[ui], g.off, g.L.E, g.T, kSmallMax);
+  const UnitTokens ut = unit_tokens(g.units[ui], g.off, g.L.E, g.T, kUnitSmall);
   const LayerDev& L = g.L;
   const int H = L.H, I = ut.shared ? L.Ish : L.I;
   const int lane = threadIdx.x & 63, q = lane >> 4, j = lane & 15;
@@ -1142,45 +1049,27 @@ hipError_t launch_experts_grouped(const LayerDev& L, const uint16_t* xhi, const 
                                   float* rs, unsigned long long* status, hipStream_t st) {
   const GroupArgs g = {L, xhi, xlo, need_lo, off, perm, units, meta, T,
                        hrh, hrl, hsh, hsl, r, rs, status};
-  const int nu = group_units_max(T, L.K, L.E);
-  // grids sized by the bound of each unit kind, so that few workgroups
-  // start only to find no unit (each still costs a dispatch and its first
-  // instructions)
-  const int nbig = min(nu, big_units_max(T, L.K, L.E));
-  const int nsmall = min(nu, small_units_max(T, L.K, L.E));
-  const int imax = L.I > L.Ish ? L.I : L.Ish;
-  // an expert holds at most T tokens (its ids per token are distinct), so
-  // units of more than 2 * kSmallMax tokens need T > 2 * kSmallMax
-  const bool big = T > 2 * kSmallMax;
-  // the big items' B row offsets are 32-bit element offsets
-  if ((size_t)T * L.K * imax >= (1ull << 32) || (size_t)T * L.H >= (1ull << 32))
+  if ((size_t)T * L.K * (L.I > L.Ish ? L.I : L.Ish) >= (1ull << 32) ||
+      (size_t)T * L.H >= (1ull << 32))
     return hipErrorInvalidValue;
-  if (big) {
-    const hipError_t e = big_attrs();
-    if (e != hipSuccess) return e;
-  }
-  const int gy = (imax + kSmallGuCols - 1) / kSmallGuCols, dy = (L.H + kSmallDnRows - 1) / kSmallDnRows;
-  if (big) {
-    // the small gate/up units ride in the big gate/up grid, after the big
-    // units, and fill the CUs its last round leaves idle; the down stage's
-    // big units run about five rounds, so its small units keep their own
-    // launch (dispatched after every big one they would add rounds)
-    const int bg = big_grid(nbig, (imax + 127) / 128), bd = big_grid(nbig, (L.H + 255) / 256);
-    // persistent big workgroups: one per CU (150 KB of LDS each), a multiple
-    // of 8 so that an item keeps its class; every item needs two stages or
-    // more (gate/up: H / 128 of them, down: 2 I / 128)
-    const int pw = L.H >= 256 ? persistent_wgs() : 0;
-    const int wg_g = pw > 0 && pw < bg ? pw : bg, wg_d = pw > 0 && pw < bd ? pw : bd;
-    hipLaunchKernelGGL(k_big<true>, dim3(wg_g + (nsmall * gy + 1) / 2), dim3(kB2Threads), kB2Lds,
-                       st, bg, wg_g, meta, units, off, perm, need_lo, g, nsmall, gy);
-    hipLaunchKernelGGL(k_big<false>, dim3(wg_d), dim3(kB2Threads), kB2Lds, st, bd, wg_d, meta,
-                       units, off, perm, need_lo, g, 0, 0);
-  } else {
-    hipLaunchKernelGGL(k_gu_small, dim3(nsmall, gy), dim3(kGThreads), 0, st, meta, units, off, perm,
+  if (T <= kSmallMaxT) {
+    const int nu = group_units_max(T, L.K, L.E, kUnitSmall);
+    const int gy = ((L.I > L.Ish ? L.I : L.Ish) + kSmallGuCols - 1) / kSmallGuCols;
+    const int dy = (L.H + kSmallDnRows - 1) / kSmallDnRows;
+    hipLaunchKernelGGL(k_gu_small, dim3(nu, gy), dim3(kGThreads), 0, st, meta, units, off, perm, g);
+    hipLaunchKernelGGL(k_down_small, dim3(nu, dy), dim3(kGThreads), 0, st, meta, units, off, perm,
                        g);
+    return hipGetLastError();
   }
-  hipLaunchKernelGGL(k_down_small, dim3(nsmall, dy), dim3(kGThreads), 0, st, meta, units, off,
-                     perm, g);
+  const hipError_t e = ex_attrs();
+  if (e != hipSuccess) return e;
+  // a grid for the most units there can be; those past the units end at once
+  const int classes = 8 * ((group_units_max(T, L.K, L.E, kUnitTok) + 7) / 8);
+  const int gb = ((L.I > L.Ish ? L.I : L.Ish) + 127) / 128, db = (L.H + 255) / 256;
+  hipLaunchKernelGGL(k_experts<true>, dim3(classes * gb), dim3(kExThreads), kExLds, st, meta, units,
+                     off, perm, need_lo, gb, g);
+  hipLaunchKernelGGL(k_experts<false>, dim3(classes * db), dim3(kExThreads), kExLds, st, meta,
+                     units, off, perm, need_lo, db, g);
   return hipGetLastError();
 }
 
