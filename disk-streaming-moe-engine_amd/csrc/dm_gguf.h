@@ -88,7 +88,7 @@ hipError_t launch_gguf_tiles(const GgufMoeDev& L, uint8_t* out, hipStream_t st);
 // the bits of its own single-token call, whatever it is batched with; from
 // here on the sums run in the matrix cores' order (as exact, other bits).
 constexpr int kGgufMmMinT = 256;
-constexpr int kGgufMmTok = 128;  // tokens per unit
+constexpr int kGgufMmTok = 64;  // tokens per unit
 bool gguf_mm_ok(const GgufMoeDev& L, int T);
 // Elements of the column sums of `elements` activations (0: not needed).
 size_t gguf_mm_sums(const GgufMoeDev& L, int64_t elements);

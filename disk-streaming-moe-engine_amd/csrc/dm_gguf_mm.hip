@@ -37,9 +37,7 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kMmCols = 64;                   // columns of a record and of a stage
 constexpr int kMmThreads = 512;               // 8 waves
-constexpr int kMmStages = 3;                  // stages in flight
 constexpr int kMmRowBytes = kMmCols * 2 * 2;  // a token row's hi and lo parts of a stage
-constexpr int kMmBBytes = kGgufMmTok * kMmRowBytes;
 
 // Bytes of a record: the codes (lane l of a wave: row l & 15, columns
 // 8 (l >> 4) .. + 7 of each 32), then the scales.
@@ -52,10 +50,20 @@ struct Rec {
   static constexpr int kCodes = TY == kGgmlQ8_0 ? 1024 : 512;
   static constexpr int kRest = TY == kGgmlQ3_K ? 192 : TY == kGgmlQ4_K ? 256 : 128;
   static constexpr int kBytes = kCodes + kRest;
-  static constexpr int kSums = TY == kGgmlQ4_K ? kGgufMmTok * 16 : 0;  // column sums of a stage
-  static constexpr int kStage = kMmBBytes + 16 * kBytes + kSums;
-  // direct-to-LDS loads per wave and stage, besides those of the token rows
+  static constexpr bool kSums = TY == kGgmlQ4_K;  // column sums in a stage
+  // direct-to-LDS loads of a wave and stage besides those of the token rows
   static constexpr int kDma = kCodes / 512 + 1 + (kSums ? 1 : 0);
+};
+// Stages of NCT column tiles: token rows, the 16 tiles' codes, their scales,
+// the column sums.  Two workgroups share a CU (160 KB).
+template <int TY, int NCT>
+struct MmBuf {
+  static constexpr int kAhead = NCT == 4 ? 1 : 2;     // stages in flight
+  static constexpr int kBufs = kAhead + 1;
+  static constexpr int kB = 16 * NCT * kMmRowBytes;
+  static constexpr int kSumsAt = kB + 16 * Rec<TY>::kBytes;
+  static constexpr int kBytes = kSumsAt + (Rec<TY>::kSums ? 16 * NCT * 16 : 0);
+  static constexpr int kRowLoads = NCT == 4 ? 2 : 1;  // of 32 rows over the 8 waves
 };
 int rec_bytes(int type) {
   switch (type) {
@@ -260,154 +268,28 @@ struct MmArgs {
   unsigned long long* status;
 };
 
-struct MmItem {
-  bool valid, shared;
-  int e, p0, n;       // expert, first position (shared: first token), tokens
-  int rows, fb, KD;   // I or Ish, block of rows, reduction length
-  int nst, nm, dma;   // stages, 32-row groups of token rows, loads per wave and stage
-  const uint8_t* t0;  // this wave's two tiles
-  const uint8_t* t1;
-  const uint16_t* b;
-  const uint16_t* sums;
-  uint32_t rowo[4];   // this lane's token row offsets (elements) of its loads
-  uint32_t srow;      // and its column sums'
-  int2 info;          // threads 0 .. 127: assignment and exponent of position threadIdx.x
+struct MmUnit {
+  bool shared;
+  int e, p0, n;  // expert, first position (shared: first token), tokens
+  int rows, fb;  // I or Ish, block of rows
 };
-
-// row of token rows of position r (0 .. n - 1) of a unit
-template <bool GU>
-__device__ __forceinline__ int mm_row(const MmArgs& g, const MmItem& it, int r) {
-  const int p = it.p0 + min(r, it.n - 1);
-  return GU && !it.shared ? g.perm[p] / g.L.K : p;
-}
-
-// Item idx, in 8 classes (idx % 8 is the XCD the dispatcher places the
-// workgroup on: a unit's row blocks share that XCD's L2 for its token rows,
-// as in k_experts).
-template <int TY, bool GU>
-__device__ __forceinline__ MmItem mm_item(const MmArgs& g, int idx, int nblk, int w, int lane) {
-  MmItem it;
-  it.valid = false;
-  const int nall = g.meta[0], span = (nall + 7) >> 3, i = idx >> 3, ul = i / nblk;
-  const int u = (idx & 7) * span + ul, f = i - ul * nblk;
-  if (ul >= span || u >= nall) return it;
-  const GgufMoeDev& L = g.L;
-  const int2 v = g.units[u];
-  it.shared = v.x >= L.E;
-  it.e = it.shared ? L.E : v.x;
-  it.p0 = it.shared ? v.y : g.off[v.x] + v.y;
-  it.n = min(kGgufMmTok, (it.shared ? g.T : g.off[v.x + 1]) - it.p0);
-  it.rows = it.shared ? L.Ish : L.I;
-  it.fb = f;
-  if (GU && f * 128 >= it.rows) return it;
-  it.KD = GU ? L.H : it.rows;
-  it.nst = it.KD / kMmCols;
-  it.nm = (it.n + 31) >> 5;
-  it.dma = it.nm + Rec<TY>::kDma;
-  const uint8_t* m0 = L.tiles + tile_offset(L.E, L.H, L.I, L.Ish, Rec<TY>::kBytes, it.e, GU ? 0 : 2);
-  const size_t rb = (size_t)it.nst * Rec<TY>::kBytes;  // bytes of 16 rows
-  if (GU) {
-    it.t0 = m0 + (size_t)(f * 8 + w) * rb;
-    it.t1 = it.t0 + (size_t)(it.rows / 16) * rb;
-  } else {
-    // H is a multiple of 128: waves past it (in the last block) load rows
-    // 0 .. 31 and store nothing
-    it.t0 = m0 + (size_t)(f * 256 + 32 * w < L.H ? f * 16 + 2 * w : 0) * rb;
-    it.t1 = it.t0 + rb;
-  }
-  const size_t before = !GU && it.shared ? (size_t)g.T * L.K * L.I : 0;
-  it.b = g.b + 2 * before;
-#pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    const int r = 4 * (w + 8 * m) + (lane >> 4);
-    // stored segment lane & 15 of row r is its segment (lane & 15) ^ (r & 15)
-    it.rowo[m] = (uint32_t)mm_row<GU>(g, it, r) * (uint32_t)(2 * it.KD) +
-                 (uint32_t)(((lane & 15) ^ (r & 15)) * 8);
-  }
-  if (TY == kGgmlQ4_K) {
-    it.sums = g.sums + before / 16;
-    it.srow = (uint32_t)mm_row<GU>(g, it, 16 * w + (lane & 15)) * (uint32_t)(it.KD / 16);
-  }
-  if (threadIdx.x < kGgufMmTok) {
-    const int p = it.p0 + min((int)threadIdx.x, it.n - 1);
-    const int a = it.shared ? p : g.perm[p];
-    it.info = make_int2(a, g.ex[GU ? (it.shared ? p : a / L.K) : (it.shared ? g.T * L.K + p : p)]);
-  }
-  it.valid = true;
-  return it;
-}
-
-template <int TY, bool GU>
-__device__ __forceinline__ MmItem mm_next(const MmArgs& g, int& idx, int step, int items, int nblk,
-                                          int w, int lane) {
-  MmItem it;
-  it.valid = false;
-  while (idx < items) {
-    it = mm_item<TY, GU>(g, idx, nblk, w, lane);
-    idx += step;
-    if (it.valid) break;
-  }
-  return it;
-}
-
-// This wave's loads of stage s of an item into the stage buffer at LDS
-// address st.
-template <int TY>
-__device__ __forceinline__ void mm_issue(const MmItem& it, int s, uint32_t st, int w, int lane) {
-  using R = Rec<TY>;
-#pragma unroll
-  for (int m = 0; m < 4; ++m)
-    if (m < it.nm)  // uniform
-      dma16_lds(it.b + it.rowo[m] + (uint32_t)s * (2 * kMmCols), st + (uint32_t)((w + 8 * m) * 1024));
-  const uint8_t* r0 = it.t0 + (size_t)s * R::kBytes;
-  const uint8_t* r1 = it.t1 + (size_t)s * R::kBytes;
-  const uint32_t ca = st + kMmBBytes + (uint32_t)(w * 2 * R::kCodes);
-  if (R::kCodes == 512) {
-    dma16_lds((lane < 32 ? r0 : r1) + (lane & 31) * 16, ca);
-  } else {
-    dma16_lds(r0 + lane * 16, ca);
-    dma16_lds(r1 + lane * 16, ca + 1024);
-  }
-  constexpr int kl = R::kRest / 16;  // lanes per tile
-  if (lane < 2 * kl)
-    dma16_lds((lane < kl ? r0 : r1) + R::kCodes + (lane < kl ? lane : lane - kl) * 16,
-              st + kMmBBytes + 16 * R::kCodes + (uint32_t)(w * 2 * R::kRest));
-  if (R::kSums && lane < 16)
-    dma16_lds(it.sums + it.srow + (s >> 1) * 8, st + kMmBBytes + 16 * R::kBytes + (uint32_t)(w * 256));
-}
 
 template <int N>
 __device__ __forceinline__ void vm_wait() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
 }
-// until at most n of this wave's memory operations are in flight (n is 0 or
-// one stage's loads), and no LDS read
-template <int TY>
-__device__ __forceinline__ void mm_wait(int n) {
-  constexpr int k = Rec<TY>::kDma;
-  if (n == k + 4) vm_wait<k + 4>();
-  else if (n == k + 3) vm_wait<k + 3>();
-  else if (n == k + 2) vm_wait<k + 2>();
-  else if (n == k + 1) vm_wait<k + 1>();
-  else vm_wait<0>();
-}
-
 // N B fragments of column tiles CT0 .. of a staged k-group as LDS reads in
 // flight together (16 rows of 256 bytes apart); not valid before lds_wait.
 template <int CT0, int N>
-__device__ __forceinline__ void lds_read_b(uint32_t a, f16x8 (&b)[4]) {
+__device__ __forceinline__ void lds_read_b(uint32_t a, f16x8 (&b)[N]) {
 #pragma unroll
   for (int i = 0; i < N; ++i)
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(b[i]) : "v"(a), "n"((CT0 + i) * 16 * kMmRowBytes));
 }
-// until at most M LDS operations are in flight; b's first N registers tied
+// until at most M LDS operations are in flight; b's registers tied
 template <int N, int M>
-__device__ __forceinline__ void lds_wait_b(f16x8 (&b)[4]) {
-  if constexpr (N == 4)
-    asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]) : "n"(M));
-  else if constexpr (N == 3)
-    asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(b[0]), "+v"(b[1]), "+v"(b[2]) : "n"(M));
-  else if constexpr (N == 2)
+__device__ __forceinline__ void lds_wait_b(f16x8 (&b)[N]) {
+  if constexpr (N == 2)
     asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(b[0]), "+v"(b[1]) : "n"(M));
   else
     asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(b[0]) : "n"(M));
@@ -464,18 +346,17 @@ struct MmAcc {
 // One stage: 2 tiles x NCT column tiles x 64 columns x (hi, lo).  ODD: the
 // second stage of 128 columns, which ends the K-quants' partial sums.
 //
-// Its steps Z: column group kg of 32, group g of up to four column tiles,
-// part (hi, lo), the part running fastest; the B fragments of step Z + 1 are
-// read while step Z multiplies.
+// Its steps Z: column group kg of 32, group of up to two column tiles, part
+// (hi, lo), the part running fastest; the B fragments of step Z + 1 are read
+// while step Z multiplies.
 template <int TY, int NCT, bool ODD>
 struct MmStage {
   using R = Rec<TY>;
-  static constexpr int kNG = (NCT + 3) / 4, kG0 = (NCT + kNG - 1) / kNG, kSteps = 4 * kNG;
+  using S = MmBuf<TY, NCT>;
+  static constexpr int kG = NCT < 2 ? NCT : 2, kNG = NCT / kG, kSteps = 4 * kNG;
   static constexpr int kg(int z) { return z / (2 * kNG); }
-  static constexpr int grp(int z) { return (z >> 1) % kNG; }
   static constexpr int part(int z) { return z & 1; }
-  static constexpr int ct0(int z) { return grp(z) * kG0; }
-  static constexpr int num(int z) { return grp(z) ? NCT - kG0 : kG0; }
+  static constexpr int ct0(int z) { return (z >> 1) % kNG * kG; }
 
   const unsigned char* st;
   const unsigned char* rs;
@@ -484,11 +365,11 @@ struct MmStage {
   uint4 cw[2];
   uint32_t sc[2];
   f16x8 a[2];
-  f16x8 b[2][4];
+  f16x8 b[2][kG];
 
   template <int Z>
   __device__ __forceinline__ void read() {
-    lds_read_b<ct0(Z), num(Z)>(bp + (uint32_t)(((8 * part(Z) + 4 * kg(Z) + q) ^ j) * 16), b[Z & 1]);
+    lds_read_b<ct0(Z), kG>(bp + (uint32_t)(((8 * part(Z) + 4 * kg(Z) + q) ^ j) * 16), b[Z & 1]);
   }
 
   template <int Z>
@@ -508,14 +389,14 @@ struct MmStage {
       }
       if constexpr (Z + 1 < kSteps) {
         read<Z + 1>();
-        lds_wait_b<num(Z), num(Z + 1)>(b[Z & 1]);
+        lds_wait_b<kG, kG>(b[Z & 1]);
       } else {
-        lds_wait_b<num(Z), 0>(b[Z & 1]);
+        lds_wait_b<kG, 0>(b[Z & 1]);
       }
       // the columns' partial sums start at zero
       constexpr bool kStart = part(Z) == 0 && (TY == kGgmlQ8_0 || (!ODD && kg(Z) == 0));
 #pragma unroll
-      for (int i = 0; i < num(Z); ++i)
+      for (int i = 0; i < kG; ++i)
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           f32x4& c = A.c[t][ct0(Z) + i];
@@ -526,10 +407,14 @@ struct MmStage {
         for (int t = 0; t < 2; ++t) {
           const f32x4 d = *reinterpret_cast<const f32x4*>(rs + t * R::kRest + kg(Z) * 64 + 16 * q);
 #pragma unroll
-          for (int i = 0; i < num(Z); ++i) fma4(A.m[t][ct0(Z) + i], d, A.c[t][ct0(Z) + i]);
+          for (int i = 0; i < kG; ++i) {
+            f32x4& m = A.m[t][ct0(Z) + i];
+            fma4(m, d, A.c[t][ct0(Z) + i]);
+            // (left alone, the additions sink to the stage's end, every step's
+            // products kept: 169 registers instead of 120)
+            asm volatile("" : "+v"(m));
+          }
         }
-        // (left alone, the scheduler keeps every step's products live)
-        __builtin_amdgcn_sched_barrier(0);
       }
       steps<Z + 1>(A);
     }
@@ -544,9 +429,9 @@ struct MmStage {
     q = lane >> 4;
     j = lane & 15;
     st = lds + off;
-    rs = st + kMmBBytes + 16 * R::kCodes + w * 2 * R::kRest;
+    rs = st + S::kB + 16 * R::kCodes + w * 2 * R::kRest;
     bp = lds_u32(lds) + (uint32_t)(off + j * kMmRowBytes);
-    const unsigned char* cd = st + kMmBBytes + w * 2 * R::kCodes;
+    const unsigned char* cd = st + S::kB + w * 2 * R::kCodes;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       if constexpr (TY == kGgmlQ8_0) {
@@ -577,7 +462,7 @@ struct MmStage {
           const f16x8 am = __builtin_bit_cast(f16x8, make_uint4(z.x, z.y, z.x, z.y));
 #pragma unroll
           for (int ct = 0; ct < NCT; ++ct) {
-            const f16x8 bs = *reinterpret_cast<const f16x8*>(st + kMmBBytes + 16 * R::kBytes +
+            const f16x8 bs = *reinterpret_cast<const f16x8*>(st + S::kSumsAt +
                                                              (16 * ct + j) * 16);
             fma4(A.m[t][ct], dn, mfma_f16(am, bs, f32x4{0, 0, 0, 0}));
           }
@@ -587,148 +472,220 @@ struct MmStage {
   }
 };
 
-// Item cur with NCT column tiles, its first two stages in flight; the next
-// item's first two are requested on the way.  gb: stages before it; par:
-// which half of the info words (assignment, exponent) behind the stages is
-// its own.  The next item's are written after the first barrier, when every
-// wave is past the epilogue that read that half.
+constexpr int kMmInfo = kGgufMmTok * (int)sizeof(int2);
+template <int TY>
+constexpr int mm_lds() {
+  constexpr int a = MmBuf<TY, 4>::kBufs * MmBuf<TY, 4>::kBytes;
+  constexpr int b = MmBuf<TY, 2>::kBufs * MmBuf<TY, 2>::kBytes;
+  constexpr int n = (a > b ? a : b) + kMmInfo;
+  static_assert(2 * n <= 160 * 1024, "two workgroups per CU");
+  return n;
+}
+// A unit's block of rows with NCT column tiles, kAhead stages in flight.
 template <int TY, bool GU, int NCT>
-__device__ __forceinline__ void mm_run(const MmArgs& g, const unsigned char* lds, const MmItem& cur,
-                                       const MmItem& nxt, int gb, int par, int w, int lane) {
+struct MmRun {
   using R = Rec<TY>;
-  const int q = lane >> 4, j = lane & 15, K = g.L.K, H = g.L.H;
-  MmAcc<NCT> A;
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int ct = 0; ct < NCT; ++ct) A.m[t][ct] = A.c[t][ct] = f32x4{0, 0, 0, 0};
-  uint2 mn[2] = {make_uint2(0, 0), make_uint2(0, 0)};
-  const uint32_t l0 = lds_u32(lds);
-  const int2* info = reinterpret_cast<const int2*>(lds + kMmStages * R::kStage);
-  auto turn = [&](int ps) {
-    // this wave's loads of stage ps have landed (the next stage's may be in
-    // flight; at the first stage of a later item everything, since the
-    // previous epilogue's stores went out after them) ...
-    const int nx = ps + 1 < cur.nst ? cur.dma : nxt.valid ? nxt.dma : 0;
-    mm_wait<TY>(ps == 0 && gb > 0 ? 0 : nx);
-    // ... and after the barrier every wave's have, and nobody reads stage
-    // ps - 1 any more, whose buffer stage ps + 2 takes
-    __builtin_amdgcn_s_barrier();
-    if (ps == 0 && nxt.valid && threadIdx.x < kGgufMmTok)
-      const_cast<int2*>(info)[(par ^ 1) * kGgufMmTok + threadIdx.x] = nxt.info;
-    const uint32_t st = l0 + (uint32_t)((gb + ps + 2) % kMmStages * R::kStage);
-    if (ps + 2 < cur.nst)
-      mm_issue<TY>(cur, ps + 2, st, w, lane);
-    else if (nxt.valid)
-      mm_issue<TY>(nxt, ps + 2 - cur.nst, st, w, lane);
-    return (gb + ps) % kMmStages * R::kStage;
-  };
-  for (int ps = 0; ps < cur.nst; ps += 2) {  // (128 columns: nst is even)
-    int o = turn(ps);
-    MmStage<TY, NCT, false>().run(lds, o, w, lane, A, mn);
-    o = turn(ps + 1);
-    MmStage<TY, NCT, true>().run(lds, o, w, lane, A, mn);
+  using S = MmBuf<TY, NCT>;
+  const uint8_t* t0;  // this wave's two tiles
+  const uint8_t* t1;
+  const uint16_t* b[S::kRowLoads];  // this lane's segment of its token rows
+  const uint16_t* sums;             // and (Q4_K) its row of column sums
+  uint32_t l0;
+  int w, lane, nst, nrow;           // stages; row loads of this wave and stage
+
+  // row of token rows of position r (0 .. n - 1) of a unit
+  static __device__ __forceinline__ int row_of(const MmArgs& g, const MmUnit& u, int r) {
+    const int p = u.p0 + min(r, u.n - 1);
+    return GU && !u.shared ? g.perm[p] / g.L.K : p;
   }
-  // rows fr .. fr + 3 of the lane in its column of each column tile
+
+  // This wave's loads of stage s.
+  __device__ __forceinline__ void issue(int s) {
+    const uint32_t st = l0 + (uint32_t)(s % S::kBufs * S::kBytes);
+    if (NCT > 1 || nrow) {  // uniform
 #pragma unroll
-  for (int ct = 0; ct < NCT; ++ct) {
-    const int c = 16 * ct + j;
-    if (c < cur.n) {
-      const int2 in = info[par * kGgufMmTok + c];
-      const int p = cur.p0 + c, a = in.x, ex = in.y;
-      const uint32_t ph = cur.shared ? kPhShared : kPhExpert;
-      if (GU) {
-        const int fr = cur.fb * 128 + 16 * w + 4 * q;
-        f32x4 gv, uv, hv;
-        bool bad = false;
+      for (int m = 0; m < S::kRowLoads; ++m)
+        dma16_lds(b[m] + s * (2 * kMmCols), st + (uint32_t)((w + 8 * m) * 1024));
+    }
+    const uint8_t* r0 = t0 + (size_t)s * R::kBytes;
+    const uint8_t* r1 = t1 + (size_t)s * R::kBytes;
+    const uint32_t ca = st + S::kB + (uint32_t)(w * 2 * R::kCodes);
+    if (R::kCodes == 512) {
+      dma16_lds((lane < 32 ? r0 : r1) + (lane & 31) * 16, ca);
+    } else {
+      dma16_lds(r0 + lane * 16, ca);
+      dma16_lds(r1 + lane * 16, ca + 1024);
+    }
+    constexpr int kl = R::kRest / 16;  // lanes per tile
+    if (lane < 2 * kl)
+      dma16_lds((lane < kl ? r0 : r1) + R::kCodes + (lane < kl ? lane : lane - kl) * 16,
+                st + S::kB + 16 * R::kCodes + (uint32_t)(w * 2 * R::kRest));
+    if (R::kSums && w < NCT && lane < 16)  // (w uniform)
+      dma16_lds(sums + (s >> 1) * 8, st + S::kSumsAt + (uint32_t)(w * 256));
+  }
+
+  // Stage s is complete everywhere, and nobody reads stage s - 1 any more,
+  // whose buffer stage s + kAhead takes; the stage's byte offset.
+  __device__ __forceinline__ int turn(int s) {
+    // this wave's loads of stage s have landed (those of the next stage may
+    // be in flight where two are ahead) ...
+    constexpr int kA = R::kDma - (R::kSums ? 1 : 0);
+    if (S::kAhead == 1 || s + 1 >= nst) {
+      vm_wait<0>();
+    } else {
+      const int n = nrow + kA + (R::kSums && w < NCT ? 1 : 0);  // uniform
+      if (n == kA + 2) vm_wait<kA + 2>();
+      else if (n == kA + 1) vm_wait<kA + 1>();
+      else vm_wait<kA>();
+    }
+    __builtin_amdgcn_s_barrier();  // ... and every wave's
+    if (s + S::kAhead < nst) issue(s + S::kAhead);
+    return s % S::kBufs * S::kBytes;
+  }
+
+  __device__ __forceinline__ void run(const MmArgs& g, const MmUnit& cur,
+                                      const unsigned char* lds) {
+    const GgufMoeDev& L = g.L;
+    const int K = L.K, H = L.H;
+    w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    lane = threadIdx.x & 63;
+    l0 = lds_u32(lds);
+    const int q = lane >> 4, j = lane & 15;
+    const int KD = GU ? H : cur.rows;
+    nst = KD / kMmCols;
+    const uint8_t* m0 = L.tiles + tile_offset(L.E, H, L.I, L.Ish, R::kBytes, cur.e, GU ? 0 : 2);
+    const size_t rb = (size_t)nst * R::kBytes;  // bytes of 16 rows
+    if (GU) {
+      t0 = m0 + (size_t)(cur.fb * 8 + w) * rb;
+      t1 = t0 + (size_t)(cur.rows / 16) * rb;
+    } else {
+      // H is a multiple of 128: waves past it (in the last block) load rows
+      // 0 .. 31 and store nothing
+      t0 = m0 + (size_t)(cur.fb * 256 + 32 * w < H ? cur.fb * 16 + 2 * w : 0) * rb;
+      t1 = t0 + rb;
+    }
+    const size_t before = !GU && cur.shared ? (size_t)g.T * K * L.I : 0;
+    // load m carries rows 4 (w + 8m) .. + 3, stored segment lane & 15 of row r
+    // being its segment (lane & 15) ^ (r & 15)
+    nrow = NCT > 1 || w < 4 ? S::kRowLoads : 0;
+    const int sg = j ^ ((4 * w + q) & 15);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          gv[i] = __builtin_amdgcn_ldexpf(A.m[0][ct][i], -ex);
-          uv[i] = __builtin_amdgcn_ldexpf(A.m[1][ct][i], -ex);
-          hv[i] = dm_silu(gv[i]) * uv[i];
-          bad |= !finite_f(gv[i]) || !finite_f(uv[i]) || !finite_f(hv[i]);
-        }
-        *reinterpret_cast<f32x4*>((cur.shared ? g.outs : g.out) + (size_t)p * cur.rows + fr) = hv;
-        if (bad) {
-          const int t = cur.shared ? p : a / K, k = cur.shared ? 0 : a % K;
+    for (int m = 0; m < S::kRowLoads; ++m)
+      b[m] = g.b + 2 * before + (size_t)row_of(g, cur, 4 * (w + 8 * m) + q) * (2 * KD) + sg * 8;
+    if (R::kSums)
+      sums = g.sums + before / 16 + (size_t)row_of(g, cur, 16 * w + j) * (KD / 16);
+    issue(0);
+    if (S::kAhead > 1) issue(1);  // (128 columns: nst is even)
+    // the epilogue's words of a position: assignment, exponent (written before
+    // the first barrier)
+    int2* info = reinterpret_cast<int2*>(const_cast<unsigned char*>(lds) + mm_lds<TY>() - kMmInfo);
+    if (threadIdx.x < kGgufMmTok) {
+      const int p = cur.p0 + min((int)threadIdx.x, cur.n - 1);
+      const int a = cur.shared ? p : g.perm[p];
+      info[threadIdx.x] =
+          make_int2(a, g.ex[GU ? (cur.shared ? p : a / K) : (cur.shared ? g.T * K + p : p)]);
+    }
+    MmAcc<NCT> A;
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (!finite_f(gv[i]) || !finite_f(uv[i]) || !finite_f(hv[i]))
-              record_err(g.status, err_key(ph, t, k, fr + i, !finite_f(gv[i])   ? kEkGate
-                                                             : !finite_f(uv[i]) ? kEkUp
-                                                                                : kEkH));
-        }
-      } else if (cur.fb * 256 + 32 * w < H) {
-        float* dst = cur.shared ? g.outs + (size_t)p * H : g.out + (size_t)a * H;
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const int d0 = cur.fb * 256 + 32 * w + 16 * t + 4 * q;
-          f32x4 v;
+      for (int ct = 0; ct < NCT; ++ct) A.m[t][ct] = A.c[t][ct] = f32x4{0, 0, 0, 0};
+    uint2 mn[2] = {make_uint2(0, 0), make_uint2(0, 0)};
+    for (int s = 0; s < nst; s += 2) {
+      int o = turn(s);
+      MmStage<TY, NCT, false>().run(lds, o, w, lane, A, mn);
+      o = turn(s + 1);
+      MmStage<TY, NCT, true>().run(lds, o, w, lane, A, mn);
+    }
+    // rows fr .. fr + 3 of the lane in its column of each column tile
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) {
+      const int c = 16 * ct + j;
+      if (c < cur.n) {
+        const int2 in = info[c];
+        const int p = cur.p0 + c, a = in.x, x = in.y;
+        const uint32_t ph = cur.shared ? kPhShared : kPhExpert;
+        if (GU) {
+          const int fr = cur.fb * 128 + 16 * w + 4 * q;
+          f32x4 gv, uv, hv;
           bool bad = false;
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            v[i] = __builtin_amdgcn_ldexpf(A.m[t][ct][i], -ex);
-            bad |= !finite_f(v[i]);
+            gv[i] = __builtin_amdgcn_ldexpf(A.m[0][ct][i], -x);
+            uv[i] = __builtin_amdgcn_ldexpf(A.m[1][ct][i], -x);
+            hv[i] = dm_silu(gv[i]) * uv[i];
+            bad |= !finite_f(gv[i]) || !finite_f(uv[i]) || !finite_f(hv[i]);
           }
-          *reinterpret_cast<f32x4*>(dst + d0) = v;
+          *reinterpret_cast<f32x4*>((cur.shared ? g.outs : g.out) + (size_t)p * cur.rows + fr) = hv;
           if (bad) {
-            const int tk = cur.shared ? p : a / K, k = cur.shared ? 0 : a % K;
+            const int t = cur.shared ? p : a / K, k = cur.shared ? 0 : a % K;
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-              if (!finite_f(v[i])) record_err(g.status, err_key(ph, tk, k, cur.rows + d0 + i, kEkDown));
+              if (!finite_f(gv[i]) || !finite_f(uv[i]) || !finite_f(hv[i]))
+                record_err(g.status, err_key(ph, t, k, fr + i, !finite_f(gv[i])   ? kEkGate
+                                                               : !finite_f(uv[i]) ? kEkUp
+                                                                                  : kEkH));
+          }
+        } else if (cur.fb * 256 + 32 * w < H) {
+          float* dst = cur.shared ? g.outs + (size_t)p * H : g.out + (size_t)a * H;
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            const int d0 = cur.fb * 256 + 32 * w + 16 * t + 4 * q;
+            f32x4 v;
+            bool bad = false;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              v[i] = __builtin_amdgcn_ldexpf(A.m[t][ct][i], -x);
+              bad |= !finite_f(v[i]);
+            }
+            *reinterpret_cast<f32x4*>(dst + d0) = v;
+            if (bad) {
+              const int tk = cur.shared ? p : a / K, k = cur.shared ? 0 : a % K;
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                if (!finite_f(v[i])) record_err(g.status, err_key(ph, tk, k, cur.rows + d0 + i, kEkDown));
+            }
           }
         }
       }
     }
   }
-}
+};
 
-// Workgroup b takes the items b, b + gridDim.x, ... (gridDim.x a multiple of
-// 8, or one item each), the stages of all its items in one pipeline.  A unit
-// of n tokens runs with the column tiles it needs.
+// Workgroup b: unit and block of rows in 8 classes (b % 8 is the XCD the
+// dispatcher places it on: a unit's row blocks share that XCD's L2 for its
+// token rows, as in k_experts).  A unit of n tokens runs with the column tiles
+// it needs; at most 128 registers and 80 KB of LDS, so that two workgroups
+// share a CU (see k_experts; one persistent workgroup on 128-token units
+// before: at hidden 2048, inter 512, 256 experts, 2048 tokens of Q3_K gate/up 286
+// -> 240 us and down 174 -> 143; per call of 256 / 2048 tokens Q3_K 313 / 627 -> 195 /
+// 505 us, Q4_K 375 / 743 -> 215 / 554, Q8_0 470 / 931 -> 243 / 537).  Bound by the
+// matrix units' two passes (hi and lo) and, between them, the codes' conversion and the
+// fp32 scaling of the partial sums.
 template <int TY, bool GU>
-__global__ __launch_bounds__(kMmThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ __launch_bounds__(kMmThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void k_gguf_mm(const int32_t* meta, const int2* units, const int32_t* off, const int32_t* perm,
-               MmArgs gk) {
+               int nblk, MmArgs gk) {
   extern __shared__ __attribute__((aligned(16))) unsigned char ldsm[];
   MmArgs g = gk;
-  g.meta = meta;
-  g.units = units;
-  g.off = off;
   g.perm = perm;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int nblk = GU ? ((g.L.I > g.L.Ish ? g.L.I : g.L.Ish) + 127) / 128 : (g.L.H + 255) / 256;
-  const int items = 8 * ((meta[0] + 7) >> 3) * nblk;
-  const int step = gridDim.x;
-  int idx = blockIdx.x;
-  MmItem cur = mm_next<TY, GU>(g, idx, step, items, nblk, w, lane);
-  if (!cur.valid) return;  // uniform per workgroup
-  const uint32_t l0 = lds_u32(ldsm);
-  mm_issue<TY>(cur, 0, l0, w, lane);
-  mm_issue<TY>(cur, 1, l0 + Rec<TY>::kStage, w, lane);
-  if (threadIdx.x < kGgufMmTok)
-    reinterpret_cast<int2*>(ldsm + kMmStages * Rec<TY>::kStage)[threadIdx.x] = cur.info;
-  int gb = 0, par = 0;
-  while (true) {
-    const MmItem nxt = mm_next<TY, GU>(g, idx, step, items, nblk, w, lane);
-    const int nct = (cur.n + 15) >> 4;  // uniform
-    if (nct <= 1) mm_run<TY, GU, 1>(g, ldsm, cur, nxt, gb, par, w, lane);
-    else if (nct <= 2) mm_run<TY, GU, 2>(g, ldsm, cur, nxt, gb, par, w, lane);
-    else if (nct <= 4) mm_run<TY, GU, 4>(g, ldsm, cur, nxt, gb, par, w, lane);
-    else if (nct <= 5) mm_run<TY, GU, 5>(g, ldsm, cur, nxt, gb, par, w, lane);
-    else if (nct <= 6) mm_run<TY, GU, 6>(g, ldsm, cur, nxt, gb, par, w, lane);
-    else mm_run<TY, GU, 8>(g, ldsm, cur, nxt, gb, par, w, lane);
-    if (!nxt.valid) break;  // uniform
-    gb = (gb + cur.nst) % kMmStages + kMmStages;  // (0: the first item)
-    par ^= 1;
-    cur = nxt;
-  }
+  const int nall = meta[0], span = (nall + 7) >> 3, idx = (int)blockIdx.x >> 3;
+  const int ul = idx / nblk, u = ((int)blockIdx.x & 7) * span + ul;
+  MmUnit it;
+  it.fb = idx - ul * nblk;
+  if (ul >= span || u >= nall) return;
+  const int2 v = units[u];
+  it.shared = v.x >= g.L.E;
+  it.e = it.shared ? g.L.E : v.x;
+  it.p0 = it.shared ? v.y : off[v.x] + v.y;
+  it.n = min(kGgufMmTok, (it.shared ? g.T : off[v.x + 1]) - it.p0);
+  it.rows = it.shared ? g.L.Ish : g.L.I;
+  if (GU && it.fb * 128 >= it.rows) return;  // uniform per workgroup
+  if (it.n <= 16) MmRun<TY, GU, 1>().run(g, it, ldsm);
+  else if (it.n <= 32) MmRun<TY, GU, 2>().run(g, it, ldsm);
+  else MmRun<TY, GU, 4>().run(g, it, ldsm);
 }
 
-template <int TY>
-constexpr int mm_lds() {
-  return kMmStages * Rec<TY>::kStage + 2 * kGgufMmTok * (int)sizeof(int2);
-}
 template <int TY>
 hipError_t mm_attrs() {
   const int lds = mm_lds<TY>();
@@ -749,18 +706,13 @@ hipError_t run_mm(const GgufMoeDev& L, const float* x, int T, const int32_t* off
   const int64_t TK = (int64_t)T * L.K;
   const size_t lds = mm_lds<TY>();
   float* hs = s.h + TK * L.I;
-  const int pw = persistent_wgs();
-  if (pw <= 0) return hipErrorInvalidValue;
-  const int imax = L.I > L.Ish ? L.I : L.Ish;
-  auto grid = [&](int nblk) {
-    const int64_t items = (int64_t)(nunits + 8) * nblk;
-    return dim3((unsigned)(items < pw ? (items + 7) / 8 * 8 : pw));
-  };
+  const int imax = L.I > L.Ish ? L.I : L.Ish, classes = 8 * ((nunits + 7) / 8);
+  const int gb = (imax + 127) / 128, db = (L.H + 255) / 256;
   hipLaunchKernelGGL(k_gguf_split<kSums>, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, st, x,
                      (int64_t)T, L.H, nullptr, (int64_t)0, L.H, s.xs, s.ex, s.xsum);
   MmArgs g{L, off, perm, units, meta, T, s.xs, s.xsum, s.ex, s.h, hs, status};
-  hipLaunchKernelGGL((k_gguf_mm<TY, true>), grid((imax + 127) / 128), dim3(kMmThreads), lds, st,
-                     meta, units, off, perm, g);
+  hipLaunchKernelGGL((k_gguf_mm<TY, true>), dim3(classes * gb), dim3(kMmThreads), lds, st, meta,
+                     units, off, perm, gb, g);
   hipLaunchKernelGGL(k_gguf_split<kSums>, dim3((unsigned)((TK + T + 3) / 4)), dim3(256), 0, st,
                      s.h, TK, L.I, hs, (int64_t)T, L.Ish, s.hs, s.ex + T, s.hsum);
   g.b = s.hs;
@@ -768,8 +720,8 @@ hipError_t run_mm(const GgufMoeDev& L, const float* x, int T, const int32_t* off
   g.ex = s.ex + T;
   g.out = r;
   g.outs = rs;
-  hipLaunchKernelGGL((k_gguf_mm<TY, false>), grid((L.H + 255) / 256), dim3(kMmThreads), lds, st,
-                     meta, units, off, perm, g);
+  hipLaunchKernelGGL((k_gguf_mm<TY, false>), dim3(classes * db), dim3(kMmThreads), lds, st, meta,
+                     units, off, perm, db, g);
   return hipGetLastError();
 }
 
