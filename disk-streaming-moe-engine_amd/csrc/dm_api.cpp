@@ -2022,6 +2022,7 @@ static int upload_gguf_body(dmh_ctx* c, int layer, const dmh_moe_dims* d,
     } else {
       if (G->tiles) (void)hipFree(G->tiles);
       G->tiles = nullptr;
+      (void)hipGetLastError();  // (a failed allocation is not the next launch's error)
     }
   }
   if (GgufLayer* old = c->glayers[layer]) {
