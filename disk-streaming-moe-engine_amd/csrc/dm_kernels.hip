@@ -1038,33 +1038,37 @@ hipError_t launch_down_dec(const LayerDev& L, const float* h, int ldh, const int
 // ===========================================================================
 // RMSNorm per token (src/layers/rmsnorm.mojo:41-48): out = x / denom *
 // gamma, denom = sqrt(sum(x * x) / H + eps), for the block-edge norm of
-// several tokens.  SEQ: the squares staged in LDS and added in element order
-// by one lane, the reference's order; otherwise 256 strided partials and a
-// halving tree (the order of the fused decode kernel's tree mode).
+// several tokens.  SEQ: the squares added in element order, the reference's:
+// a chain of H dependent adds, which bounds the kernel; up to 2048 elements
+// on one wave in rounds (seq_sum_wave_rounds; rows of the staged squares padded
+// by one word, so that writing along and reading across them both use every
+// bank: 1533 tokens of 2048 33 -> 26 us, 8 tokens 12 -> 8), else on one thread.
+// Otherwise 256 strided partials and a halving
+// tree (the order of the fused decode kernel's tree mode).
 // ===========================================================================
 template <bool SEQ>
 __global__ __launch_bounds__(256) void k_rmsnorm_rows(const float* __restrict__ x, int H,
                                                        float eps, const float* __restrict__ gamma,
                                                        float* __restrict__ out) {
-  __shared__ float part[SEQ ? kNormMaxH : 256];
+  __shared__ __attribute__((aligned(16))) float part[SEQ ? kNormMaxH : 256];
   const int t = blockIdx.x;
   const float* xr = x + (size_t)t * H;
   if (SEQ) {
-    for (int i = threadIdx.x; i < H; i += 256) part[i] = xr[i] * xr[i];
+    static_assert(kSeqPerLane * 65 <= kNormMaxH, "padded rows");
+    const bool rounds = H % 64 == 0 && H <= 64 * kSeqPerLane;
+    const int per = H / 64;
+    for (int i = threadIdx.x; i < H; i += 256)
+      part[rounds ? (i % per) * 65 + i / per : i] = xr[i] * xr[i];
     __syncthreads();
-    if (threadIdx.x == 0) {
-      float a = 0.0f;
-      int i = 0;
-      for (; i + 8 <= H; i += 8) {  // reads 8 ahead of the adds
-        float v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = part[i + u];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) a = a + v[u];
-      }
-      for (; i < H; ++i) a = a + part[i];
-      part[0] = a;
+    float a = 0.0f;
+    if (rounds) {
+      if (threadIdx.x < 64) a = seq_sum_wave_rounds(part, per, 65);
+    } else if (threadIdx.x == 0) {
+      a = seq_sum_squares(part, H & ~31);
+      for (int i = H & ~31; i < H; ++i) a = a + part[i];
     }
+    __syncthreads();
+    if (threadIdx.x == 0) part[0] = a;
     __syncthreads();
   } else {
     float acc = 0.0f;
