@@ -74,7 +74,7 @@ struct GgufLayer {
   int grid = 0;
   unsigned launches = 0;
   float* rchain = nullptr;  // the router in chain order (dev.rchain)
-  uint8_t* tiles = nullptr; // the experts in matrix-core records (dev.tiles)
+  uint8_t* tiles = nullptr; // the experts in matrix-core records, or null
 };
 
 void free_glayer(GgufLayer* G) {
@@ -686,9 +686,9 @@ hipError_t run_gguf_block(dmh_ctx* c, GgufLayer* G, unsigned long long* status, 
   if ((e = dm::launch_router_select(c->z.p, L.E + 1, T, L.E, L.K, 1, dids, dprobs, dshg, status,
                                     st)) != hipSuccess)
     return e;
-  if (T > 1 && L.E <= kGgufGroupMaxE && (dm::gguf_units_pay(L, T) || dm::gguf_mm_ok(L, T))) {
+  if (T > 1 && L.E <= kGgufGroupMaxE && (dm::gguf_units_pay(L, T) || dm::gguf_mm_ok(L, G->tiles, T))) {
     // several tokens: grouped by expert, each expert row read once per unit
-    const bool mm = dm::gguf_mm_ok(L, T);
+    const bool mm = dm::gguf_mm_ok(L, G->tiles, T);
     const int tok = mm ? dm::kGgufMmTok : dm::gguf_unit_tokens(L, T);
     const int nu = dm::group_units_max(T, L.K, L.E, tok);
     if ((e = c->g_off.ensure(L.E + 1)) != hipSuccess) return e;
@@ -712,7 +712,7 @@ hipError_t run_gguf_block(dmh_ctx* c, GgufLayer* G, unsigned long long* status, 
       const dm::GgufMmScratch s{c->g_xhi.p,  c->g_hr.p,           c->g_ex.p,
                                 c->g_sums.p, c->g_sums.p + xsum, c->h.p};
       float* rs = c->g_r.p + TK * L.H;
-      if ((e = dm::launch_gguf_mm(L, dx, T, c->g_off.p, c->g_perm.p, c->g_units.p, c->g_meta.p,
+      if ((e = dm::launch_gguf_mm(L, G->tiles, dx, T, c->g_off.p, c->g_perm.p, c->g_units.p, c->g_meta.p,
                                   nu, s, c->g_r.p, rs, status, st)) != hipSuccess)
         return e;
       return dm::launch_combine(c->g_r.p, rs, dprobs, dshg, dres, T, L.H, L.K, dy, status, st);
@@ -2015,11 +2015,9 @@ static int upload_gguf_body(dmh_ctx* c, int layer, const dmh_moe_dims* d,
   // the matrix-core form of the experts; without room for it, calls of many
   // tokens keep the grouped form on the payload
   if (const size_t nt = dm::gguf_tiles_bytes(G->dev)) {
-    if (hipMalloc(&G->tiles, nt) == hipSuccess &&
-        dm::launch_gguf_tiles(G->dev, G->tiles, st) == hipSuccess &&
-        hipStreamSynchronize(st) == hipSuccess) {
-      G->dev.tiles = G->tiles;
-    } else {
+    if (hipMalloc(&G->tiles, nt) != hipSuccess ||
+        dm::launch_gguf_tiles(G->dev, G->tiles, st) != hipSuccess ||
+        hipStreamSynchronize(st) != hipSuccess) {
       if (G->tiles) (void)hipFree(G->tiles);
       G->tiles = nullptr;
       (void)hipGetLastError();  // (a failed allocation is not the next launch's error)

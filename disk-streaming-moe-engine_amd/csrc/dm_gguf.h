@@ -42,7 +42,6 @@ struct GgufMoeDev {
   const float* shgate; // [H]
   int64_t estride;     // > 0: off[3e + k] = (3e + k) * estride for the routed experts (else 0)
   const float* rchain; // [E + 1][H] router and shared gate in chain order (one-token form), or null
-  const uint8_t* tiles;  // the experts in matrix-core records (launch_gguf_tiles), or null
 };
 
 // h[t][s][i] = SiLU(W_gate x_t)_i * (W_up x_t)_i for slots s < K (expert
@@ -89,7 +88,9 @@ hipError_t launch_gguf_tiles(const GgufMoeDev& L, uint8_t* out, hipStream_t st);
 // here on the sums run in the matrix cores' order (as exact, other bits).
 constexpr int kGgufMmMinT = 256;
 constexpr int kGgufMmTok = 64;  // tokens per unit
-bool gguf_mm_ok(const GgufMoeDev& L, int T);
+// tiles: the records of launch_gguf_tiles, or null.  (Not a member of GgufMoeDev:
+// eight more bytes of arguments cost the one-token launch 0.1 us.)
+bool gguf_mm_ok(const GgufMoeDev& L, const uint8_t* tiles, int T);
 // Elements of the column sums of `elements` activations (0: not needed).
 size_t gguf_mm_sums(const GgufMoeDev& L, int64_t elements);
 struct GgufMmScratch {
@@ -104,7 +105,7 @@ struct GgufMmScratch {
 // of launch_group_build with tok = kGgufMmTok, nunits = group_units_max): r [T*K][H] by
 // assignment, rs [T][H] of the shared expert, unweighted, with the checks of
 // launch_gguf_units; launch_combine forms y from them.
-hipError_t launch_gguf_mm(const GgufMoeDev& L, const float* x, int T, const int32_t* off,
+hipError_t launch_gguf_mm(const GgufMoeDev& L, const uint8_t* tiles, const float* x, int T, const int32_t* off,
                           const int32_t* perm, const int2* units, const int32_t* meta, int nunits,
                           const GgufMmScratch& s, float* r, float* rs, unsigned long long* status,
                           hipStream_t st);

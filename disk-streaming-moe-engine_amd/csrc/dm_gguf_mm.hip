@@ -255,6 +255,7 @@ __global__ __launch_bounds__(256) void k_gguf_split(const float* __restrict__ a,
 // ---- the products ----------------------------------------------------------------
 struct MmArgs {
   GgufMoeDev L;
+  const uint8_t* tiles;
   const int32_t* off;
   const int32_t* perm;
   const int2* units;
@@ -553,7 +554,7 @@ struct MmRun {
     const int q = lane >> 4, j = lane & 15;
     const int KD = GU ? H : cur.rows;
     nst = KD / kMmCols;
-    const uint8_t* m0 = L.tiles + tile_offset(L.E, H, L.I, L.Ish, R::kBytes, cur.e, GU ? 0 : 2);
+    const uint8_t* m0 = g.tiles + tile_offset(L.E, H, L.I, L.Ish, R::kBytes, cur.e, GU ? 0 : 2);
     const size_t rb = (size_t)nst * R::kBytes;  // bytes of 16 rows
     if (GU) {
       t0 = m0 + (size_t)(cur.fb * 8 + w) * rb;
@@ -698,7 +699,7 @@ hipError_t mm_attrs() {
 }
 
 template <int TY>
-hipError_t run_mm(const GgufMoeDev& L, const float* x, int T, const int32_t* off,
+hipError_t run_mm(const GgufMoeDev& L, const uint8_t* tiles, const float* x, int T, const int32_t* off,
                   const int32_t* perm, const int2* units, const int32_t* meta, int nunits,
                   const GgufMmScratch& s, float* r, float* rs, unsigned long long* status,
                   hipStream_t st) {
@@ -710,7 +711,7 @@ hipError_t run_mm(const GgufMoeDev& L, const float* x, int T, const int32_t* off
   const int gb = (imax + 127) / 128, db = (L.H + 255) / 256;
   hipLaunchKernelGGL(k_gguf_split<kSums>, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, st, x,
                      (int64_t)T, L.H, nullptr, (int64_t)0, L.H, s.xs, s.ex, s.xsum);
-  MmArgs g{L, off, perm, units, meta, T, s.xs, s.xsum, s.ex, s.h, hs, status};
+  MmArgs g{L, tiles, off, perm, units, meta, T, s.xs, s.xsum, s.ex, s.h, hs, status};
   hipLaunchKernelGGL((k_gguf_mm<TY, true>), dim3(classes * gb), dim3(kMmThreads), lds, st, meta,
                      units, off, perm, gb, g);
   hipLaunchKernelGGL(k_gguf_split<kSums>, dim3((unsigned)((TK + T + 3) / 4)), dim3(256), 0, st,
@@ -755,10 +756,10 @@ hipError_t launch_gguf_tiles(const GgufMoeDev& L, uint8_t* out, hipStream_t st) 
   return hipGetLastError();
 }
 
-bool gguf_mm_ok(const GgufMoeDev& L, int T) {
+bool gguf_mm_ok(const GgufMoeDev& L, const uint8_t* tiles, int T) {
   // the kernels' row offsets are 32-bit element offsets
   const uint64_t n = L.I > L.Ish ? L.I : L.Ish;
-  return L.tiles && T >= kGgufMmMinT && 2ull * T * L.H < (1ull << 32) &&
+  return tiles && T >= kGgufMmMinT && 2ull * T * L.H < (1ull << 32) &&
          2ull * T * L.K * n < (1ull << 32);
 }
 
@@ -766,18 +767,18 @@ size_t gguf_mm_sums(const GgufMoeDev& L, int64_t elements) {
   return L.type == kGgmlQ4_K ? (size_t)elements / 16 : 0;
 }
 
-hipError_t launch_gguf_mm(const GgufMoeDev& L, const float* x, int T, const int32_t* off,
+hipError_t launch_gguf_mm(const GgufMoeDev& L, const uint8_t* tiles, const float* x, int T, const int32_t* off,
                           const int32_t* perm, const int2* units, const int32_t* meta, int nunits,
                           const GgufMmScratch& s, float* r, float* rs, unsigned long long* status,
                           hipStream_t st) {
-  if (!gguf_mm_ok(L, T) || nunits <= 0) return hipErrorInvalidValue;
+  if (!gguf_mm_ok(L, tiles, T) || nunits <= 0) return hipErrorInvalidValue;
   switch (L.type) {
     case kGgmlQ3_K:
-      return run_mm<kGgmlQ3_K>(L, x, T, off, perm, units, meta, nunits, s, r, rs, status, st);
+      return run_mm<kGgmlQ3_K>(L, tiles, x, T, off, perm, units, meta, nunits, s, r, rs, status, st);
     case kGgmlQ4_K:
-      return run_mm<kGgmlQ4_K>(L, x, T, off, perm, units, meta, nunits, s, r, rs, status, st);
+      return run_mm<kGgmlQ4_K>(L, tiles, x, T, off, perm, units, meta, nunits, s, r, rs, status, st);
     default:
-      return run_mm<kGgmlQ8_0>(L, x, T, off, perm, units, meta, nunits, s, r, rs, status, st);
+      return run_mm<kGgmlQ8_0>(L, tiles, x, T, off, perm, units, meta, nunits, s, r, rs, status, st);
   }
 }
 
