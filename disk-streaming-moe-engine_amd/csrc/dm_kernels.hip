@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include "dm_device.h"
+#include "dm_grouped.h"
 #include "dm_kernels.h"
 
 namespace dm {
@@ -391,7 +392,7 @@ template <int N>
 __device__ __forceinline__ void lds_wait_steps4(f32x4 (&v)[4]) {
   asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]) : "n"(N));
 }
-template <int NJ8>
+template <int NJ8, int R>
 __global__ __launch_bounds__(256) void k_router_rows(
     const float* __restrict__ x, const int* __restrict__ gate, const uint16_t* __restrict__ router_,
     int E_, int T, int tpw, LayerDev Lk, float* __restrict__ z, unsigned long long* status) {
@@ -402,34 +403,68 @@ __global__ __launch_bounds__(256) void k_router_rows(
   if (gate && gate[0] == 0) return;  // uniform: k_router_mfma computed these logits
   constexpr int H = NJ8 * 128;
   const int l = threadIdx.x & 15;
-  const int e = blockIdx.x * 16 + (threadIdx.x >> 4);
-  const bool wave_live = blockIdx.x * 16 + (threadIdx.x >> 6) * 4 <= L.E;  // uniform per wave
-  uint4 wr[NJ8];
-  {
-    const uint4* wp = reinterpret_cast<const uint4*>(L.router + r16_index(H, min(e, L.E), l));
+  const int e = blockIdx.x * (16 * R) + (threadIdx.x >> 4);  // rows e, e + 16
+  const bool wave_live = blockIdx.x * (16 * R) + (threadIdx.x >> 6) * 4 <= L.E;  // uniform per wave
+  uint4 wr[R][NJ8];
 #pragma unroll
-    for (int u = 0; u < NJ8; ++u) wr[u] = wp[(size_t)u * 16];
+  for (int r = 0; r < R; ++r) {
+    const uint4* wp =
+        reinterpret_cast<const uint4*>(L.router + r16_index(H, min(e + 16 * r, L.E), l));
+#pragma unroll
+    for (int u = 0; u < NJ8; ++u) wr[r][u] = wp[(size_t)u * 16];
   }
   const int tb = blockIdx.y * tpw, te = min(T, tb + tpw);
   static_assert(kRdTok == 4, "the float4 staging below");
+  // this thread's activations of a pass, k = threadIdx.x + 256 j,
+  // with two rows requested during the pass before
+  float v[(H + 255) / 256][kRdTok];
+  auto fetch = [&](int t0) {
+#pragma unroll
+    for (int j = 0; j < (H + 255) / 256; ++j)
+#pragma unroll
+      for (int tt = 0; tt < kRdTok; ++tt)
+        v[j][tt] = x[(size_t)min(t0 + tt, te - 1) * H + min((int)threadIdx.x + 256 * j, H - 1)];
+  };
+  constexpr bool kAhead = R > 1;
+  if (kAhead) fetch(tb);
   for (int t0 = tb; t0 < te; t0 += kRdTok) {
     const int nt = min(kRdTok, te - t0);
     bool bad = false;
-    for (int k = threadIdx.x; k < H; k += 256) {
-      float v[kRdTok];
+    if constexpr (kAhead) {
 #pragma unroll
-      for (int tt = 0; tt < kRdTok; ++tt) {
-        v[tt] = x[(size_t)(t0 + min(tt, nt - 1)) * H + k];
-        bad |= tt < nt && !finite_f(v[tt]);
+      for (int j = 0; j < (H + 255) / 256; ++j) {
+        const int k = threadIdx.x + 256 * j;
+#pragma unroll
+        for (int tt = 0; tt < kRdTok; ++tt) bad |= k < H && !finite_f(v[j][tt]);
+        if (k < H)
+          *reinterpret_cast<float4*>(xs4 + (size_t)k * kRdTok) =
+              make_float4(v[j][0], v[j][1], v[j][2], v[j][3]);
       }
-      *reinterpret_cast<float4*>(xs4 + (size_t)k * kRdTok) = make_float4(v[0], v[1], v[2], v[3]);
+    } else {
+      for (int k = threadIdx.x; k < H; k += 256) {
+        float q[kRdTok];
+#pragma unroll
+        for (int tt = 0; tt < kRdTok; ++tt) {
+          q[tt] = x[(size_t)(t0 + min(tt, nt - 1)) * H + k];
+          bad |= tt < nt && !finite_f(q[tt]);
+        }
+        *reinterpret_cast<float4*>(xs4 + (size_t)k * kRdTok) = make_float4(q[0], q[1], q[2], q[3]);
+      }
     }
     if (bad && blockIdx.x == 0) record_err(status, err_key(kPhX, 0, 0, 0, 0));
     __syncthreads();
+    if (kAhead && t0 + kRdTok < te) {
+      fetch(t0 + kRdTok);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     // a wave whose four rows are all past row E (the last block's tail)
     // only helps to stage the activations
     if (wave_live) {
-      float acc[kRdTok] = {0.0f, 0.0f, 0.0f, 0.0f};
+      float acc[R][kRdTok];
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int tt = 0; tt < kRdTok; ++tt) acc[r][tt] = 0.0f;
       // group c of 4 steps: steps 4c .. 4c + 3, i.e. word u = c / 2, registers
       // i = 2 (c % 2) and i + 1 (step 8u + 2i: low half, 8u + 2i + 1: high)
       const uint32_t xa0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)(
@@ -445,39 +480,49 @@ __global__ __launch_bounds__(256) void k_router_rows(
           lds_wait_steps4<0>(xc);
         }
         const int u = c >> 1;
-        // this group's two weight words pass through an empty asm, so their
+        // this group's weight words pass through an empty asm, so their
         // conversions stay in the group (hoisted to the top of the token loop as
         // 128 floats they did not fit in the registers)
-        uint32_t wg[2] = {(c & 1) ? wr[u].z : wr[u].x, (c & 1) ? wr[u].w : wr[u].y};
-        asm volatile("" : "+v"(wg[0]), "+v"(wg[1]));
+        uint32_t wg[R][2];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          wg[r][0] = (c & 1) ? wr[r][u].z : wr[r][u].x;
+          wg[r][1] = (c & 1) ? wr[r][u].w : wr[r][u].y;
+          asm volatile("" : "+v"(wg[r][0]), "+v"(wg[r][1]));
+        }
 #pragma unroll
         for (int i2 = 0; i2 < 2; ++i2) {
           const f32x4 xa = xc[2 * i2], xb = xc[2 * i2 + 1];
-          const float wl = bf16lo(wg[i2]), wh = bf16hi(wg[i2]);
-          acc[0] = acc[0] + xa[0] * wl;
-          acc[1] = acc[1] + xa[1] * wl;
-          acc[2] = acc[2] + xa[2] * wl;
-          acc[3] = acc[3] + xa[3] * wl;
-          acc[0] = acc[0] + xb[0] * wh;
-          acc[1] = acc[1] + xb[1] * wh;
-          acc[2] = acc[2] + xb[2] * wh;
-          acc[3] = acc[3] + xb[3] * wh;
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            const float wl = bf16lo(wg[r][i2]), wh = bf16hi(wg[r][i2]);
+#pragma unroll
+            for (int tt = 0; tt < kRdTok; ++tt) acc[r][tt] = acc[r][tt] + xa[tt] * wl;
+#pragma unroll
+            for (int tt = 0; tt < kRdTok; ++tt) acc[r][tt] = acc[r][tt] + xb[tt] * wh;
+          }
         }
-        // (the four chains are complete at every group: sunk below the
-        // first token's store, the others kept every read of the pass live)
-        asm volatile("" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
+        // (the chains are complete at every group: sunk below the first
+        // token's store, the others kept every read of the pass live)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          asm volatile("" : "+v"(acc[r][0]), "+v"(acc[r][1]), "+v"(acc[r][2]), "+v"(acc[r][3]));
         if (c + 1 < 2 * NJ8) {
 #pragma unroll
           for (int k = 0; k < 4; ++k) xc[k] = xn[k];
         }
       }
 #pragma unroll
-      for (int tt = 0; tt < kRdTok; ++tt) {
-        // halving tree over the 16 chains of a row: lane l += lane l + w
+      for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int wdt = 8; wdt >= 1; wdt >>= 1) acc[tt] = acc[tt] + __shfl_down(acc[tt], wdt, 16);
-        if (l == 0 && e <= L.E && tt < nt) z[(size_t)(t0 + tt) * (L.E + 1) + e] = acc[tt];
-      }
+        for (int tt = 0; tt < kRdTok; ++tt) {
+          // halving tree over the 16 chains of a row: lane l += lane l + w
+          float a = acc[r][tt];
+#pragma unroll
+          for (int wdt = 8; wdt >= 1; wdt >>= 1) a = a + __shfl_down(a, wdt, 16);
+          if (l == 0 && e + 16 * r <= L.E && tt < nt)
+            z[(size_t)(t0 + tt) * (L.E + 1) + e + 16 * r] = a;
+        }
     }
     __syncthreads();  // xs4 is restaged for the next tokens
   }
@@ -516,20 +561,36 @@ __global__ __launch_bounds__(256) void k_router_rows_f32(const float* __restrict
     if (bad) record_err(status, err_key(kPhRouterW, 0, 0, 0, 0));
   }
   const int tb = blockIdx.y * tpw, te = min(T, tb + tpw);
+  static_assert(kRdTok == 4, "the float4 staging below");
+  // this thread's activations of a pass, k = threadIdx.x + 256 j,
+  // requested during the pass before
+  float v[(H + 255) / 256][kRdTok];
+  auto fetch = [&](int t0) {
+#pragma unroll
+    for (int j = 0; j < (H + 255) / 256; ++j)
+#pragma unroll
+      for (int tt = 0; tt < kRdTok; ++tt)
+        v[j][tt] = x[(size_t)min(t0 + tt, te - 1) * H + min((int)threadIdx.x + 256 * j, H - 1)];
+  };
+  fetch(tb);
   for (int t0 = tb; t0 < te; t0 += kRdTok) {
     const int nt = min(kRdTok, te - t0);
     bool bad = false;
-    for (int k = threadIdx.x; k < H; k += 256) {
-      float v[kRdTok];
 #pragma unroll
-      for (int tt = 0; tt < kRdTok; ++tt) {
-        v[tt] = x[(size_t)(t0 + min(tt, nt - 1)) * H + k];
-        bad |= tt < nt && !finite_f(v[tt]);
-      }
-      *reinterpret_cast<float4*>(xs4 + (size_t)k * kRdTok) = make_float4(v[0], v[1], v[2], v[3]);
+    for (int j = 0; j < (H + 255) / 256; ++j) {
+      const int k = threadIdx.x + 256 * j;
+#pragma unroll
+      for (int tt = 0; tt < kRdTok; ++tt) bad |= k < H && !finite_f(v[j][tt]);
+      if (k < H)
+        *reinterpret_cast<float4*>(xs4 + (size_t)k * kRdTok) =
+            make_float4(v[j][0], v[j][1], v[j][2], v[j][3]);
     }
     if (bad && blockIdx.x == 0) record_err(status, err_key(kPhX, 0, 0, 0, 0));
     __syncthreads();
+    if (t0 + kRdTok < te) {
+      fetch(t0 + kRdTok);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     if (wave_live) {
       float acc[kRdTok] = {0.0f, 0.0f, 0.0f, 0.0f};
       const uint32_t xa0 = lds_u32(xs4 + (size_t)l * kRdTok);
@@ -599,25 +660,37 @@ hipError_t launch_router_dec(const LayerDev& L, const float* x, int T, float* z,
   const int blocks = (L.E + 1 + 15) / 16;
   const int nj8 = L.H % 128 == 0 ? L.H / 128 : 0;
   if (T >= 2 * kRdTok && (nj8 == 2 || nj8 == 4 || nj8 == 8 || nj8 == 16)) {
-    // tokens per workgroup: a multiple of kRdTok, about 1024 workgroups
-    const int want = (1024 + blocks - 1) / blocks;
+    // From 512 tokens on two rows per lane: an LDS read then serves 16
+    // products instead of 8 (LDS reads took 0.9 of the time the products do)
+    // and the next pass's activations are requested ahead; at most 512
+    // workgroups (two per CU at their 220 registers), so one round.  1533
+    // tokens: 79 -> 70 us.  Below, one row (1024 workgroups).  Tokens per
+    // workgroup: a multiple of kRdTok.
+    const bool two = T >= 512;
+    const int bl = two ? (L.E + 1 + 31) / 32 : blocks;
+    const int want = two ? (512 >= bl ? 512 / bl : 1) : (1024 + bl - 1) / bl;
     int tpw = (T + want - 1) / want;
     tpw = ((tpw + kRdTok - 1) / kRdTok) * kRdTok;
     const int ty = (T + tpw - 1) / tpw;
     const size_t lds = (size_t)L.H * kRdTok * sizeof(float);
-    const dim3 g(blocks, ty);
-    if (nj8 == 16)
-      hipLaunchKernelGGL(k_router_rows<16>, g, dim3(256), lds, st, x, gate, L.router, L.E, T, tpw,
-                         L, z, status);
-    else if (nj8 == 8)
-      hipLaunchKernelGGL(k_router_rows<8>, g, dim3(256), lds, st, x, gate, L.router, L.E, T, tpw,
-                         L, z, status);
-    else if (nj8 == 4)
-      hipLaunchKernelGGL(k_router_rows<4>, g, dim3(256), lds, st, x, gate, L.router, L.E, T, tpw,
-                         L, z, status);
-    else
-      hipLaunchKernelGGL(k_router_rows<2>, g, dim3(256), lds, st, x, gate, L.router, L.E, T, tpw,
-                         L, z, status);
+    const dim3 g(bl, ty);
+#define DM_ROUTER_ROWS(NJ8, R)                                                                 \
+  hipLaunchKernelGGL((k_router_rows<NJ8, R>), g, dim3(256), lds, st, x, gate, L.router, L.E, T, \
+                     tpw, L, z, status)
+    if (nj8 == 16) {
+      if (two) DM_ROUTER_ROWS(16, 2);
+      else DM_ROUTER_ROWS(16, 1);
+    } else if (nj8 == 8) {
+      if (two) DM_ROUTER_ROWS(8, 2);
+      else DM_ROUTER_ROWS(8, 1);
+    } else if (nj8 == 4) {
+      if (two) DM_ROUTER_ROWS(4, 2);
+      else DM_ROUTER_ROWS(4, 1);
+    } else {
+      if (two) DM_ROUTER_ROWS(2, 2);
+      else DM_ROUTER_ROWS(2, 1);
+    }
+#undef DM_ROUTER_ROWS
     return hipGetLastError();
   }
   const int ty = T < 256 ? T : 256;  // workgroups loop over the tokens beyond
@@ -639,16 +712,23 @@ hipError_t launch_router_dec(const LayerDev& L, const float* x, int T, float* z,
 // j + 16 (i / 4), register 4b + i % 4, so the 16 chains of one logit share a
 // lane and the halving tree (l += l + w, w = 8, 4, 2, 1) is plain adds.
 //
-// Workgroup: 16 tokens x 64 experts (wave w: experts 64 blockIdx.x + 16 w);
-// the last column of workgroups computes the shared-expert gate logit (row E)
-// with one lane per (token, chain) instead.  The tokens' activations are
+// Workgroup: 16 tokens x 16 NW experts (wave w: experts 16 (NW blockIdx.x +
+// w)).  The shared-expert gate logit (row E) takes one lane per (token,
+// chain): the last column of workgroups with NW = 4, the first four waves of
+// the first column with NW = 8.  A wave's 512 matrix instructions take about
+// 7 us, the staging as much again, and a workgroup's 66 KB of LDS leave room
+// for two on a CU: NW = 4 while every workgroup has a CU of its own (131
+// tokens: 23 us, 25 with the gate inside), NW = 8 beyond (2048 tokens, 256
+// experts: 256 workgroups in one round, 46 -> 34 us; with the gate's
+// workgroups apart 51).  The tokens' activations are
 // staged once in LDS in chain-major order: xs[i][l][s] = x[t0 + i][16 s + l]
 // (bf16), rows padded by 16 bytes so that the 16 lanes of one operand fetch
 // hit distinct banks.
 // ===========================================================================
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-__global__ __launch_bounds__(256) void k_router_mfma(const uint16_t* __restrict__ xhi,
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_router_mfma(const uint16_t* __restrict__ xhi,
                                                       const int* __restrict__ need_lo,
                                                       const uint16_t* __restrict__ router_, int H_,
                                                       int E_, int T, LayerDev Lk,
@@ -662,19 +742,36 @@ __global__ __launch_bounds__(256) void k_router_mfma(const uint16_t* __restrict_
   if (need_lo[0] != 0) return;  // uniform: k_router_dec takes these tokens
   const int H = L.H, E = L.E, ns = H / 16;
   const int pitch = 16 * ns + 8;  // elements per staged token (16 B of padding)
-  const int t0 = blockIdx.y * 16, tid = threadIdx.x;
+  const int t0 = blockIdx.y * 16, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int e0 = 16 * (blockIdx.x * NW + w), b = lane >> 4, jj = lane & 15, nc = ns / 8;
+  // the wave's first router words, requested before the staging (the router
+  // comes from HBM when a layer's turn comes): steps 8c .. 8c + 7 of its chains,
+  // two rounds ahead of their products, four with one workgroup of four waves
+  // per CU (131 tokens 23 -> 22 us; with eight waves 35 -> 39); requests clamped
+  // to the last round
+  constexpr int kRing = NW == 4 ? 4 : 2;
+  const uint16_t* wb = L.router + r16_index(H, min(e0 + jj, E - 1), b);
+  uint4 wr[kRing][4];
+  auto load_w = [&](int c, uint4 (&d)[4]) {
+    const int cc = min(c, nc - 1);
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      d[g] = *reinterpret_cast<const uint4*>(wb + (size_t)cc * 128 + 4 * g * 8);
+  };
+#pragma unroll
+  for (int u = 0; u < kRing; ++u) load_w(u, wr[u]);
   // stage: thread item (token i, step pair sp) reads x[32 sp .. 32 sp + 31]
   // and writes, for each chain l, steps 2 sp and 2 sp + 1 as one word.
   // The reads of up to kStage items are all requested before the first
   // write (one round trip instead of one per item: x was just written by
   // another launch, so it comes from beyond this XCD's L2).
-  constexpr int kStage = 4;
+  constexpr int kStage = 16 / NW, kThr = 64 * NW;
   const int npair = ns / 2;
-  for (int idx0 = tid; idx0 < 16 * npair; idx0 += 256 * kStage) {
+  for (int idx0 = tid; idx0 < 16 * npair; idx0 += kThr * kStage) {
     uint4 xv[kStage][4];
 #pragma unroll
     for (int it = 0; it < kStage; ++it) {
-      const int idx = min(idx0 + 256 * it, 16 * npair - 1);
+      const int idx = min(idx0 + kThr * it, 16 * npair - 1);
       const int i = idx / npair, sp = idx % npair;
       const uint4* src =
           reinterpret_cast<const uint4*>(xhi + (size_t)min(t0 + i, T - 1) * H + 32 * sp);
@@ -683,7 +780,7 @@ __global__ __launch_bounds__(256) void k_router_mfma(const uint16_t* __restrict_
     }
 #pragma unroll
     for (int it = 0; it < kStage; ++it) {
-      const int idx = idx0 + 256 * it;
+      const int idx = idx0 + kThr * it;
       if (idx < 16 * npair) {
         const int i = idx / npair, sp = idx % npair;
         uint32_t v[16];
@@ -705,8 +802,7 @@ __global__ __launch_bounds__(256) void k_router_mfma(const uint16_t* __restrict_
     }
   }
   __syncthreads();
-  const int lane = tid & 63, w = tid >> 6;
-  if ((int)blockIdx.x == (E + 63) / 64) {
+  if (NW == 4 ? (int)blockIdx.x == (E + 63) / 64 : blockIdx.x == 0 && w < 4) {
     // shared-expert gate: lane (token i, chain l), 8 steps per 16-byte read
     const int i = tid >> 4, l = tid & 15;
     const uint16_t* xr = xs + i * pitch + l * ns;
@@ -716,7 +812,6 @@ __global__ __launch_bounds__(256) void k_router_mfma(const uint16_t* __restrict_
     // the first product (one round trip per sixteen rounds; requested one
     // per round they made these workgroups the launch's longest)
     constexpr int kGw = 16;
-    const int nc = ns / 8;
     for (int c0 = 0; c0 < nc; c0 += kGw) {
       uint4 wv[kGw];
 #pragma unroll
@@ -739,29 +834,16 @@ __global__ __launch_bounds__(256) void k_router_mfma(const uint16_t* __restrict_
 #pragma unroll
     for (int wdt = 8; wdt >= 1; wdt >>= 1) acc = acc + __shfl_down(acc, wdt, 16);
     if (l == 0 && t0 + i < T) z[(size_t)(t0 + i) * (E + 1) + E] = acc;
-    return;
+    if (NW == 4) return;
   }
-  const int e0 = blockIdx.x * 64 + 16 * w;
   if (e0 >= E) return;  // uniform per wave (no barrier below)
-  const int b = lane >> 4, jj = lane & 15;
-  const int er = min(e0 + jj, E - 1);
   // A: token jj (as row i = lane & 15 of block b), chain 4g + b
   const uint16_t* xa = xs + jj * pitch + b * ns;
-  const uint16_t* wb = L.router + r16_index(H, er, b);
   f32x16 acc[4];
 #pragma unroll
   for (int g = 0; g < 4; ++g) acc[g] = f32x16{};
-  // steps 8c .. 8c + 7 of the wave's chains: the router words two rounds
-  // ahead of their products (a ring of two, requests clamped to the last
-  // round), x from LDS one round ahead
-  const int nc = ns / 8;
-  uint4 wr[2][4], xr[2][4];
-  auto load_w = [&](int c, uint4 (&d)[4]) {
-    const int cc = min(c, nc - 1);
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-      d[g] = *reinterpret_cast<const uint4*>(wb + (size_t)cc * 128 + 4 * g * 8);
-  };
+  // x from LDS one round ahead
+  uint4 xr[2][4];
   auto load_x = [&](int c, uint4 (&d)[4]) {
     const int cc = min(c, nc - 1);
 #pragma unroll
@@ -786,19 +868,23 @@ __global__ __launch_bounds__(256) void k_router_mfma(const uint16_t* __restrict_
       }
     }
   };
-  load_w(0, wr[0]);
-  load_w(1, wr[1]);
   load_x(0, xr[0]);
   int c = 0;
-  for (; c + 1 < nc; c += 2) {
-    load_x(c + 1, xr[1]);
-    steps(xr[0], wr[0]);
-    load_w(c + 2, wr[0]);
-    load_x(c + 2, xr[0]);
-    steps(xr[1], wr[1]);
-    load_w(c + 3, wr[1]);
+  for (; c + kRing <= nc; c += kRing) {
+#pragma unroll
+    for (int u = 0; u < kRing; ++u) {
+      load_x(c + u + 1, xr[(u + 1) & 1]);
+      steps(xr[u & 1], wr[u]);
+      load_w(c + u + kRing, wr[u]);
+    }
   }
-  if (c < nc) steps(xr[0], wr[0]);
+#pragma unroll
+  for (int u = 0; u + 1 < kRing; ++u) {
+    if (c + u < nc) {
+      load_x(c + u + 1, xr[(u + 1) & 1]);
+      steps(xr[u & 1], wr[u]);
+    }
+  }
   // lane holds tokens t0 + 4 b + r, expert e0 + jj; chain 4g + bb at acc[g][4 bb + r]
   const int e = e0 + jj;
 #pragma unroll
@@ -826,8 +912,13 @@ __global__ __launch_bounds__(256) void k_router_mfma(const uint16_t* __restrict_
 hipError_t launch_router_mfma(const LayerDev& L, const uint16_t* xhi, const int* need_lo, int T,
                               float* z, hipStream_t st) {
   const size_t lds = (size_t)16 * (16 * (L.H / 16) + 8) * sizeof(uint16_t);
-  hipLaunchKernelGGL(k_router_mfma, dim3((L.E + 63) / 64 + 1, (T + 15) / 16), dim3(256), lds, st,
-                     xhi, need_lo, L.router, L.H, L.E, T, L, z);
+  const int tiles = (T + 15) / 16;
+  if (tiles * ((L.E + 63) / 64) <= persistent_wgs())
+    hipLaunchKernelGGL(k_router_mfma<4>, dim3((L.E + 63) / 64 + 1, tiles), dim3(256), lds, st, xhi,
+                       need_lo, L.router, L.H, L.E, T, L, z);
+  else
+    hipLaunchKernelGGL(k_router_mfma<8>, dim3((L.E + 127) / 128, tiles), dim3(512), lds, st, xhi,
+                       need_lo, L.router, L.H, L.E, T, L, z);
   return hipGetLastError();
 }
 
@@ -1042,7 +1133,7 @@ hipError_t launch_down_dec(const LayerDev& L, const float* h, int ldh, const int
 // a chain of H dependent adds, which bounds the kernel; up to 2048 elements
 // on one wave in rounds (seq_sum_wave_rounds; rows of the staged squares padded
 // by one word, so that writing along and reading across them both use every
-// bank: 1533 tokens of 2048 33 -> 26 us, 8 tokens 12 -> 8), else on one thread.
+// bank: 1533 tokens of 2048 33 -> 26 us, calls of 8 tokens 3 us less), else on one thread.
 // Otherwise 256 strided partials and a halving
 // tree (the order of the fused decode kernel's tree mode).
 // ===========================================================================
