@@ -1781,7 +1781,8 @@ hipError_t launch_gguf_units(const GgufMoeDev& L, const float* x, int T, const i
   // more, so that more workgroups share a CU) and rows per wave.
   const int usz = gguf_unit_tokens(L, T);
   const bool tm8 = usz == 8;
-  // rows per wave: enough waves for the device first, then fewer of them
+  // rows per wave: enough waves for the device first, then fewer of them (at
+  // 2048 / 512 4, 8 and 16 rows measure within 1 % from 6 tokens on)
   const auto rpw_of = [&](int64_t n) { return n >= 49152 ? 16 : n >= 24576 ? 8 : 4; };
   const int rpw_g = rpw_of((int64_t)nunits * rows), rpw_d = rpw_of((int64_t)nunits * L.H / 2);
   if (tm8 && L.H > 1024) {
