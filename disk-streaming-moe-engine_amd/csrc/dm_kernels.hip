@@ -1130,12 +1130,13 @@ hipError_t launch_down_dec(const LayerDev& L, const float* h, int ldh, const int
 // RMSNorm per token (src/layers/rmsnorm.mojo:41-48): out = x / denom *
 // gamma, denom = sqrt(sum(x * x) / H + eps), for the block-edge norm of
 // several tokens.  SEQ: the squares added in element order, the reference's:
-// a chain of H dependent adds, which bounds the kernel; up to 2048 elements
-// on one wave in rounds (seq_sum_wave_rounds; rows of the staged squares padded
+// a chain of H dependent adds, which bounds the kernel.  2048 elements run on
+// one wave in rounds (seq_sum_wave_rounds; rows of the staged squares padded
 // by one word, so that writing along and reading across them both use every
-// bank: 1533 tokens of 2048 33 -> 26 us, calls of 8 tokens 3 us less), else on one thread.
-// Otherwise 256 strided partials and a halving
-// tree (the order of the fused decode kernel's tree mode).
+// bank: 1533 tokens 33 -> 26 us, calls of 8 tokens 3 us less), other sizes on
+// one thread (with 640 elements the rounds' steps past a lane's ten took 5 us
+// more).  Otherwise 256 strided partials and a halving tree (the order of the
+// fused decode kernel's tree mode).
 // ===========================================================================
 template <bool SEQ>
 __global__ __launch_bounds__(256) void k_rmsnorm_rows(const float* __restrict__ x, int H,
@@ -1146,14 +1147,13 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows(const float* __restrict__ 
   const float* xr = x + (size_t)t * H;
   if (SEQ) {
     static_assert(kSeqPerLane * 65 <= kNormMaxH, "padded rows");
-    const bool rounds = H % 64 == 0 && H <= 64 * kSeqPerLane;
-    const int per = H / 64;
+    const bool rounds = H == 64 * kSeqPerLane;
     for (int i = threadIdx.x; i < H; i += 256)
-      part[rounds ? (i % per) * 65 + i / per : i] = xr[i] * xr[i];
+      part[rounds ? (i % kSeqPerLane) * 65 + i / kSeqPerLane : i] = xr[i] * xr[i];
     __syncthreads();
     float a = 0.0f;
     if (rounds) {
-      if (threadIdx.x < 64) a = seq_sum_wave_rounds(part, per, 65);
+      if (threadIdx.x < 64) a = seq_sum_wave_rounds(part, kSeqPerLane, 65);
     } else if (threadIdx.x == 0) {
       a = seq_sum_squares(part, H & ~31);
       for (int i = H & ~31; i < H; ++i) a = a + part[i];
