@@ -720,14 +720,18 @@ hipError_t launch_router_dec(const LayerDev& L, const float* x, int T, float* z,
 // for two on a CU: NW = 4 while every workgroup has a CU of its own (131
 // tokens: 23 us, 25 with the gate inside), NW = 8 beyond (2048 tokens, 256
 // experts: 256 workgroups in one round, 46 -> 34 us; with the gate's
-// workgroups apart 51).  The tokens' activations are
+// workgroups apart 51).  SPLIT, for few tokens: 16 experts per workgroup, wave g
+// running their chains 4g .. 4g + 3 (a quarter of the matrix instructions, and all
+// its router words requested before the staging), the chains then joined
+// through LDS in the halving tree's order; while every workgroup has a CU of its
+// own (131 tokens 22 -> 11 us).  The tokens' activations are
 // staged once in LDS in chain-major order: xs[i][l][s] = x[t0 + i][16 s + l]
 // (bf16), rows padded by 16 bytes so that the 16 lanes of one operand fetch
 // hit distinct banks.
 // ===========================================================================
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-template <int NW>
+template <int NW, bool SPLIT>
 __global__ __launch_bounds__(64 * NW) void k_router_mfma(const uint16_t* __restrict__ xhi,
                                                       const int* __restrict__ need_lo,
                                                       const uint16_t* __restrict__ router_, int H_,
@@ -743,19 +747,21 @@ __global__ __launch_bounds__(64 * NW) void k_router_mfma(const uint16_t* __restr
   const int H = L.H, E = L.E, ns = H / 16;
   const int pitch = 16 * ns + 8;  // elements per staged token (16 B of padding)
   const int t0 = blockIdx.y * 16, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int e0 = 16 * (blockIdx.x * NW + w), b = lane >> 4, jj = lane & 15, nc = ns / 8;
+  const int e0 = 16 * (SPLIT ? blockIdx.x : blockIdx.x * NW + w), b = lane >> 4, jj = lane & 15, nc = ns / 8;
   // the wave's first router words, requested before the staging (the router
   // comes from HBM when a layer's turn comes): steps 8c .. 8c + 7 of its chains,
   // two rounds ahead of their products, four with one workgroup of four waves
   // per CU (131 tokens 23 -> 22 us; with eight waves 35 -> 39); requests clamped
   // to the last round
-  constexpr int kRing = NW == 4 ? 4 : 2;
-  const uint16_t* wb = L.router + r16_index(H, min(e0 + jj, E - 1), b);
-  uint4 wr[kRing][4];
-  auto load_w = [&](int c, uint4 (&d)[4]) {
+  constexpr int kRing = SPLIT ? 16 : NW == 4 ? 4 : 2;
+  constexpr int kG = SPLIT ? 1 : 4;  // groups of four chains of a wave: g, or its own
+  const int g0 = SPLIT ? w : 0;
+  const uint16_t* wb = L.router + r16_index(H, min(e0 + jj, E - 1), b) + 4 * g0 * 8;
+  uint4 wr[kRing][kG];
+  auto load_w = [&](int c, uint4 (&d)[kG]) {
     const int cc = min(c, nc - 1);
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
+    for (int g = 0; g < kG; ++g)
       d[g] = *reinterpret_cast<const uint4*>(wb + (size_t)cc * 128 + 4 * g * 8);
   };
 #pragma unroll
@@ -802,7 +808,7 @@ __global__ __launch_bounds__(64 * NW) void k_router_mfma(const uint16_t* __restr
     }
   }
   __syncthreads();
-  if (NW == 4 ? (int)blockIdx.x == (E + 63) / 64 : blockIdx.x == 0 && w < 4) {
+  if (NW == 4 ? blockIdx.x == gridDim.x - 1 : blockIdx.x == 0 && w < 4) {
     // shared-expert gate: lane (token i, chain l), 8 steps per 16-byte read
     const int i = tid >> 4, l = tid & 15;
     const uint16_t* xr = xs + i * pitch + l * ns;
@@ -836,32 +842,32 @@ __global__ __launch_bounds__(64 * NW) void k_router_mfma(const uint16_t* __restr
     if (l == 0 && t0 + i < T) z[(size_t)(t0 + i) * (E + 1) + E] = acc;
     if (NW == 4) return;
   }
-  if (e0 >= E) return;  // uniform per wave (no barrier below)
+  if (e0 >= E) return;  // uniform per wave (SPLIT: per workgroup; else no barrier below)
   // A: token jj (as row i = lane & 15 of block b), chain 4g + b
-  const uint16_t* xa = xs + jj * pitch + b * ns;
-  f32x16 acc[4];
+  const uint16_t* xa = xs + jj * pitch + (4 * g0 + b) * ns;
+  f32x16 acc[kG];
 #pragma unroll
-  for (int g = 0; g < 4; ++g) acc[g] = f32x16{};
+  for (int g = 0; g < kG; ++g) acc[g] = f32x16{};
   // x from LDS one round ahead
-  uint4 xr[2][4];
-  auto load_x = [&](int c, uint4 (&d)[4]) {
+  uint4 xr[2][kG];
+  auto load_x = [&](int c, uint4 (&d)[kG]) {
     const int cc = min(c, nc - 1);
 #pragma unroll
-    for (int g = 0; g < 4; ++g) d[g] = *reinterpret_cast<const uint4*>(xa + 4 * g * ns + 8 * cc);
+    for (int g = 0; g < kG; ++g) d[g] = *reinterpret_cast<const uint4*>(xa + 4 * g * ns + 8 * cc);
   };
   // the four accumulators' steps interleaved (each one's steps in order),
   // so that consecutive matrix instructions are independent
-  auto steps = [&](const uint4 (&xv)[4], const uint4 (&wv)[4]) {
+  auto steps = [&](const uint4 (&xv)[kG], const uint4 (&wv)[kG]) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
+      for (int g = 0; g < kG; ++g) {
         const uint32_t xw = u == 0 ? xv[g].x : u == 1 ? xv[g].y : u == 2 ? xv[g].z : xv[g].w;
         const uint32_t ww = u == 0 ? wv[g].x : u == 1 ? wv[g].y : u == 2 ? wv[g].z : wv[g].w;
         acc[g] = __builtin_amdgcn_mfma_f32_16x16x1f32(bf16lo(xw), bf16lo(ww), acc[g], 0, 0, 0);
       }
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
+      for (int g = 0; g < kG; ++g) {
         const uint32_t xw = u == 0 ? xv[g].x : u == 1 ? xv[g].y : u == 2 ? xv[g].z : xv[g].w;
         const uint32_t ww = u == 0 ? wv[g].x : u == 1 ? wv[g].y : u == 2 ? wv[g].z : wv[g].w;
         acc[g] = __builtin_amdgcn_mfma_f32_16x16x1f32(bf16hi(xw), bf16hi(ww), acc[g], 0, 0, 0);
@@ -887,38 +893,56 @@ __global__ __launch_bounds__(64 * NW) void k_router_mfma(const uint16_t* __restr
   }
   // lane holds tokens t0 + 4 b + r, expert e0 + jj; chain 4g + bb at acc[g][4 bb + r]
   const int e = e0 + jj;
+  auto join = [&](const float (&u)[4][4], int r) {  // the halving tree over the 16 chains
+    float v[4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    float v[4][4];
+    for (int bb = 0; bb < 4; ++bb)  // w = 8: chain l += chain l + 8; w = 4
+      v[bb] = (u[0][bb] + u[2][bb]) + (u[1][bb] + u[3][bb]);
+    const float s = (v[0] + v[2]) + (v[1] + v[3]);  // w = 2, 1
+    const int t = t0 + 4 * b + r;
+    if (t < T && e < E) z[(size_t)t * (E + 1) + e] = s;
+  };
+  if constexpr (SPLIT) {
+    float* part = reinterpret_cast<float*>(xs_chain);  // [4 g][16][64 lanes]
+    __syncthreads();  // the staged activations are no longer read
+#pragma unroll
+    for (int i = 0; i < 16; ++i) part[(w * 16 + i) * 64 + lane] = acc[0][i];
+    __syncthreads();
+    float u[4][4];  // wave w: r = w
 #pragma unroll
     for (int g = 0; g < 4; ++g)
 #pragma unroll
-      for (int bb = 0; bb < 4; ++bb) v[g][bb] = acc[g][4 * bb + r];
+      for (int bb = 0; bb < 4; ++bb) u[g][bb] = part[(g * 16 + 4 * bb + w) * 64 + lane];
+    join(u, w);
+  } else {
 #pragma unroll
-    for (int bb = 0; bb < 4; ++bb) {  // w = 8: chain l += chain l + 8
-      v[0][bb] = v[0][bb] + v[2][bb];
-      v[1][bb] = v[1][bb] + v[3][bb];
+    for (int r = 0; r < 4; ++r) {
+      float u[4][4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int bb = 0; bb < 4; ++bb) u[g][bb] = acc[g][4 * bb + r];
+      join(u, r);
     }
-#pragma unroll
-    for (int bb = 0; bb < 4; ++bb) v[0][bb] = v[0][bb] + v[1][bb];  // w = 4
-    v[0][0] = v[0][0] + v[0][2];  // w = 2
-    v[0][1] = v[0][1] + v[0][3];
-    const float s = v[0][0] + v[0][1];  // w = 1
-    const int t = t0 + 4 * b + r;
-    if (t < T && e < E) z[(size_t)t * (E + 1) + e] = s;
   }
 }
 
 hipError_t launch_router_mfma(const LayerDev& L, const uint16_t* xhi, const int* need_lo, int T,
                               float* z, hipStream_t st) {
-  const size_t lds = (size_t)16 * (16 * (L.H / 16) + 8) * sizeof(uint16_t);
-  const int tiles = (T + 15) / 16;
-  if (tiles * ((L.E + 63) / 64) <= persistent_wgs())
-    hipLaunchKernelGGL(k_router_mfma<4>, dim3((L.E + 63) / 64 + 1, tiles), dim3(256), lds, st, xhi,
-                       need_lo, L.router, L.H, L.E, T, L, z);
+  // the staged activations, then (SPLIT) the 16 KB of the chains' sums
+  size_t lds = (size_t)16 * (16 * (L.H / 16) + 8) * sizeof(uint16_t);
+  if (lds < 16384) lds = 16384;
+  const int tiles = (T + 15) / 16, cus = persistent_wgs();
+#define DM_ROUTER_MFMA(NW, SPLIT, COLS)                                                          \
+  hipLaunchKernelGGL((k_router_mfma<NW, SPLIT>), dim3(COLS, tiles), dim3(64 * NW), lds, st, xhi, \
+                     need_lo, L.router, L.H, L.E, T, L, z)
+  if (tiles * ((L.E + 15) / 16 + 1) <= cus)
+    DM_ROUTER_MFMA(4, true, (L.E + 15) / 16 + 1);
+  else if (tiles * ((L.E + 63) / 64) <= cus)
+    DM_ROUTER_MFMA(4, false, (L.E + 63) / 64 + 1);
   else
-    hipLaunchKernelGGL(k_router_mfma<8>, dim3((L.E + 127) / 128, tiles), dim3(512), lds, st, xhi,
-                       need_lo, L.router, L.H, L.E, T, L, z);
+    DM_ROUTER_MFMA(8, false, (L.E + 127) / 128);
+#undef DM_ROUTER_MFMA
   return hipGetLastError();
 }
 
