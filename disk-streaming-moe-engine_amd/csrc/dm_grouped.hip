@@ -1084,10 +1084,10 @@ __global__ __launch_bounds__(256) void k_combine(const float* __restrict__ r,
                                                   const float* __restrict__ residual, int H, int K,
                                                   float* __restrict__ y,
                                                   unsigned long long* status,
-                                                  int* __restrict__ clear_flag) {
+                                                  int* __restrict__ clear_flag, int t0) {
   // four consecutive outputs per thread (H % 4 == 0); the slots' rows are
   // requested eight at a time before their products
-  const int t = blockIdx.y, d = (blockIdx.x * 256 + threadIdx.x) * 4;
+  const int t = t0 + blockIdx.y, d = (blockIdx.x * 256 + threadIdx.x) * 4;
   // the last kernel of a call clears the call's need-lo flag for the next
   if (clear_flag && t == 0 && d == 0) *clear_flag = 0;
   if (d >= H) return;
@@ -1132,8 +1132,11 @@ hipError_t launch_combine(const float* r, const float* rs, const float* probs, c
                           const float* residual, int T, int H, int K, float* y,
                           unsigned long long* status, hipStream_t st, int* clear_flag) {
   if (H % 4) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_combine, dim3((H / 4 + 255) / 256, T), dim3(256), 0, st, r, rs, probs, shg,
-                     residual, H, K, y, status, clear_flag);
+  for (int t0 = 0; t0 < T; t0 += 65535) {  // grid.y holds at most 65535 tokens
+    const int n = T - t0 < 65535 ? T - t0 : 65535;
+    hipLaunchKernelGGL(k_combine, dim3((H / 4 + 255) / 256, n), dim3(256), 0, st, r, rs, probs, shg,
+                       residual, H, K, y, status, clear_flag, t0);
+  }
   return hipGetLastError();
 }
 

@@ -142,6 +142,24 @@ def test_rows_of_any_scale(block, oracle, tmp_path, ty):
     block.free_layer_gguf(65)
 
 
+def test_more_tokens_than_one_launch_combines(block, oracle, tmp_path):
+    """65537 tokens: the combine splits at 65535; rows on either side of the
+    split against float64, and the same bits as in a call of their own of 256
+    tokens."""
+    dims, T = (128, 4, 2, 128, 128), 65537
+    g = _upload(block, tmp_path, 67, dims, 11)
+    x = np.random.default_rng(11).standard_normal((T, 128)).astype(np.float32)
+    y, ids, probs, shg = block.forward_port_moe_gguf(x, None, 67, T)
+    y2, ids2, _, _ = block.forward_port_moe_gguf(x[-256:], None, 67, 256)
+    assert np.array_equal(ids[-256:], ids2)
+    assert np.array_equal(y[-256:].view(np.uint32), y2.view(np.uint32))
+    rows = np.array([0, 65534, 65535, 65536])
+    ref = _reference(oracle, g, dims, x[rows], ids[rows], probs[rows], shg[rows])
+    err = np.linalg.norm(y[rows] - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert err.max() < BAR, err
+    block.free_layer_gguf(67)
+
+
 def test_errors(block, tmp_path):
     """The texts of the other forms: a non-finite activation, an infinite
     super-scale in a shared and in a routed expert."""
