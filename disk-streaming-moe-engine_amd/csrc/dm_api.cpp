@@ -689,7 +689,7 @@ hipError_t run_gguf_block(dmh_ctx* c, GgufLayer* G, unsigned long long* status, 
   if (T > 1 && L.E <= kGgufGroupMaxE && (dm::gguf_units_pay(L, T) || dm::gguf_mm_ok(L, G->tiles, T))) {
     // several tokens: grouped by expert, each expert row read once per unit
     const bool mm = dm::gguf_mm_ok(L, G->tiles, T);
-    const int tok = mm ? dm::kGgufMmTok : dm::gguf_unit_tokens(L, T);
+    const int tok = mm ? dm::gguf_mm_tok(L) : dm::gguf_unit_tokens(L, T);
     const int nu = dm::group_units_max(T, L.K, L.E, tok);
     if ((e = c->g_off.ensure(L.E + 1)) != hipSuccess) return e;
     if ((e = c->g_perm.ensure((size_t)T * L.K)) != hipSuccess) return e;
@@ -704,8 +704,8 @@ hipError_t run_gguf_block(dmh_ctx* c, GgufLayer* G, unsigned long long* status, 
       const size_t TK = (size_t)T * L.K, TH = (size_t)T * L.H;
       const size_t hn = TK * L.I + (size_t)T * L.Ish;
       const size_t xsum = dm::gguf_mm_sums(L, (int64_t)TH);
-      if ((e = c->g_xhi.ensure(2 * TH)) != hipSuccess) return e;
-      if ((e = c->g_hr.ensure(2 * hn)) != hipSuccess) return e;
+      if ((e = c->g_xhi.ensure(3 * TH)) != hipSuccess) return e;
+      if ((e = c->g_hr.ensure(3 * hn)) != hipSuccess) return e;
       if ((e = c->g_ex.ensure(T + TK + T)) != hipSuccess) return e;
       if ((e = c->g_sums.ensure(xsum + dm::gguf_mm_sums(L, (int64_t)hn) + 1)) != hipSuccess)
         return e;

@@ -85,24 +85,26 @@ size_t gguf_tiles_bytes(const GgufMoeDev& L);
 hipError_t launch_gguf_tiles(const GgufMoeDev& L, uint8_t* out, hipStream_t st);
 // Fewest tokens of the matrix-core form.  Below, a call gives every token
 // the bits of its own single-token call, whatever it is batched with; from
-// here on the sums run in the matrix cores' order (as exact, other bits).
+// here on the sums run in the matrix cores' order (as exact, other bits).  The
+// line keeps decode batches on the former: by speed alone it would lie lower
+// (Qwen3.6 shape, Q3_K 444 us at 200 tokens grouped, 229 at 256 here).
 constexpr int kGgufMmMinT = 256;
-constexpr int kGgufMmTok = 64;  // tokens per unit
+int gguf_mm_tok(const GgufMoeDev& L);  // tokens per unit
 // tiles: the records of launch_gguf_tiles, or null.  (Not a member of GgufMoeDev:
 // eight more bytes of arguments cost the one-token launch 0.1 us.)
 bool gguf_mm_ok(const GgufMoeDev& L, const uint8_t* tiles, int T);
 // Elements of the column sums of `elements` activations (0: not needed).
 size_t gguf_mm_sums(const GgufMoeDev& L, int64_t elements);
 struct GgufMmScratch {
-  uint16_t* xs;    // [T][H][2] x in f16 parts
-  uint16_t* hs;    // [T K][I][2], [T][Ish][2] h in f16 parts
+  uint16_t* xs;    // [T][H][3] x in f16 parts
+  uint16_t* hs;    // [T K][I][3], [T][Ish][3] h in f16 parts
   int32_t* ex;     // [T] exponents of x, [T K + T] of h
   uint16_t* xsum;  // gguf_mm_sums(T H) column sums of x
   uint16_t* hsum;  // gguf_mm_sums(T K I + T Ish) of h
   float* h;        // [T K][I], [T][Ish]
 };
 // The experts' outputs of T tokens grouped by expert (off, perm, units, meta
-// of launch_group_build with tok = kGgufMmTok, nunits = group_units_max): r [T*K][H] by
+// of launch_group_build with tok = gguf_mm_tok, nunits = group_units_max): r [T*K][H] by
 // assignment, rs [T][H] of the shared expert, unweighted, with the checks of
 // launch_gguf_units; launch_combine forms y from them.
 hipError_t launch_gguf_mm(const GgufMoeDev& L, const uint8_t* tiles, const float* x, int T, const int32_t* off,

@@ -6,18 +6,23 @@
 // (s - 32)(q - 4) (at most 892 in magnitude), s q (at most 945) and q (8
 // bits) are exact in f16, so they enter v_mfma_f32_16x16x32_f16 as they are,
 // and the block scale d multiplies the fp32 partial sum of its columns.  An
-// fp32 activation enters as two f16 parts, hi = f16(x 2^s) and
-// lo = f16(x 2^s - hi), with s such that the row's largest value lies in
-// [2^14, 2^15): the parts keep 24 bits of it (the error is at most 2^-24 of
-// the value, and below 2^-39 of the row's largest value for the small
-// ones).  Both parts' products go into one fp32 accumulator.  Against 64
-// bits the block's outputs are as far off as those of the fp32 lane sums of
-// dm_gguf.hip (measured over the Qwen3.6 shape and ragged ones: see
-// tests/test_gpu_gguf_mm.py).
+// fp32 activation enters whole, as three f16 parts (two hold 23 of its 24
+// bits): with s such that the row's largest value lies in [2^14, 2^15),
+// hi = f16(x 2^s), mid = f16(2^12 (x 2^s - hi)) and lo = 2^12 (x 2^s - hi) -
+// mid.  mid and lo meet the integers times 2^-12, exact in f16 too, so all
+// products go into one fp32 accumulator, and a value far below its row's
+// largest keeps its bits: hi + 2^-12 (mid + lo) is x 2^s exactly down to 2^-27
+// of the largest value, and within 2^-51 of that value below.  (hi and a lo
+// part unscaled lose bits from 2^-16 on, which counts where the weight at the
+// largest value is zero: relative errors of 3e-4 to 2e-3 in a block's outputs
+// against 2e-7 to 1e-6, and of the whole result where the leading bits of two
+// activations cancel.)  Against 64 bits the block's outputs are as far off as
+// those of the fp32 lane sums of dm_gguf.hip, or closer
+// (tests/test_gpu_gguf_mm.py).
 //
 //   k_gguf_tile   (at upload) expert payloads -> records of 16 rows x 64
 //                 columns in the order the matrix cores read them
-//   k_gguf_split  fp32 rows -> f16 parts, hi and lo of 64 columns side by
+//   k_gguf_split  fp32 rows -> f16 parts, the three of 64 columns side by
 //                 side, and the row's exponent; Q4_K: the sums of 32 columns
 //   k_gguf_mm     gate/up (h = SiLU(g) u) and down products over the units of
 //                 launch_group_build
@@ -37,7 +42,9 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kMmCols = 64;                   // columns of a record and of a stage
 constexpr int kMmThreads = 512;               // 8 waves
-constexpr int kMmRowBytes = kMmCols * 2 * 2;  // a token row's hi and lo parts of a stage
+constexpr int kMmRowBytes = kMmCols * 2 * 2;  // a token row's hi and mid parts of a stage
+constexpr int kMmRow3 = kMmCols * 3;          // elements of a token row and stage, all parts
+constexpr float kMmMid = 4096.0f;             // scale of mid and lo
 
 // Bytes of a record: the codes (lane l of a wave: row l & 15, columns
 // 8 (l >> 4) .. + 7 of each 32), then the scales.
@@ -54,16 +61,26 @@ struct Rec {
   // direct-to-LDS loads of a wave and stage besides those of the token rows
   static constexpr int kDma = kCodes / 512 + 1 + (kSums ? 1 : 0);
 };
-// Stages of NCT column tiles: token rows, the 16 tiles' codes, their scales,
-// the column sums.  Two workgroups share a CU (160 KB).
+// Tokens per unit: 64, where two workgroups' stages fit a CU (160 KB); the
+// codes of Q8_0 leave room for 48.
+constexpr int mm_tok(int type) { return type == kGgmlQ8_0 ? 48 : 64; }
+// Stages of NCT column tiles: token rows (hi and mid, then lo), the 16 tiles'
+// codes, their scales, the column sums.
 template <int TY, int NCT>
 struct MmBuf {
-  static constexpr int kAhead = NCT == 4 ? 1 : 2;     // stages in flight
+  // stages in flight
+  static constexpr int kAhead = NCT > 2 || (NCT == 2 && TY == kGgmlQ8_0) ? 1 : 2;
   static constexpr int kBufs = kAhead + 1;
-  static constexpr int kB = 16 * NCT * kMmRowBytes;
+  static constexpr int kLoAt = 16 * NCT * kMmRowBytes;
+  static constexpr int kB = kLoAt + kLoAt / 2;
   static constexpr int kSumsAt = kB + 16 * Rec<TY>::kBytes;
-  static constexpr int kBytes = kSumsAt + (Rec<TY>::kSums ? 16 * NCT * 16 : 0);
-  static constexpr int kRowLoads = NCT == 4 ? 2 : 1;  // of 32 rows over the 8 waves
+  static constexpr int kBytes = kSumsAt + (Rec<TY>::kSums ? 16 * NCT * 32 : 0);
+  static constexpr int kRowLoads = NCT > 2 ? 2 : 1;  // of 32 rows over the 8 waves
+  // The lo parts lie two rows to a line of 256 bytes.  Four column tiles: line r
+  // holds rows r and r + 32, segment c of row r + 32 m at (8 m + c) ^ (r & 15), so
+  // that the addresses are those of the hi and mid parts; else line l holds rows
+  // 2 l + m, segment c at 8 m + (c ^ (l & 7)).
+  static constexpr bool kLoFar = NCT == 4;
 };
 int rec_bytes(int type) {
   switch (type) {
@@ -185,10 +202,22 @@ __global__ __launch_bounds__(256) void k_gguf_tile(GgufMoeDev L, uint8_t* __rest
 }
 
 // ---- activations ---------------------------------------------------------------
+struct F16Parts {
+  _Float16 hi, mid, lo;
+};
+__device__ __forceinline__ F16Parts split3(float x) {
+  F16Parts p;
+  p.hi = (_Float16)x;
+  const float r = (x - (float)p.hi) * kMmMid;  // exact
+  p.mid = (_Float16)r;
+  p.lo = (_Float16)(r - (float)p.mid);
+  return p;
+}
+
 // Wave per row: rows [0, na) of a (width wa), then rows of b (width wb), the
 // parts one after the other in out, exponents in ex.  Row layout: per 64
-// columns 64 hi parts, 64 lo parts.  sums (Q4_K): per 128 columns the f16
-// parts [4 hi][4 lo] of the sums of 32 columns.
+// columns 64 hi, 64 mid, 64 lo parts.  sums (Q4_K): per 128 columns the f16
+// parts [4 hi][4 mid][4 lo][4 zeros] of the sums of 32 columns.
 template <bool SUMS>
 __global__ __launch_bounds__(256) void k_gguf_split(const float* __restrict__ a, int64_t na, int wa,
                                                     const float* __restrict__ b, int64_t nb, int wb,
@@ -218,21 +247,24 @@ __global__ __launch_bounds__(256) void k_gguf_split(const float* __restrict__ a,
   for (int c0 = 0; c0 < n; c0 += 512) {
     const int c = c0 + lane * 8;
     const bool in = c < n;
-    f16x8 hi, lo;
+    f16x8 hi, mid, lo;
     float sum = 0.0f;
     const f32x4 u = *reinterpret_cast<const f32x4*>(src + (in ? c : 0));
     const f32x4 v = *reinterpret_cast<const f32x4*>(src + (in ? c + 4 : 4));
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const float x = __builtin_amdgcn_ldexpf(i < 4 ? u[i & 3] : v[i & 3], s);
-      hi[i] = (_Float16)x;
-      lo[i] = (_Float16)(x - (float)hi[i]);
+      const F16Parts p = split3(x);
+      hi[i] = p.hi;
+      mid[i] = p.mid;
+      lo[i] = p.lo;
       sum = sum + x;
     }
     if (in) {
-      uint16_t* dst = out + 2 * (o + (c & ~63)) + (c & 63);
+      uint16_t* dst = out + 3 * (o + (c & ~63)) + (c & 63);
       *reinterpret_cast<f16x8*>(dst) = hi;
-      *reinterpret_cast<f16x8*>(dst + 64) = lo;
+      *reinterpret_cast<f16x8*>(dst + 64) = mid;
+      *reinterpret_cast<f16x8*>(dst + 128) = lo;
     }
     if constexpr (SUMS) {
       // sums of 32 columns: four lanes; sixteen lanes hold the four of 128.
@@ -240,14 +272,19 @@ __global__ __launch_bounds__(256) void k_gguf_split(const float* __restrict__ a,
       sum = sum + __shfl_xor(sum, 1, 64);
       sum = sum + __shfl_xor(sum, 2, 64);
       const float q = sum * 0.03125f;
-      f16x8 p;
+      f16x8 p, p2{};
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float t = __shfl(q, (lane & 48) + 4 * j, 64);
-        p[j] = (_Float16)t;
-        p[4 + j] = (_Float16)(t - (float)p[j]);
+        const F16Parts t = split3(__shfl(q, (lane & 48) + 4 * j, 64));
+        p[j] = t.hi;
+        p[4 + j] = t.mid;
+        p2[j] = t.lo;
       }
-      if (in && (lane & 15) == 0) *reinterpret_cast<f16x8*>(sums + (o + c) / 128 * 8) = p;
+      if (in && (lane & 15) == 0) {
+        f16x8* dst = reinterpret_cast<f16x8*>(sums + (o + c) / 128 * 16);
+        dst[0] = p;
+        dst[1] = p2;
+      }
     }
   }
 }
@@ -279,18 +316,20 @@ template <int N>
 __device__ __forceinline__ void vm_wait() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
 }
-// N B fragments of column tiles CT0 .. of a staged k-group as LDS reads in
-// flight together (16 rows of 256 bytes apart); not valid before lds_wait.
-template <int CT0, int N>
+// N B fragments of a staged k-group at byte AT from a as LDS reads in flight
+// together, PITCH bytes apart; not valid before lds_wait.
+template <int AT, int PITCH, int N>
 __device__ __forceinline__ void lds_read_b(uint32_t a, f16x8 (&b)[N]) {
 #pragma unroll
   for (int i = 0; i < N; ++i)
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(b[i]) : "v"(a), "n"((CT0 + i) * 16 * kMmRowBytes));
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(b[i]) : "v"(a), "n"(AT + i * PITCH));
 }
 // until at most M LDS operations are in flight; b's registers tied
 template <int N, int M>
 __device__ __forceinline__ void lds_wait_b(f16x8 (&b)[N]) {
-  if constexpr (N == 2)
+  if constexpr (N == 3)
+    asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(b[0]), "+v"(b[1]), "+v"(b[2]) : "n"(M));
+  else if constexpr (N == 2)
     asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(b[0]), "+v"(b[1]) : "n"(M));
   else
     asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(b[0]) : "n"(M));
@@ -344,24 +383,24 @@ struct MmAcc {
   f32x4 c[2][NCT];  // K-quants: the integer products of the columns that share a d
 };
 
-// One stage: 2 tiles x NCT column tiles x 64 columns x (hi, lo).  ODD: the
+// One stage: 2 tiles x NCT column tiles x 64 columns x (hi, mid, lo).  ODD: the
 // second stage of 128 columns, which ends the K-quants' partial sums.
 //
-// Its steps Z: column group kg of 32, group of up to two column tiles, part
-// (hi, lo), the part running fastest; the B fragments of step Z + 1 are read
+// Its steps Z: column group kg of 32, part (hi, mid, lo), group of up to three
+// column tiles, running fastest; the B fragments of step Z + 1 are read
 // while step Z multiplies.
 template <int TY, int NCT, bool ODD>
 struct MmStage {
   using R = Rec<TY>;
   using S = MmBuf<TY, NCT>;
-  static constexpr int kG = NCT < 2 ? NCT : 2, kNG = NCT / kG, kSteps = 4 * kNG;
-  static constexpr int kg(int z) { return z / (2 * kNG); }
-  static constexpr int part(int z) { return z & 1; }
-  static constexpr int ct0(int z) { return (z >> 1) % kNG * kG; }
+  static constexpr int kG = NCT < 4 ? NCT : 2, kNG = NCT / kG, kSteps = 6 * kNG;
+  static constexpr int kg(int z) { return z / (3 * kNG); }
+  static constexpr int part(int z) { return z / kNG % 3; }
+  static constexpr int ct0(int z) { return z % kNG * kG; }
 
   const unsigned char* st;
   const unsigned char* rs;
-  uint32_t bp;
+  uint32_t bp, bl;  // row j's hi and mid parts, its line of lo parts
   int q, j;
   uint4 cw[2];
   uint32_t sc[2];
@@ -370,13 +409,21 @@ struct MmStage {
 
   template <int Z>
   __device__ __forceinline__ void read() {
-    lds_read_b<ct0(Z), kG>(bp + (uint32_t)(((8 * part(Z) + 4 * kg(Z) + q) ^ j) * 16), b[Z & 1]);
+    constexpr int ct = ct0(Z), k = 4 * kg(Z);
+    if constexpr (part(Z) < 2)
+      lds_read_b<ct * 16 * kMmRowBytes, 16 * kMmRowBytes>(
+          bp + (uint32_t)(((8 * part(Z) + k + q) ^ j) * 16), b[Z & 1]);
+    else if constexpr (S::kLoFar)
+      lds_read_b<S::kLoAt, 16 * kMmRowBytes>(bp + (uint32_t)(((4 * ct + k + q) ^ j) * 16), b[Z & 1]);
+    else
+      lds_read_b<S::kLoAt + ct * 8 * kMmRowBytes, 8 * kMmRowBytes>(
+          bl + (uint32_t)((8 * (j & 1) + ((k + q) ^ (j >> 1))) * 16), b[Z & 1]);
   }
 
   template <int Z>
   __device__ __forceinline__ void steps(MmAcc<NCT>& A) {
     if constexpr (Z < kSteps) {
-      if constexpr (Z % (2 * kNG) == 0) {
+      if constexpr (Z % (3 * kNG) == 0) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           if constexpr (TY == kGgmlQ8_0) {
@@ -387,6 +434,10 @@ struct MmStage {
             a[t] = codes4(kg(Z) ? cw[t].y : cw[t].x, s, s * f16x2{(_Float16)kBias, (_Float16)kBias});
           }
         }
+      }
+      if constexpr (part(Z) == 1 && ct0(Z) == 0) {  // for mid and lo
+#pragma unroll
+        for (int t = 0; t < 2; ++t) a[t] = a[t] * (_Float16)(1.0f / kMmMid);
       }
       if constexpr (Z + 1 < kSteps) {
         read<Z + 1>();
@@ -403,7 +454,7 @@ struct MmStage {
           f32x4& c = A.c[t][ct0(Z) + i];
           c = mfma_f16(a[t], b[Z & 1][i], kStart ? f32x4{0, 0, 0, 0} : c);
         }
-      if constexpr (TY == kGgmlQ8_0 && part(Z) == 1) {
+      if constexpr (TY == kGgmlQ8_0 && part(Z) == 2) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           const f32x4 d = *reinterpret_cast<const f32x4*>(rs + t * R::kRest + kg(Z) * 64 + 16 * q);
@@ -420,6 +471,10 @@ struct MmStage {
       steps<Z + 1>(A);
     }
   }
+  static __device__ __forceinline__ uint32_t mul_mid(uint32_t w) {
+    constexpr _Float16 k = (_Float16)(1.0f / kMmMid);
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, w) * f16x2{k, k});
+  }
   static __device__ __forceinline__ void fma4(f32x4& m, const f32x4& d, const f32x4& c) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) m[i] = __builtin_fmaf(d[i], c[i], m[i]);
@@ -432,6 +487,7 @@ struct MmStage {
     st = lds + off;
     rs = st + S::kB + 16 * R::kCodes + w * 2 * R::kRest;
     bp = lds_u32(lds) + (uint32_t)(off + j * kMmRowBytes);
+    bl = lds_u32(lds) + (uint32_t)(off + (j >> 1) * kMmRowBytes);
     const unsigned char* cd = st + S::kB + w * 2 * R::kCodes;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -456,15 +512,18 @@ struct MmStage {
         for (int ct = 0; ct < NCT; ++ct) fma4(A.m[t][ct], d, A.c[t][ct]);
         if constexpr (TY == kGgmlQ4_K) {
           // - dmin sum_j m_j (sum of sub-block j's activations): the mins of
-          // the four sub-blocks against the hi and lo parts of 2^-5 the sums
+          // the four sub-blocks against the parts of 2^-5 the sums (lanes 0 .. 15
+          // hi and mid, 16 .. 31 lo)
           const f32x4 dm = *reinterpret_cast<const f32x4*>(rs + t * R::kRest + 192 + 16 * q);
           const f32x4 dn = dm * -32.0f;
-          const uint2 z = q == 0 ? mn[t] : make_uint2(0, 0);
-          const f16x8 am = __builtin_bit_cast(f16x8, make_uint4(z.x, z.y, z.x, z.y));
+          const uint2 z = q < 2 ? mn[t] : make_uint2(0, 0);
+          const uint2 y = make_uint2(mul_mid(z.x), mul_mid(z.y));
+          const f16x8 am = __builtin_bit_cast(
+              f16x8, q == 0 ? make_uint4(z.x, z.y, y.x, y.y) : make_uint4(y.x, y.y, 0, 0));
 #pragma unroll
           for (int ct = 0; ct < NCT; ++ct) {
             const f16x8 bs = *reinterpret_cast<const f16x8*>(st + S::kSumsAt +
-                                                             (16 * ct + j) * 16);
+                                                             (16 * ct + j) * 32 + (q & 1) * 16);
             fma4(A.m[t][ct], dn, mfma_f16(am, bs, f32x4{0, 0, 0, 0}));
           }
         }
@@ -473,12 +532,14 @@ struct MmStage {
   }
 };
 
-constexpr int kMmInfo = kGgufMmTok * (int)sizeof(int2);
+constexpr int kMmInfo = 64 * (int)sizeof(int2);
 template <int TY>
 constexpr int mm_lds() {
-  constexpr int a = MmBuf<TY, 4>::kBufs * MmBuf<TY, 4>::kBytes;
+  constexpr int kMax = mm_tok(TY) / 16;
+  constexpr int a = MmBuf<TY, kMax>::kBufs * MmBuf<TY, kMax>::kBytes;
   constexpr int b = MmBuf<TY, 2>::kBufs * MmBuf<TY, 2>::kBytes;
-  constexpr int n = (a > b ? a : b) + kMmInfo;
+  constexpr int c = MmBuf<TY, 1>::kBufs * MmBuf<TY, 1>::kBytes;
+  constexpr int n = (a > b ? a > c ? a : c : b > c ? b : c) + kMmInfo;
   static_assert(2 * n <= 160 * 1024, "two workgroups per CU");
   return n;
 }
@@ -489,10 +550,11 @@ struct MmRun {
   using S = MmBuf<TY, NCT>;
   const uint8_t* t0;  // this wave's two tiles
   const uint8_t* t1;
-  const uint16_t* b[S::kRowLoads];  // this lane's segment of its token rows
-  const uint16_t* sums;             // and (Q4_K) its row of column sums
+  const uint16_t* b[S::kRowLoads];  // this lane's segment of its token rows: hi or mid
+  const uint16_t* bl;               // lo (unless kLoFar)
+  const uint16_t* sums;             // and (Q4_K) half a row of column sums
   uint32_t l0;
-  int w, lane, nst, nrow;           // stages; row loads of this wave and stage
+  int w, lane, nst, nload;          // stages; loads of this wave and stage
 
   // row of token rows of position r (0 .. n - 1) of a unit
   static __device__ __forceinline__ int row_of(const MmArgs& g, const MmUnit& u, int r) {
@@ -503,10 +565,15 @@ struct MmRun {
   // This wave's loads of stage s.
   __device__ __forceinline__ void issue(int s) {
     const uint32_t st = l0 + (uint32_t)(s % S::kBufs * S::kBytes);
-    if (NCT > 1 || nrow) {  // uniform
 #pragma unroll
-      for (int m = 0; m < S::kRowLoads; ++m)
-        dma16_lds(b[m] + s * (2 * kMmCols), st + (uint32_t)((w + 8 * m) * 1024));
+    for (int m = 0; m < S::kRowLoads; ++m)
+      if (w + 8 * m < 4 * NCT)  // uniform
+        dma16_lds(b[m] + s * kMmRow3, st + (uint32_t)((w + 8 * m) * 1024));
+    if (w < 2 * NCT) {
+      const uint16_t* src = bl;
+      if constexpr (S::kLoFar)  // segment c of row 4 w + q + 32 m, where 8 m + c is b's segment
+        src = ((lane ^ (4 * w + (lane >> 4))) & 8) ? b[S::kRowLoads - 1] + kMmCols : b[0] + 2 * kMmCols;
+      dma16_lds(src + s * kMmRow3, st + (uint32_t)(S::kLoAt + w * 1024));
     }
     const uint8_t* r0 = t0 + (size_t)s * R::kBytes;
     const uint8_t* r1 = t1 + (size_t)s * R::kBytes;
@@ -521,8 +588,8 @@ struct MmRun {
     if (lane < 2 * kl)
       dma16_lds((lane < kl ? r0 : r1) + R::kCodes + (lane < kl ? lane : lane - kl) * 16,
                 st + S::kB + 16 * R::kCodes + (uint32_t)(w * 2 * R::kRest));
-    if (R::kSums && w < NCT && lane < 16)  // (w uniform)
-      dma16_lds(sums + (s >> 1) * 8, st + S::kSumsAt + (uint32_t)(w * 256));
+    if (R::kSums && w < NCT && lane < 32)  // (w uniform)
+      dma16_lds(sums + (s >> 1) * 16, st + S::kSumsAt + (uint32_t)(w * 512));
   }
 
   // Stage s is complete everywhere, and nobody reads stage s - 1 any more,
@@ -534,9 +601,9 @@ struct MmRun {
     if (S::kAhead == 1 || s + 1 >= nst) {
       vm_wait<0>();
     } else {
-      const int n = nrow + kA + (R::kSums && w < NCT ? 1 : 0);  // uniform
-      if (n == kA + 2) vm_wait<kA + 2>();
-      else if (n == kA + 1) vm_wait<kA + 1>();
+      if (nload == kA + 3) vm_wait<kA + 3>();  // uniform
+      else if (nload == kA + 2) vm_wait<kA + 2>();
+      else if (nload == kA + 1) vm_wait<kA + 1>();
       else vm_wait<kA>();
     }
     __builtin_amdgcn_s_barrier();  // ... and every wave's
@@ -567,20 +634,26 @@ struct MmRun {
     }
     const size_t before = !GU && cur.shared ? (size_t)g.T * K * L.I : 0;
     // load m carries rows 4 (w + 8m) .. + 3, stored segment lane & 15 of row r
-    // being its segment (lane & 15) ^ (r & 15)
-    nrow = NCT > 1 || w < 4 ? S::kRowLoads : 0;
+    // being its segment (lane & 15) ^ (r & 15) of hi and mid; the load of the lo
+    // parts lines 4 w .. + 3
+    nload = (w < 4 * NCT ? 1 : 0) + (w < 2 * NCT ? 1 : 0) + (R::kSums && w < NCT ? 1 : 0) +
+            R::kDma - (R::kSums ? 1 : 0);  // (kAhead 2: one row load)
     const int sg = j ^ ((4 * w + q) & 15);
 #pragma unroll
     for (int m = 0; m < S::kRowLoads; ++m)
-      b[m] = g.b + 2 * before + (size_t)row_of(g, cur, 4 * (w + 8 * m) + q) * (2 * KD) + sg * 8;
+      b[m] = g.b + 3 * before + (size_t)row_of(g, cur, 4 * (w + 8 * m) + q) * (3 * KD) + sg * 8;
+    if (!S::kLoFar)
+      bl = g.b + 3 * before + (size_t)row_of(g, cur, 8 * w + 2 * q + (j >> 3)) * (3 * KD) +
+           2 * kMmCols + ((j & 7) ^ ((4 * w + q) & 7)) * 8;
     if (R::kSums)
-      sums = g.sums + before / 16 + (size_t)row_of(g, cur, 16 * w + j) * (KD / 16);
+      sums = g.sums + before / 8 + (size_t)row_of(g, cur, 16 * w + (lane >> 1)) * (KD / 8) +
+             (lane & 1) * 8;
     issue(0);
     if (S::kAhead > 1) issue(1);  // (128 columns: nst is even)
     // the epilogue's words of a position: assignment, exponent (written before
     // the first barrier)
     int2* info = reinterpret_cast<int2*>(const_cast<unsigned char*>(lds) + mm_lds<TY>() - kMmInfo);
-    if (threadIdx.x < kGgufMmTok) {
+    if (threadIdx.x < mm_tok(TY)) {
       const int p = cur.p0 + min((int)threadIdx.x, cur.n - 1);
       const int a = cur.shared ? p : g.perm[p];
       info[threadIdx.x] =
@@ -657,12 +730,12 @@ struct MmRun {
 // dispatcher places it on: a unit's row blocks share that XCD's L2 for its
 // token rows, as in k_experts).  A unit of n tokens runs with the column tiles
 // it needs; at most 128 registers and 80 KB of LDS, so that two workgroups
-// share a CU (see k_experts; one persistent workgroup on 128-token units
-// before: at hidden 2048, inter 512, 256 experts, 2048 tokens of Q3_K gate/up 286
-// -> 240 us and down 174 -> 143; per call of 256 / 2048 tokens Q3_K 313 / 627 -> 195 /
-// 505 us, Q4_K 375 / 743 -> 215 / 554, Q8_0 470 / 931 -> 243 / 537).  Bound by the
-// matrix units' two passes (hi and lo) and, between them, the codes' conversion and the
-// fp32 scaling of the partial sums.
+// share a CU (see k_experts; one persistent workgroup on 128-token units took 1.2
+// times as long).  At hidden 2048, inter 512, 256 experts, top 8, per call of 256 /
+// 2048 tokens: Q3_K 229 / 588 us, Q4_K 247 / 682, Q8_0 259 / 642 (with two parts of
+// 23 bits 197 / 515, 218 / 568, 245 / 549).  Bound by the matrix units' three
+// passes and, between them, the codes' conversion and the fp32 scaling of the
+// partial sums.
 template <int TY, bool GU>
 __global__ __launch_bounds__(kMmThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void k_gguf_mm(const int32_t* meta, const int2* units, const int32_t* off, const int32_t* perm,
@@ -679,12 +752,12 @@ void k_gguf_mm(const int32_t* meta, const int2* units, const int32_t* off, const
   it.shared = v.x >= g.L.E;
   it.e = it.shared ? g.L.E : v.x;
   it.p0 = it.shared ? v.y : off[v.x] + v.y;
-  it.n = min(kGgufMmTok, (it.shared ? g.T : off[v.x + 1]) - it.p0);
+  it.n = min(mm_tok(TY), (it.shared ? g.T : off[v.x + 1]) - it.p0);
   it.rows = it.shared ? g.L.Ish : g.L.I;
   if (GU && it.fb * 128 >= it.rows) return;  // uniform per workgroup
   if (it.n <= 16) MmRun<TY, GU, 1>().run(g, it, ldsm);
   else if (it.n <= 32) MmRun<TY, GU, 2>().run(g, it, ldsm);
-  else MmRun<TY, GU, 4>().run(g, it, ldsm);
+  else MmRun<TY, GU, mm_tok(TY) / 16>().run(g, it, ldsm);
 }
 
 template <int TY>
@@ -756,15 +829,17 @@ hipError_t launch_gguf_tiles(const GgufMoeDev& L, uint8_t* out, hipStream_t st) 
   return hipGetLastError();
 }
 
+int gguf_mm_tok(const GgufMoeDev& L) { return mm_tok(L.type); }
+
 bool gguf_mm_ok(const GgufMoeDev& L, const uint8_t* tiles, int T) {
-  // the kernels' row offsets are 32-bit element offsets
+  // (2^32 parts and more: not measured, the grouped form)
   const uint64_t n = L.I > L.Ish ? L.I : L.Ish;
   return tiles && T >= kGgufMmMinT && 2ull * T * L.H < (1ull << 32) &&
          2ull * T * L.K * n < (1ull << 32);
 }
 
 size_t gguf_mm_sums(const GgufMoeDev& L, int64_t elements) {
-  return L.type == kGgmlQ4_K ? (size_t)elements / 16 : 0;
+  return L.type == kGgmlQ4_K ? (size_t)elements / 8 : 0;
 }
 
 hipError_t launch_gguf_mm(const GgufMoeDev& L, const uint8_t* tiles, const float* x, int T, const int32_t* off,

@@ -1,15 +1,15 @@
 """GGUF layers with many tokens per call (from 256 on, experts in Q3_K, Q4_K
 or Q8_0 with hidden, inter and inter_sh multiples of 128): the experts'
 products on the matrix cores, integer codes in f16 against activations in
-two f16 parts.
+three f16 parts.
 
 Reference: the reference's composition on the dequantized weights in float64
 (ids and probabilities of the oracle, which must match bit for bit).  Bar: the
 relative 2-norm error of a token's output stays below 2e-6.  The parts hold
-24 bits of an activation (2^-24 each, in x and again in h), the longest chain
-of fp32 additions is 2048 / 64 matrix instructions for each of hi and lo, and
-random rounding over n additions grows as sqrt(n) 2^-24 = 8 * 6e-8 per
-product; gate, up and down together stay under 4 * 5e-7."""
+an activation exactly, the longest chain of fp32 additions is 2048 / 32
+matrix instructions for each of the three parts, and random rounding over n
+additions grows as sqrt(n) 2^-24 = 14 * 6e-8 = 8.3e-7 per product; those of
+gate, up and down are independent: sqrt(3) * 8.3e-7 = 1.5e-6."""
 import json
 
 import numpy as np
@@ -140,6 +140,93 @@ def test_rows_of_any_scale(block, oracle, tmp_path, ty):
     keep[5] = False
     assert np.array_equal(y[keep], y2[keep])
     block.free_layer_gguf(65)
+
+
+def _encode(ty, codes, d):
+    """A payload whose weight i is d[block of i] * codes[i] (fp16 d; Q3_K codes
+    -4 .. 3, Q4_K 0 .. 15 without mins, Q8_0 -127 .. 127)."""
+    bs, n = (32, 34) if ty == 8 else (256, 114 if ty == 11 else 144)
+    q = np.asarray(codes).reshape(-1, bs)
+    raw = np.zeros((q.shape[0], n), np.uint8)
+    half = np.broadcast_to(d, q.shape[0]).astype("<f2").view(np.uint8).reshape(-1, 2)
+    if ty == 8:
+        raw[:, :2], raw[:, 2:] = half, q.astype(np.int8).view(np.uint8)
+    elif ty == 11:
+        u = (q + 4).astype(np.uint8)
+        raw[:, :32] = np.packbits(u >> 2, axis=1, bitorder="little")
+        raw[:, 32:96] = ((u & 3).reshape(-1, 64, 4) << np.array([0, 2, 4, 6])).sum(2)
+        raw[:, 96:112], raw[:, 112:] = 33, half
+    else:
+        raw[:, :2], raw[:, 4:16] = half, 1
+        u = q.astype(np.uint8).reshape(-1, 8, 2, 16)
+        raw[:, 16:] = (u[:, :, 0] | u[:, :, 1] << 4).reshape(-1, 128)
+    return raw.tobytes()
+
+
+@pytest.mark.parametrize("ty", [11, 12, 8])
+def test_every_bit_of_an_activation(block, oracle, tmp_path, ty):
+    """gate = x0 + x1 where x1 is -x0 but for its last bits, up = x2: the
+    difference is exact in fp32, and the outputs keep the bar only if the last
+    bit of every activation counts."""
+    dims, T = (256, 4, 2, 128, 128), 256
+
+    def f(ts):
+        gate, up = np.zeros((128, 256), int), np.zeros((128, 256), int)
+        gate[:, :2] = 1
+        up[:, 2] = 1
+        return [(n, d, t, _encode(ty, gate if "gate" in n else up, 1.0))
+                if n.split(".")[2] in ("ffn_gate", "ffn_up", "ffn_shared_gate", "ffn_shared_up")
+                else (n, d, t, raw) for n, d, t, raw in ts]
+
+    g = _upload(block, tmp_path, 68, dims, ty, f)
+    rng = np.random.default_rng(21)
+    x = rng.standard_normal((T, 256)).astype(np.float32)
+    x[:, 0] = rng.uniform(1, 2, T).astype(np.float32)
+    x[:, 1] = -(x[:, 0].view(np.int32) + rng.integers(1, 9, T).astype(np.int32)).view(np.float32)
+    _check(block, oracle, g, 68, dims, x)
+    block.free_layer_gguf(68)
+
+
+@pytest.mark.parametrize("ty", [11, 12, 8])
+def test_values_far_below_the_rows_largest(block, oracle, tmp_path, ty):
+    """x5 is 2^26 times the others where every weight is zero, and h7 2^20
+    times the others where every down weight is: the small values alone make
+    the outputs."""
+    dims, T = (256, 4, 2, 128, 128), 256
+    lo, hi = {11: (-4, 4), 12: (0, 16), 8: (-127, 128)}[ty]
+    rng = np.random.default_rng(22)
+
+    def f(ts):
+        out = []
+        for n, dm, t, raw in ts:
+            k = n.split(".")[2]
+            if k == "shared_gate":
+                w = np.frombuffer(raw, "<f4").copy()
+                w[5] = 0
+                raw = w.tobytes()
+            elif k == "ffn_gate_exps":
+                w = np.frombuffer(raw, np.uint8).reshape(4, 8, 34).copy()
+                w[:, 0, 2 + 5] = 0
+                raw = w.tobytes()
+            elif k in ("ffn_down", "ffn_shared_down"):
+                c = rng.integers(lo, hi, (256, 128))
+                c[:, 7] = 0
+                raw = _encode(ty, c, 2.0 ** -6)
+            elif k.startswith("ffn"):
+                c = rng.integers(lo, hi, (128, 256))
+                c[:, 5] = 0
+                d = np.full((128, 256 // (32 if ty == 8 else 256)), 2.0 ** (-11 if ty == 8 else -7))
+                if "up" in k:
+                    d[7] *= 2.0 ** 20
+                raw = _encode(ty, c, d.reshape(-1))
+            out.append((n, dm, t, raw))
+        return out
+
+    g = _upload(block, tmp_path, 69, dims, ty, f)
+    x = rng.standard_normal((T, 256)).astype(np.float32)
+    x[:, 5] *= np.float32(2.0 ** 26)
+    _check(block, oracle, g, 69, dims, x)
+    block.free_layer_gguf(69)
 
 
 def test_more_tokens_than_one_launch_combines(block, oracle, tmp_path):
