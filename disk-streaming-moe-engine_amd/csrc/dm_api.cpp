@@ -118,10 +118,8 @@ struct DevBuf {
     if (e == hipSuccess) cap = n;
     return e;
   }
-  void release() {
+  ~DevBuf() {
     if (p) (void)hipFree(p);
-    p = nullptr;
-    cap = 0;
   }
 };
 
@@ -155,6 +153,7 @@ struct PinBuf {
     p = d = nullptr;
     cap = 0;
   }
+  ~PinBuf() { release(); }
 };
 
 }  // namespace
@@ -824,26 +823,6 @@ int dmh_destroy(dmh_ctx* c) {
   if (c->cur) (void)hipStreamSynchronize(c->cur);
   for (Layer* L : c->layers) free_layer(L);
   for (GgufLayer* G : c->glayers) free_glayer(G);
-  DevBuf<float>* fb[] = {&c->x, &c->res, &c->y, &c->z, &c->probs, &c->shg, &c->h, &c->xn, &c->hstack};
-  for (auto* b : fb) b->release();
-  c->ids.release();
-  c->uids.release();
-  c->io_in.release();
-  c->io_out.release();
-  c->pin.release();
-  c->pin_out.release();
-  c->stage.release();
-  c->g_off.release();
-  c->g_perm.release();
-  c->g_meta.release();
-  c->g_needlo.release();
-  c->g_units.release();
-  c->g_xhi.release();
-  c->g_xlo.release();
-  c->g_hr.release();
-  c->g_hs.release();
-  c->g_r.release();
-  c->g_rs.release();
   if (c->status) (void)hipFree(c->status);
   if (c->ones) (void)hipFree(c->ones);
   if (c->switch_ev) (void)hipEventDestroy(c->switch_ev);
@@ -851,7 +830,7 @@ int dmh_destroy(dmh_ctx* c) {
   if (c->flags) (void)hipFree(c->flags);
   if (c->own) (void)hipStreamDestroy(c->own);
   if (c->counted) g_live_ctx[c->device].fetch_sub(1);
-  delete c;
+  delete c;  // and its buffers
   return DMH_OK;
 }
 

@@ -279,3 +279,21 @@ def test_errors(block, tmp_path):
             texts.append(str(ei.value))
         assert texts[0] == texts[1] and json.loads(texts[0])["detail"] == detail
     block.free_layer_gguf(66)
+
+
+def test_closed_contexts_keep_nothing(tmp_path):
+    """A context's buffers go with it, those of the column sums (12 MB here)
+    among them."""
+    import torch
+    from dismoen import MoEBlock
+    dims, T = (2048, 2, 1, 512, 512), 16384
+    x = np.zeros((T, 2048), np.float32)
+    free = []
+    for _ in range(4):
+        b = MoEBlock(0)
+        _upload(b, tmp_path, 0, dims, 12)
+        b.forward_port_moe_gguf(x, None, 0, T)
+        b.close()
+        torch.cuda.synchronize()
+        free.append(torch.cuda.mem_get_info()[0])
+    assert free[0] - free[-1] < 8 << 20, free
