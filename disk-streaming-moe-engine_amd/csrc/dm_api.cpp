@@ -65,7 +65,6 @@ constexpr int kStatusSlots = kGgufSlot0 + kMaxLayers;
 struct GgufLayer {
   dmh_moe_dims dims{};
   void* buf = nullptr;
-  size_t bytes = 0;
   dm::GgufMoeDev dev{};
   // single-token form (dm::launch_gguf_one_token): its sync area, grid and
   // launch count (the hand-off count only grows)
@@ -74,11 +73,92 @@ struct GgufLayer {
   int grid = 0;
   unsigned launches = 0;
   float* rchain = nullptr;  // the router in chain order (dev.rchain)
-  uint8_t* tiles = nullptr; // the experts in matrix-core records, or null
+  // the experts in matrix-core records, or null; guarded by its device's
+  // RecordPool, as are the calls being queued on them and whether a graph holds
+  // their address
+  uint8_t* tiles = nullptr;
+  int device = 0, tiles_held = 0;
+  bool tiles_captured = false;
+};
+
+// The layers with matrix-core records on a device.  The records are a second
+// form of weights that a layer has anyway, so they never stand in the way of
+// an allocation: one that the device has no room for takes records back, the
+// last uploaded layer's first, whichever context they belong to, and the
+// layer's calls of many tokens run grouped from then on.  (Not where a call is
+// being queued on them or a captured graph holds their address.)
+struct RecordPool {
+  std::mutex mu;
+  std::vector<GgufLayer*> layers;
+};
+RecordPool g_records[kMaxDevices];
+
+// hipMalloc on the current device.  A request that cannot be met with all
+// records taken back takes none.
+hipError_t dev_malloc(void** p, size_t n) {
+  hipError_t e = hipMalloc(p, n);
+  int dev = 0;
+  if (e != hipErrorOutOfMemory || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
+    return e;
+  RecordPool& pool = g_records[dev];
+  std::lock_guard<std::mutex> g(pool.mu);
+  const auto idle = [](const GgufLayer* G) { return !G->tiles_held && !G->tiles_captured; };
+  size_t room = 0, total = 0;
+  if (hipMemGetInfo(&room, &total) != hipSuccess) return e;
+  for (const GgufLayer* G : pool.layers)
+    if (idle(G)) room += dm::gguf_tiles_bytes(G->dev);
+  // (queued calls may still read the records)
+  if (room < n || hipDeviceSynchronize() != hipSuccess) return e;
+  for (size_t i = pool.layers.size(); e == hipErrorOutOfMemory && i-- > 0;) {
+    GgufLayer* G = pool.layers[i];
+    if (!idle(G)) continue;
+    (void)hipFree(G->tiles);
+    G->tiles = nullptr;
+    pool.layers.erase(pool.layers.begin() + (ptrdiff_t)i);
+    (void)hipGetLastError();  // (the failed allocation is not the next launch's error)
+    e = hipMalloc(p, n);
+  }
+  return e;
+}
+template <typename T>
+hipError_t dev_malloc(T** p, size_t n) {
+  return dev_malloc(reinterpret_cast<void**>(p), n);
+}
+
+// A layer's records for the calls queued while this lives; p is null without
+// any.
+struct RecordHold {
+  GgufLayer* G;
+  uint8_t* p = nullptr;
+  explicit RecordHold(GgufLayer* layer) : G(layer) {}
+  hipError_t take(hipStream_t st) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    const hipError_t e = hipStreamIsCapturing(st, &cap);
+    if (e != hipSuccess) return e;
+    std::lock_guard<std::mutex> g(g_records[G->device].mu);
+    if (!(p = G->tiles)) return hipSuccess;
+    ++G->tiles_held;
+    if (cap != hipStreamCaptureStatusNone) G->tiles_captured = true;
+    return hipSuccess;
+  }
+  void drop() {
+    if (!p) return;
+    std::lock_guard<std::mutex> g(g_records[G->device].mu);
+    --G->tiles_held;
+    p = nullptr;
+  }
+  ~RecordHold() { drop(); }
+  RecordHold(const RecordHold&) = delete;
+  RecordHold& operator=(const RecordHold&) = delete;
 };
 
 void free_glayer(GgufLayer* G) {
   if (!G) return;
+  {
+    RecordPool& pool = g_records[G->device];
+    std::lock_guard<std::mutex> g(pool.mu);
+    pool.layers.erase(std::remove(pool.layers.begin(), pool.layers.end(), G), pool.layers.end());
+  }
   if (G->buf) (void)hipFree(G->buf);
   if (G->sync) (void)hipFree(G->sync);
   if (G->rchain) (void)hipFree(G->rchain);
@@ -114,7 +194,7 @@ struct DevBuf {
     if (p) (void)hipFree(p);
     p = nullptr;
     cap = 0;
-    hipError_t e = hipMalloc(&p, n * sizeof(T) + 256);
+    hipError_t e = dev_malloc(&p, n * sizeof(T) + 256);
     if (e == hipSuccess) cap = n;
     return e;
   }
@@ -685,39 +765,51 @@ hipError_t run_gguf_block(dmh_ctx* c, GgufLayer* G, unsigned long long* status, 
   if ((e = dm::launch_router_select(c->z.p, L.E + 1, T, L.E, L.K, 1, dids, dprobs, dshg, status,
                                     st)) != hipSuccess)
     return e;
-  if (T > 1 && L.E <= kGgufGroupMaxE && (dm::gguf_units_pay(L, T) || dm::gguf_mm_ok(L, G->tiles, T))) {
+  if (T > 1 && L.E <= kGgufGroupMaxE) {
     // several tokens: grouped by expert, each expert row read once per unit
-    const bool mm = dm::gguf_mm_ok(L, G->tiles, T);
-    const int tok = mm ? dm::gguf_mm_tok(L) : dm::gguf_unit_tokens(L, T);
-    const int nu = dm::group_units_max(T, L.K, L.E, tok);
-    if ((e = c->g_off.ensure(L.E + 1)) != hipSuccess) return e;
-    if ((e = c->g_perm.ensure((size_t)T * L.K)) != hipSuccess) return e;
-    if ((e = c->g_meta.ensure(2)) != hipSuccess) return e;
-    if ((e = c->g_units.ensure(nu)) != hipSuccess) return e;
-    if ((e = c->g_r.ensure((size_t)T * (L.K + 1) * L.H)) != hipSuccess) return e;
-    if ((e = dm::launch_group_build(dids, T, L.K, L.E, tok, c->g_off.p, c->g_perm.p, c->g_units.p,
-                                    c->g_meta.p, st)) != hipSuccess)
-      return e;
-    if (mm) {
-      // prefill: the experts' products on the matrix cores
-      const size_t TK = (size_t)T * L.K, TH = (size_t)T * L.H;
-      const size_t hn = TK * L.I + (size_t)T * L.Ish;
-      const size_t xsum = dm::gguf_mm_sums(L, (int64_t)TH);
+    RecordHold rec(G);
+    if (dm::gguf_mm_ok(L, T) && (e = rec.take(st)) != hipSuccess) return e;
+    const size_t TK = (size_t)T * L.K, TH = (size_t)T * L.H;
+    const size_t hn = TK * L.I + (size_t)T * L.Ish, xsum = dm::gguf_mm_sums(L, (int64_t)TH);
+    int tok = 0, nu = 0;
+    const auto buffers = [&]() -> hipError_t {
+      hipError_t e;
+      tok = rec.p ? dm::gguf_mm_tok(L) : dm::gguf_unit_tokens(L, T);
+      nu = dm::group_units_max(T, L.K, L.E, tok);
+      if ((e = c->g_off.ensure(L.E + 1)) != hipSuccess) return e;
+      if ((e = c->g_perm.ensure(TK)) != hipSuccess) return e;
+      if ((e = c->g_meta.ensure(2)) != hipSuccess) return e;
+      if ((e = c->g_units.ensure(nu)) != hipSuccess) return e;
+      if ((e = c->g_r.ensure((size_t)T * (L.K + 1) * L.H)) != hipSuccess) return e;
+      if (!rec.p) return hipSuccess;
       if ((e = c->g_xhi.ensure(3 * TH)) != hipSuccess) return e;
       if ((e = c->g_hr.ensure(3 * hn)) != hipSuccess) return e;
       if ((e = c->g_ex.ensure(T + TK + T)) != hipSuccess) return e;
-      if ((e = c->g_sums.ensure(xsum + dm::gguf_mm_sums(L, (int64_t)hn) + 1)) != hipSuccess)
+      return c->g_sums.ensure(xsum + dm::gguf_mm_sums(L, (int64_t)hn) + 1);
+    };
+    if (rec.p && (e = buffers()) != hipSuccess) {
+      if (e != hipErrorOutOfMemory) return e;
+      (void)hipGetLastError();
+      rec.drop();  // the grouped form needs less, and may take these records back
+    }
+    const bool mm = rec.p != nullptr;
+    if (mm || dm::gguf_units_pay(L, T)) {
+      if (!mm && (e = buffers()) != hipSuccess) return e;
+      if ((e = dm::launch_group_build(dids, T, L.K, L.E, tok, c->g_off.p, c->g_perm.p, c->g_units.p,
+                                      c->g_meta.p, st)) != hipSuccess)
         return e;
+      if (!mm)
+        return dm::launch_gguf_units(L, dx, T, c->g_off.p, c->g_perm.p, c->g_units.p, c->g_meta.p,
+                                     nu, c->h.p, ldh, c->g_r.p, dprobs, dshg, dres, dy, status, st);
+      // prefill: the experts' products on the matrix cores
       const dm::GgufMmScratch s{c->g_xhi.p,  c->g_hr.p,           c->g_ex.p,
                                 c->g_sums.p, c->g_sums.p + xsum, c->h.p};
       float* rs = c->g_r.p + TK * L.H;
-      if ((e = dm::launch_gguf_mm(L, G->tiles, dx, T, c->g_off.p, c->g_perm.p, c->g_units.p, c->g_meta.p,
-                                  nu, s, c->g_r.p, rs, status, st)) != hipSuccess)
+      if ((e = dm::launch_gguf_mm(L, rec.p, dx, T, c->g_off.p, c->g_perm.p, c->g_units.p,
+                                  c->g_meta.p, nu, s, c->g_r.p, rs, status, st)) != hipSuccess)
         return e;
       return dm::launch_combine(c->g_r.p, rs, dprobs, dshg, dres, T, L.H, L.K, dy, status, st);
     }
-    return dm::launch_gguf_units(L, dx, T, c->g_off.p, c->g_perm.p, c->g_units.p, c->g_meta.p, nu,
-                                 c->h.p, ldh, c->g_r.p, dprobs, dshg, dres, dy, status, st);
   }
   if ((e = dm::launch_gguf_gateup(L, dx, T, dids, c->h.p, ldh, status, st)) != hipSuccess) return e;
   return dm::launch_gguf_down_combine(L, c->h.p, ldh, T, dids, dprobs, dshg, dres, dy, status,
@@ -761,12 +853,12 @@ int dmh_create(int device, dmh_ctx** out, char* err, size_t errlen) {
   dmh_ctx* c = new dmh_ctx();
   c->device = device;
   hipError_t e = hipStreamCreateWithFlags(&c->own, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipMalloc(&c->status, sizeof(unsigned long long) * kStatusSlots);
-  if (e == hipSuccess) e = hipMalloc(&c->vkey, sizeof(unsigned long long));
-  if (e == hipSuccess) e = hipMalloc(&c->flags, sizeof(unsigned));
+  if (e == hipSuccess) e = dev_malloc(&c->status, sizeof(unsigned long long) * kStatusSlots);
+  if (e == hipSuccess) e = dev_malloc(&c->vkey, sizeof(unsigned long long));
+  if (e == hipSuccess) e = dev_malloc(&c->flags, sizeof(unsigned));
   if (e == hipSuccess)
     e = hipMemset(c->status, 0xFF, sizeof(unsigned long long) * kStatusSlots);
-  if (e == hipSuccess) e = hipMalloc(&c->ones, sizeof(float) * dm::kNormMaxH);
+  if (e == hipSuccess) e = dev_malloc(&c->ones, sizeof(float) * dm::kNormMaxH);
   if (e == hipSuccess) {
     const std::vector<float> one(dm::kNormMaxH, 1.0f);
     e = hipMemcpy(c->ones, one.data(), sizeof(float) * one.size(), hipMemcpyHostToDevice);
@@ -908,7 +1000,7 @@ int dmh_upload_moe_layer(dmh_ctx* c, int layer, const dmh_moe_dims* d, const dmh
   const size_t total = b_router + b_gun + b_gus + b_dn + b_ds + b_sgun + b_sgus + b_sdn + b_sds;
   Layer* Ly = new Layer();
   Ly->dims = *d;
-  hipError_t e = hipMalloc(&Ly->buf, total);
+  hipError_t e = dev_malloc(&Ly->buf, total);
   if (e != hipSuccess) {
     delete Ly;
     return set_err(err, errlen, DMH_ERR_NO_MEMORY, "dmh_upload_moe_layer: hipMalloc(%zu): %s",
@@ -1018,7 +1110,7 @@ int dmh_upload_moe_layer(dmh_ctx* c, int layer, const dmh_moe_dims* d, const dmh
     Ly->sync_bytes = dm::decode_sync_bytes(Ly->dev, Ly->plan);
     if (dm::decode_occupancy(Ly->dev, Ly->plan, &per_cu) == hipSuccess && c->num_cus > 0 &&
         per_cu * c->num_cus >= Ly->plan.grid && Ly->plan.lds_bytes <= 65536 && K + 1 <= 64 &&
-        hipMalloc(&Ly->sync, Ly->sync_bytes) == hipSuccess &&
+        dev_malloc(&Ly->sync, Ly->sync_bytes) == hipSuccess &&
         hipMemsetAsync(Ly->sync, 0, Ly->sync_bytes, st) == hipSuccess)
       Ly->fused = true;
   }
@@ -1378,7 +1470,7 @@ int dmh_set_layer_norm(dmh_ctx* c, int layer, const float* gamma, int hidden, un
     Ly->gamma = nullptr;
     return DMH_OK;
   }
-  if (!Ly->gamma) HIP_TRY(hipMalloc(&Ly->gamma, sizeof(float) * (size_t)hidden));
+  if (!Ly->gamma) HIP_TRY(dev_malloc(&Ly->gamma, sizeof(float) * (size_t)hidden));
   HIP_TRY(hipMemcpy(Ly->gamma, gamma, sizeof(float) * (size_t)hidden,
                     (flags & DMH_F_DEVICE) ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice));
   return DMH_OK;
@@ -1933,7 +2025,7 @@ static int upload_gguf_body(dmh_ctx* c, int layer, const dmh_moe_dims* d,
                b_sr = align256(sg_raw.size());
   const size_t bytes = b_router + b_sg + b_off + payload.size() + b_rr + b_sr;
   GgufLayer* G = new GgufLayer();
-  if (hipMalloc(&G->buf, bytes) != hipSuccess) {
+  if (dev_malloc(&G->buf, bytes) != hipSuccess) {
     delete G;
     return set_err(err, errlen, DMH_ERR_NO_MEMORY,
                    "dmh_upload_moe_layer_gguf: cannot allocate %zu bytes", bytes);
@@ -1963,7 +2055,6 @@ static int upload_gguf_body(dmh_ctx* c, int layer, const dmh_moe_dims* d,
     HIP_TRY(e);
   }
   G->dims = *d;
-  G->bytes = bytes;
   // routed expert tensors of one size, appended in order from offset 0:
   // their offsets are (3e + k) * stride, no table lookup needed
   int64_t estride = off.size() > 1 ? off[1] - off[0] : 0;
@@ -1976,8 +2067,8 @@ static int upload_gguf_body(dmh_ctx* c, int layer, const dmh_moe_dims* d,
     G->sync_bytes = dm::gguf_one_token_sync_bytes(G->dev);
     if (dm::gguf_one_token_supported(G->dev) && dm::gguf_one_token_grid_ok(G->dev, c->num_cus) &&
         dm::gguf_experts_occupancy(G->dev, &per_cu) == 0 && per_cu >= 1 &&
-        hipMalloc(&G->sync, G->sync_bytes) == hipSuccess) {
-      if (hipMalloc(&G->rchain, dm::gguf_chain_router_bytes(G->dev)) == hipSuccess &&
+        dev_malloc(&G->sync, G->sync_bytes) == hipSuccess) {
+      if (dev_malloc(&G->rchain, dm::gguf_chain_router_bytes(G->dev)) == hipSuccess &&
           dm::launch_chain_router(G->dev, G->rchain, st) == hipSuccess &&
           hipMemsetAsync(G->sync, 0, G->sync_bytes, st) == hipSuccess &&
           hipStreamSynchronize(st) == hipSuccess) {
@@ -1991,15 +2082,22 @@ static int upload_gguf_body(dmh_ctx* c, int layer, const dmh_moe_dims* d,
       }
     }
   }
-  // the matrix-core form of the experts; without room for it, calls of many
-  // tokens keep the grouped form on the payload
-  if (const size_t nt = dm::gguf_tiles_bytes(G->dev)) {
-    if (hipMalloc(&G->tiles, nt) != hipSuccess ||
-        dm::launch_gguf_tiles(G->dev, G->tiles, st) != hipSuccess ||
-        hipStreamSynchronize(st) != hipSuccess) {
-      if (G->tiles) (void)hipFree(G->tiles);
-      G->tiles = nullptr;
+  // the matrix-core form of the experts, unless declined; without room for
+  // it, calls of many tokens keep the grouped form on the payload
+  G->device = c->device;
+  if (const size_t nt = flags & DMH_F_NO_RECORDS ? 0 : dm::gguf_tiles_bytes(G->dev)) {
+    if ((e = hipMalloc(&G->tiles, nt)) == hipErrorOutOfMemory) {
       (void)hipGetLastError();  // (a failed allocation is not the next launch's error)
+      G->tiles = nullptr;
+    } else {
+      if (e == hipSuccess) e = dm::launch_gguf_tiles(G->dev, G->tiles, st);
+      if (e == hipSuccess) e = hipStreamSynchronize(st);
+      if (e != hipSuccess) {
+        free_glayer(G);
+        HIP_TRY(e);
+      }
+      std::lock_guard<std::mutex> g(g_records[c->device].mu);
+      g_records[c->device].layers.push_back(G);
     }
   }
   if (GgufLayer* old = c->glayers[layer]) {

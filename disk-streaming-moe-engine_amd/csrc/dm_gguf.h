@@ -90,9 +90,8 @@ hipError_t launch_gguf_tiles(const GgufMoeDev& L, uint8_t* out, hipStream_t st);
 // (Qwen3.6 shape, Q3_K 444 us at 200 tokens grouped, 229 at 256 here).
 constexpr int kGgufMmMinT = 256;
 int gguf_mm_tok(const GgufMoeDev& L);  // tokens per unit
-// tiles: the records of launch_gguf_tiles, or null.  (Not a member of GgufMoeDev:
-// eight more bytes of arguments cost the one-token launch 0.1 us.)
-bool gguf_mm_ok(const GgufMoeDev& L, const uint8_t* tiles, int T);
+// Whether T tokens of L can run on its records, when it has them.
+bool gguf_mm_ok(const GgufMoeDev& L, int T);
 // Elements of the column sums of `elements` activations (0: not needed).
 size_t gguf_mm_sums(const GgufMoeDev& L, int64_t elements);
 struct GgufMmScratch {
@@ -106,7 +105,9 @@ struct GgufMmScratch {
 // The experts' outputs of T tokens grouped by expert (off, perm, units, meta
 // of launch_group_build with tok = gguf_mm_tok, nunits = group_units_max): r [T*K][H] by
 // assignment, rs [T][H] of the shared expert, unweighted, with the checks of
-// launch_gguf_units; launch_combine forms y from them.
+// launch_gguf_units; launch_combine forms y from them.  tiles: the records of
+// launch_gguf_tiles.  (Not a member of GgufMoeDev: eight more bytes of arguments
+// cost the one-token launch 0.1 us.)
 hipError_t launch_gguf_mm(const GgufMoeDev& L, const uint8_t* tiles, const float* x, int T, const int32_t* off,
                           const int32_t* perm, const int2* units, const int32_t* meta, int nunits,
                           const GgufMmScratch& s, float* r, float* rs, unsigned long long* status,

@@ -831,10 +831,10 @@ hipError_t launch_gguf_tiles(const GgufMoeDev& L, uint8_t* out, hipStream_t st) 
 
 int gguf_mm_tok(const GgufMoeDev& L) { return mm_tok(L.type); }
 
-bool gguf_mm_ok(const GgufMoeDev& L, const uint8_t* tiles, int T) {
+bool gguf_mm_ok(const GgufMoeDev& L, int T) {
   // (2^32 parts and more: not measured, the grouped form)
   const uint64_t n = L.I > L.Ish ? L.I : L.Ish;
-  return tiles && T >= kGgufMmMinT && 2ull * T * L.H < (1ull << 32) &&
+  return gguf_tiles_bytes(L) && T >= kGgufMmMinT && 2ull * T * L.H < (1ull << 32) &&
          2ull * T * L.K * n < (1ull << 32);
 }
 
@@ -846,7 +846,7 @@ hipError_t launch_gguf_mm(const GgufMoeDev& L, const uint8_t* tiles, const float
                           const int32_t* perm, const int2* units, const int32_t* meta, int nunits,
                           const GgufMmScratch& s, float* r, float* rs, unsigned long long* status,
                           hipStream_t st) {
-  if (!gguf_mm_ok(L, tiles, T) || nunits <= 0) return hipErrorInvalidValue;
+  if (!tiles || !gguf_mm_ok(L, T) || nunits <= 0) return hipErrorInvalidValue;
   switch (L.type) {
     case kGgmlQ3_K:
       return run_mm<kGgmlQ3_K>(L, tiles, x, T, off, perm, units, meta, nunits, s, r, rs, status, st);

@@ -16,6 +16,7 @@ LIB_PATH = os.environ.get("DISMOEN_LIB") or os.path.join(PKG_ROOT, "libdismoen_h
 DMH_F_DEVICE = 0x1
 DMH_F_Q4K_PY_SCALES = 0x10
 DMH_F_NORM_TREE = 0x20
+DMH_F_NO_RECORDS = 0x40
 
 ERROR_NAMES = {
     1: "INVALID_ARG", 2: "CONFIG", 3: "HIP", 4: "NO_MEMORY", 5: "DEQUANT", 6: "ACT",

@@ -18,8 +18,8 @@ from dataclasses import dataclass, field
 
 import numpy as np
 
-from ._lib import (DMH_F_DEVICE, DMH_F_NORM_TREE, DMH_F_Q4K_PY_SCALES, DismoenError, DmhDims,
-                   DmhWeights, check, errbuf, lib)
+from ._lib import (DMH_F_DEVICE, DMH_F_NO_RECORDS, DMH_F_NORM_TREE, DMH_F_Q4K_PY_SCALES,
+                   DismoenError, DmhDims, DmhWeights, check, errbuf, lib)
 
 
 @dataclass
@@ -182,17 +182,17 @@ class MoEBlock:
 
     # -- GGUF layers (slots of their own) ---------------------------------
     def upload_layer_gguf(self, layer_idx: int, dims: tuple, index, model_layer: int = 0,
-                          py_scales: bool = False) -> None:
+                          py_scales: bool = False, records: bool = True) -> None:
         """load_port_block_from_gguf's MoE tensors of model layer model_layer
         (src/layers/gguf_port_loader.mojo:207-256) from a dismoen.gguf.GGUFIndex;
-        dims = (hidden, num_experts, top_k, inter, inter_sh)."""
+        dims = (hidden, num_experts, top_k, inter, inter_sh).  records=False: no
+        second form of the experts for calls of 256 tokens and more."""
         H, E, K, I, Ish = dims
         d = DmhDims(H, E, K, I, Ish, 32, 0)
+        flags = (DMH_F_Q4K_PY_SCALES if py_scales else 0) | (0 if records else DMH_F_NO_RECORDS)
         e = errbuf()
         check(self._lib.dmh_upload_moe_layer_gguf(self._h, layer_idx, C.byref(d), index.handle,
-                                                  model_layer,
-                                                  DMH_F_Q4K_PY_SCALES if py_scales else 0, e,
-                                                  len(e)), e)
+                                                  model_layer, flags, e, len(e)), e)
         self.gguf_dims[layer_idx] = dims
 
     def free_layer_gguf(self, layer_idx: int) -> None:

@@ -341,6 +341,9 @@ int dmh_upload_moe_layer_files(dmh_ctx* ctx, int layer, const dmh_moe_dims* dims
 /* Q4_K sub-blocks 4..7 with the scale/min packing of the reference's Python
  * twin (tools/oracle/oracle_port.py:104-110) instead of gguf.mojo:482-488. */
 #define DMH_F_Q4K_PY_SCALES 0x10u
+/* GGUF layers without the second, matrix-core form of their experts (see
+ * dmh_upload_moe_layer_gguf): for a program that only decodes. */
+#define DMH_F_NO_RECORDS 0x40u
 
 typedef struct dmh_gguf_file dmh_gguf_file;
 
@@ -412,7 +415,16 @@ int dmh_gguf_stream_tensor_f32(dmh_ctx* ctx, const dmh_gguf_file* f, const char*
  * Errors: the loader's WEIGHT_LOAD_FAILED / GGUF_READ_ERROR /
  * GGUF_UNSUPPORTED_DTYPE / "GGUF_FILE_CORRUPT: dimension mismatch" texts in
  * its order.  dims: hidden, inter, inter_sh multiples of 4; group_size is
- * ignored.  flags: DMH_F_Q4K_PY_SCALES. */
+ * ignored.  flags: DMH_F_Q4K_PY_SCALES, DMH_F_NO_RECORDS.
+ *
+ * Experts in Q3_K, Q4_K or Q8_0 whose hidden, inter and inter_sh are
+ * multiples of 128 are also kept in matrix-core records, which calls of 256
+ * tokens and more read: 0.69, 0.75 and 1.13 bytes per weight beside the
+ * payload's 0.45, 0.56 and 1.06.  DMH_F_NO_RECORDS declines them.  An upload
+ * without room for the records succeeds without them, and any later
+ * allocation of the library that finds no room takes records back (none
+ * that a captured graph uses); the layer's calls then run as below 256
+ * tokens. */
 int dmh_upload_moe_layer_gguf(dmh_ctx* ctx, int layer, const dmh_moe_dims* dims,
                               const dmh_gguf_file* f, int model_layer, unsigned flags, char* err,
                               size_t errlen);
@@ -423,7 +435,9 @@ int dmh_free_layer_gguf(dmh_ctx* ctx, int layer);
  * RMSNorm output [seq_len][H], residual (x_mid, may be NULL) is added last;
  * ids / probs [seq_len][K] and shg [seq_len] may be NULL.  Router, top-k,
  * shared gate and aggregation are bit-exact with the reference's fp32
- * order; the experts accumulate in fp32 in another order.  Expert error
+ * order; the experts accumulate in fp32 in another order: one for all calls
+ * of fewer than 256 tokens (a token's outputs are the same bits however it
+ * is batched), another from 256 on where the layer has its records.  Expert error
  * texts carry hidden as "layer" and the intermediate size as "expert_id", as
  * forward_port_block's swiglu_forward calls do (port_scheduler.mojo:450-464).
  * DMH_F_DEVICE: x, residual and y 16-byte aligned device memory. */

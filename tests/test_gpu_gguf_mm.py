@@ -297,3 +297,75 @@ def test_closed_contexts_keep_nothing(tmp_path):
         torch.cuda.synchronize()
         free.append(torch.cuda.mem_get_info()[0])
     assert free[0] - free[-1] < 8 << 20, free
+
+
+def _both_forms(block, slot, x):
+    """Outputs of one call, and of calls below the matrix-core form."""
+    T = x.shape[0]
+    y = block.forward_port_moe_gguf(x, None, slot, T)[0]
+    z = np.concatenate([block.forward_port_moe_gguf(x[i:i + 128], None, slot, x[i:i + 128].shape[0])[0]
+                        for i in range(0, T, 128)])
+    return y, z
+
+
+def test_records_declined(block, tmp_path):
+    dims = (256, 8, 2, 128, 128)
+    p = str(tmp_path / "l.gguf")
+    gguf.write_gguf(p, synth.make_gguf_moe_layer(256, 8, 128, 128, seed=70, expert_type=11))
+    x = np.random.default_rng(3).standard_normal((300, 256)).astype(np.float32)
+    with gguf.parse_gguf_index(p) as g:
+        for records in (True, False):
+            block.upload_layer_gguf(70, dims, g, records=records)
+            y, z = _both_forms(block, 70, x)
+            assert np.array_equal(y, z) != records
+    block.free_layer_gguf(70)
+
+
+def test_records_make_room(block, tmp_path):
+    """With the device's memory all but full, an upload takes the records of
+    another layer, not those a captured graph uses; that layer's calls run in
+    the form of fewer tokens, and the graph's replays are right."""
+    import torch
+    dims, T = (2048, 32, 2, 512, 512), 256
+    p = str(tmp_path / "l.gguf")
+    gguf.write_gguf(p, synth.make_gguf_moe_layer(2048, 32, 512, 512, seed=71, expert_type=11))
+    x = np.random.default_rng(4).standard_normal((T, 2048)).astype(np.float32)
+    xd = torch.from_numpy(x).cuda()
+    yd = torch.zeros_like(xd)
+    fill, s, graph = [], torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with gguf.parse_gguf_index(p) as g:
+        for slot in (71, 72):
+            block.upload_layer_gguf(slot, dims, g)
+            y, z = _both_forms(block, slot, x)
+            assert not np.array_equal(y, z)
+        block.forward_gguf_device(72, xd.data_ptr(), T, yd.data_ptr())  # (its buffers)
+        torch.cuda.synchronize()
+        block.set_stream(s.cuda_stream)
+        try:
+            with torch.cuda.graph(graph, stream=s):
+                block.forward_gguf_device(72, xd.data_ptr(), T, yd.data_ptr())
+        finally:
+            block.set_stream(None)
+        block.sync()
+        try:
+            left = 24 << 20  # a payload is 47 MB, its records 71 MB
+            while (free := torch.cuda.mem_get_info()[0]) > left + (8 << 20) and len(fill) < 40:
+                fill.append(torch.empty(min(free - left, 32 << 30), dtype=torch.uint8, device="cuda"))
+            print("free", free >> 20, "MB", flush=True)
+            block.upload_layer_gguf(73, dims, g)
+        finally:
+            fill.clear()
+            torch.cuda.empty_cache()
+    for slot in (71, 73):  # taken back; not made
+        y1, z1 = _both_forms(block, slot, x)
+        assert np.array_equal(y1, z) and np.array_equal(z1, z), slot
+    for _ in range(3):
+        yd.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(yd.cpu().numpy(), y)
+        assert np.array_equal(_both_forms(block, 72, x)[0], y)
+    del graph
+    for slot in (71, 72, 73):
+        block.free_layer_gguf(slot)
