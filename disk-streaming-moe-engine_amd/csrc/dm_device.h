@@ -316,18 +316,18 @@ __device__ __forceinline__ float seq_sum_squares(const float* sq, int n) {
 
 // The same sum on one wave, every lane holding per <= kSeqPerLane of the
 // squares in registers: lane l the elements l*per .. l*per + per - 1, read
-// from sqT[i * pitch + l] = element l*per + i.  Round l adds every lane's
+// from sqT[i * 64 + l] = element l*per + i.  Round l adds every lane's
 // values to the running sum; lane l's total is then the sum through its
 // last element and is broadcast to all lanes for round l + 1.  The adds are
 // the same dependent chain in the same order, without LDS reads on it:
 // 2048 squares in about 4.2 us on MI355X against 6.5-7.2 us for the LDS
 // loop (one chain of plain register adds: 3.8-4.7 us).
 constexpr int kSeqPerLane = 32;
-__device__ __forceinline__ float seq_sum_wave_rounds(const float* sqT, int per, int pitch = 64) {
+__device__ __forceinline__ float seq_sum_wave_rounds(const float* sqT, int per) {
   const int lane = threadIdx.x & 63;
   float r[kSeqPerLane];
 #pragma unroll
-  for (int i = 0; i < kSeqPerLane; ++i) r[i] = i < per ? sqT[i * pitch + lane] : 0.0f;
+  for (int i = 0; i < kSeqPerLane; ++i) r[i] = i < per ? sqT[i * 64 + lane] : 0.0f;
   float a = 0.0f;
   if (per == kSeqPerLane) {
     for (int l = 0; l < 64; ++l) {

@@ -1153,34 +1153,69 @@ hipError_t launch_down_dec(const LayerDev& L, const float* h, int ldh, const int
 // ===========================================================================
 // RMSNorm per token (src/layers/rmsnorm.mojo:41-48): out = x / denom *
 // gamma, denom = sqrt(sum(x * x) / H + eps), for the block-edge norm of
-// several tokens.  SEQ: the squares added in element order, the reference's:
-// a chain of H dependent adds, which bounds the kernel.  2048 elements run on
-// one wave in rounds (seq_sum_wave_rounds; rows of the staged squares padded
-// by one word, so that writing along and reading across them both use every
-// bank: 1533 tokens 33 -> 26 us, calls of 8 tokens 3 us less), other sizes on
-// one thread (with 640 elements the rounds' steps past a lane's ten took 5 us
-// more).  Otherwise 256 strided partials and a halving tree (the order of the
-// fused decode kernel's tree mode).
+// several tokens.  H % 128 == 0.  SEQ: the squares added in element order, the
+// reference's: a chain of H dependent adds, which bounds the kernel.  From
+// kRoundsMinH elements on it runs on one wave in rounds over segments of 2048
+// (norm_rounds), the last one of what remains; shorter rows on one thread, since
+// a round costs about 29 cycles beside its adds (4 cycles each, 8 on one thread).
+// Otherwise 256 strided partials and a halving tree (the order of the fused
+// decode kernel's tree mode).
+//
+// Whole calls of 4 / 300 tokens, 16 experts, one thread against rounds (us): 384
+// elements 24.4 / 40.0 against 24.6 / 39.6, 512 25.9 / 41.5 against 25.7 / 41.0,
+// 1024 31.1 / 53.5 against 30.2 / 52.1, 1920 41.4 / 79.8 against 38.9 / 76.8, 4096
+// 64.5 / 132.5 against 58.8 / 124.5; calls of 1533 tokens, bound by the rows a
+// CU holds, within 1 %.
 // ===========================================================================
+constexpr int kRoundsMinH = 512, kRoundsSeg = 2048;
+// A segment's square k (of 64 per) lies at (k % per) * 65 + k / per: writing
+// along and reading across such rows both use every bank.
+constexpr int kRoundsPitch = 65;
+// The chain a + .. over a segment of 64 PER squares: lane l holds the squares
+// l PER .. l PER + PER - 1, round l adds every lane's values to the running
+// sum, and lane l's total is broadcast for the next (as seq_sum_wave_rounds,
+// which runs 32 steps whatever a lane holds).
+template <int PER>
+__device__ __forceinline__ float norm_rounds(const float* sq, int per, float a) {
+  if constexpr (PER == 0) {
+    return a;
+  } else {
+    if (per != PER) return norm_rounds<PER - 2>(sq, per, a);  // uniform
+    float r[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) r[i] = sq[i * kRoundsPitch + (threadIdx.x & 63)];
+    for (int l = 0; l < 64; ++l) {
+#pragma unroll
+      for (int i = 0; i < PER; ++i) a = a + r[i];
+      a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(a), l));
+    }
+    return a;
+  }
+}
 template <bool SEQ>
 __global__ __launch_bounds__(256) void k_rmsnorm_rows(const float* __restrict__ x, int H,
                                                        float eps, const float* __restrict__ gamma,
                                                        float* __restrict__ out) {
-  __shared__ __attribute__((aligned(16))) float part[SEQ ? kNormMaxH : 256];
+  extern __shared__ __attribute__((aligned(16))) float part[];
   const int t = blockIdx.x;
   const float* xr = x + (size_t)t * H;
   if (SEQ) {
-    static_assert(kSeqPerLane * 65 <= kNormMaxH, "padded rows");
-    const bool rounds = H == 64 * kSeqPerLane;
-    for (int i = threadIdx.x; i < H; i += 256)
-      part[rounds ? (i % kSeqPerLane) * 65 + i / kSeqPerLane : i] = xr[i] * xr[i];
+    const bool rounds = H >= kRoundsMinH;
+    const int full = H / kRoundsSeg, last = H % kRoundsSeg / 64;
+    for (int i = threadIdx.x; i < H; i += 256) {
+      const int g = i / kRoundsSeg, k = i % kRoundsSeg, per = g < full ? kRoundsSeg / 64 : last;
+      part[rounds ? g * (kRoundsSeg / 64 * kRoundsPitch) + k % per * kRoundsPitch + k / per : i] =
+          xr[i] * xr[i];
+    }
     __syncthreads();
     float a = 0.0f;
-    if (rounds) {
-      if (threadIdx.x < 64) a = seq_sum_wave_rounds(part, kSeqPerLane, 65);
-    } else if (threadIdx.x == 0) {
-      a = seq_sum_squares(part, H & ~31);
-      for (int i = H & ~31; i < H; ++i) a = a + part[i];
+    if (!rounds) {
+      if (threadIdx.x == 0) a = seq_sum_squares(part, H);
+    } else if (threadIdx.x < 64) {
+      const float* sq = part;
+      for (int g = 0; g < full; ++g, sq += kRoundsSeg / 64 * kRoundsPitch)
+        a = norm_rounds<kRoundsSeg / 64>(sq, kRoundsSeg / 64, a);
+      a = norm_rounds<kRoundsSeg / 64 - 2>(sq, last, a);
     }
     __syncthreads();
     if (threadIdx.x == 0) part[0] = a;
@@ -1201,12 +1236,14 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows(const float* __restrict__ 
 
 hipError_t launch_rmsnorm_rows(const float* x, int T, int H, const NormSpec& nm, float* out,
                                hipStream_t st) {
-  if (H <= 0 || H > kNormMaxH || !nm.gamma) return hipErrorInvalidValue;
+  if (H <= 0 || H % 128 || H > kNormMaxH || !nm.gamma) return hipErrorInvalidValue;
+  const int words = !nm.seq ? 256 : H >= kRoundsMinH ? H / 64 * kRoundsPitch : H;
+  const size_t lds = (size_t)words * sizeof(float);
   if (nm.seq)
-    hipLaunchKernelGGL(k_rmsnorm_rows<true>, dim3(T), dim3(256), 0, st, x, H, nm.eps, nm.gamma,
+    hipLaunchKernelGGL(k_rmsnorm_rows<true>, dim3(T), dim3(256), lds, st, x, H, nm.eps, nm.gamma,
                        out);
   else
-    hipLaunchKernelGGL(k_rmsnorm_rows<false>, dim3(T), dim3(256), 0, st, x, H, nm.eps, nm.gamma,
+    hipLaunchKernelGGL(k_rmsnorm_rows<false>, dim3(T), dim3(256), lds, st, x, H, nm.eps, nm.gamma,
                        out);
   return hipGetLastError();
 }

@@ -71,6 +71,21 @@ def test_port_moe_with_norm_qwen_vs_oracle(block, oracle, tree):
     block.free_layer(71)
 
 
+@pytest.mark.parametrize("H", [128, 384, 512, 640, 1024, 1920, 2048, 2176, 4096, 4608, 8192])
+def test_norm_of_several_tokens_at_hidden_sizes_vs_oracle(block, oracle, H):
+    """The element-order sum on one thread (below 512 elements), in rounds of
+    what a lane holds, and over several segments with and without a
+    remainder: probabilities and shared gates bit-exact, so every normed value
+    is."""
+    rng = np.random.default_rng(715 + H)
+    L = synth.make_layer(H, 16, 2, 128, 128, seed=H)
+    block.upload_layer(74, L)
+    g = _gamma(rng, H)
+    block.set_layer_norm(74, g)
+    _port_check(block, oracle, L, 74, _residual_stream(rng, (12, H)), g, 1e-6, False)
+    block.free_layer(74)
+
+
 def test_norm_errors_match_reference(block, oracle):
     L = synth.make_layer(**synth.CONFIG_TOY, seed=72)
     block.upload_layer(72, L)
