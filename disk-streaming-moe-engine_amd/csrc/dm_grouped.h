@@ -7,10 +7,6 @@
 
 namespace dm {
 
-// Workgroups of a persistent launch with one workgroup per CU: the device's
-// CU count rounded down to a multiple of 8 (0 when it cannot be read).
-int persistent_wgs();
-
 // Upper bound of the work units of up to tok tokens (size of the units buffer).
 int group_units_max(int T, int K, int E, int tok);
 

@@ -870,19 +870,6 @@ static hipError_t ex_attrs() {
   return e;
 }
 
-int persistent_wgs() {
-  static std::atomic<int> cus[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  int n = cus[dev].load();
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    n &= ~7;
-    cus[dev].store(n);
-  }
-  return n;
-}
-
 // ---------------------------------------------------------------------------
 // Calls of at most kSmallMaxT tokens: units of up to 16, one column tile.
 // Their few workgroups are bound by the latency of their stages, so waves are

@@ -7,8 +7,9 @@
 // src/quant/dequant_kernel.mojo:22-155.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+
 #include "dm_device.h"
-#include "dm_grouped.h"
 #include "dm_kernels.h"
 
 namespace dm {
@@ -717,10 +718,11 @@ hipError_t launch_router_dec(const LayerDev& L, const float* x, int T, float* z,
 // chain): the last column of workgroups with NW = 4, the first four waves of
 // the first column with NW = 8.  A wave's 512 matrix instructions take about
 // 7 us, the staging as much again, and a workgroup's 66 KB of LDS leave room
-// for two on a CU: NW = 4 while every workgroup has a CU of its own (131
-// tokens: 23 us, 25 with the gate inside), NW = 8 beyond (2048 tokens, 256
-// experts: 256 workgroups in one round, 46 -> 34 us; with the gate's
-// workgroups apart 51).  SPLIT, for few tokens: 16 experts per workgroup, wave g
+// for two on a CU: NW = 4 while every workgroup, the gate's too, has a CU of
+// its own (131 tokens: 23 us, 25 with the gate inside), NW = 8 beyond (2048
+// tokens, 256 experts: 256 workgroups in one round, 46 -> 34 us; with the gate's
+// workgroups apart 51; whole calls of 1024 tokens, where NW = 4 is 320
+// workgroups, 137 us against 131).  SPLIT, for few tokens: 16 experts per workgroup, wave g
 // running their chains 4g .. 4g + 3 (a quarter of the matrix instructions, and all
 // its router words requested before the staging), the chains then joined
 // through LDS in the halving tree's order; while every workgroup has a CU of its
@@ -927,18 +929,31 @@ __global__ __launch_bounds__(64 * NW) void k_router_mfma(const uint16_t* __restr
   }
 }
 
+// The device's CU count (0 when it cannot be read).
+static int device_cus() {
+  static std::atomic<int> cus[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  int n = cus[dev].load();
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    cus[dev].store(n);
+  }
+  return n;
+}
+
 hipError_t launch_router_mfma(const LayerDev& L, const uint16_t* xhi, const int* need_lo, int T,
                               float* z, hipStream_t st) {
   // the staged activations, then (SPLIT) the 16 KB of the chains' sums
   size_t lds = (size_t)16 * (16 * (L.H / 16) + 8) * sizeof(uint16_t);
   if (lds < 16384) lds = 16384;
-  const int tiles = (T + 15) / 16, cus = persistent_wgs();
+  const int tiles = (T + 15) / 16, cus = device_cus();
 #define DM_ROUTER_MFMA(NW, SPLIT, COLS)                                                          \
   hipLaunchKernelGGL((k_router_mfma<NW, SPLIT>), dim3(COLS, tiles), dim3(64 * NW), lds, st, xhi, \
                      need_lo, L.router, L.H, L.E, T, L, z)
   if (tiles * ((L.E + 15) / 16 + 1) <= cus)
     DM_ROUTER_MFMA(4, true, (L.E + 15) / 16 + 1);
-  else if (tiles * ((L.E + 63) / 64) <= cus)
+  else if (tiles * ((L.E + 63) / 64 + 1) <= cus)
     DM_ROUTER_MFMA(4, false, (L.E + 63) / 64 + 1);
   else
     DM_ROUTER_MFMA(8, false, (L.E + 127) / 128);
