@@ -661,15 +661,19 @@ hipError_t launch_router_dec(const LayerDev& L, const float* x, int T, float* z,
   const int blocks = (L.E + 1 + 15) / 16;
   const int nj8 = L.H % 128 == 0 ? L.H / 128 : 0;
   if (T >= 2 * kRdTok && (nj8 == 2 || nj8 == 4 || nj8 == 8 || nj8 == 16)) {
-    // From 512 tokens on two rows per lane: an LDS read then serves 16
-    // products instead of 8 (LDS reads took 0.9 of the time the products do)
-    // and the next pass's activations are requested ahead; at most 512
-    // workgroups (two per CU at their 220 registers), so one round.  1533
-    // tokens: 79 -> 70 us.  Below, one row (1024 workgroups).  Tokens per
-    // workgroup: a multiple of kRdTok.
-    const bool two = T >= 512;
+    // Many logits: two rows per lane.  An LDS read then serves 16 products
+    // instead of 8 (LDS reads took 0.9 of the time the products do) and the
+    // next pass's activations are requested ahead; in one round of workgroups,
+    // two per CU at hidden 2048 and 1024 (255 and 152 registers), four below (104
+    // and 79).  1533 tokens of 256 experts, hidden 2048: 79 -> 70 us.  Fewer
+    // logits leave too few such workgroups (whole calls, one row against two, us:
+    // hidden 2048, 40 experts, 1088 tokens 103 / 109; 1024, 128 experts, 832
+    // tokens 72 / 76; 2048, 256 experts, 1024 tokens 173 / 169): one row, 1024
+    // workgroups.  Tokens per workgroup: a multiple of kRdTok.
+    const bool two = (int64_t)T * (L.E + 1) >= 512 * 256;
     const int bl = two ? (L.E + 1 + 31) / 32 : blocks;
-    const int want = two ? (512 >= bl ? 512 / bl : 1) : (1024 + bl - 1) / bl;
+    const int wgs = nj8 >= 8 ? 512 : 1024;
+    const int want = two ? (wgs >= bl ? wgs / bl : 1) : (1024 + bl - 1) / bl;
     int tpw = (T + want - 1) / want;
     tpw = ((tpw + kRdTok - 1) / kRdTok) * kRdTok;
     const int ty = (T + tpw - 1) / tpw;

@@ -3,7 +3,7 @@ probabilities of every token, shared gates of a sample, bit-exact against the
 oracle.  256 CUs: the matrix-core router splits an expert group's chains over
 four waves while tiles (of 16 tokens) x (ceil(E / 16) + 1) workgroups fit them,
 takes four waves of 16 experts while tiles x (ceil(E / 64) + 1) do, and eight
-beyond."""
+beyond; the lane-chain router holds two rows per lane from 131072 logits on."""
 import numpy as np
 import pytest
 
@@ -42,3 +42,13 @@ def test_matrix_core_router(block, oracle, H, E, T):
     x = synth.make_activations(np.random.default_rng(T), (T, H))
     _check(block, oracle, 75, H, E, 4, x)
 
+
+@pytest.mark.parametrize("H", [256, 512, 1024, 2048])
+@pytest.mark.parametrize("E,T", [
+    (200, 652),     # one row, the last size
+    (200, 661),     # two rows; the last block's second rows past row E; a ragged last pass
+    (33, 4001),     # two rows, one live wave in the last block
+])
+def test_lane_chain_router(block, oracle, H, E, T):
+    x = np.random.default_rng(T).standard_normal((T, H)).astype(np.float32)
+    _check(block, oracle, 76, H, E, 4, x)
