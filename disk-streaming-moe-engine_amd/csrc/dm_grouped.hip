@@ -1040,7 +1040,11 @@ hipError_t launch_experts_grouped(const LayerDev& L, const uint16_t* xhi, const 
       (size_t)T * L.H >= (1ull << 32))
     return hipErrorInvalidValue;
   if (T <= kSmallMaxT) {
-    const int nu = group_units_max(T, L.K, L.E, kUnitSmall);
+    // (workgroups go to the XCDs in rotation: with a multiple of 8 units a row of
+    // the grid, all blocks of a unit would run on one XCD; 24 tokens, 32 experts,
+    // hidden 4096: 97 -> 93 us per call.  The two more end at once)
+    int nu = group_units_max(T, L.K, L.E, kUnitSmall);
+    if (nu % 8 == 0) nu += 2;
     const int gy = ((L.I > L.Ish ? L.I : L.Ish) + kSmallGuCols - 1) / kSmallGuCols;
     const int dy = (L.H + kSmallDnRows - 1) / kSmallDnRows;
     hipLaunchKernelGGL(k_gu_small, dim3(nu, gy), dim3(kGThreads), 0, st, meta, units, off, perm, g);
