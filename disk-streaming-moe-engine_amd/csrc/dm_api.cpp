@@ -521,7 +521,10 @@ hipError_t ctx_scratch(dmh_ctx* ctx, const LayerDev& L, int T, bool norm, BlockS
   if (ctx->g_needlo.cap != nl_cap &&
       (e = hipMemsetAsync(ctx->g_needlo.p, 0, kFlagInts * sizeof(int), ctx->cur)) != hipSuccess)
     return e;
-  if ((e = ctx->g_units.ensure(dm::group_units_max(T, L.K, L.E, dm::unit_tok(T)))) != hipSuccess) return e;
+  // (for the smallest units, so that a call leaves room for all shorter ones,
+  // which may then be captured)
+  if ((e = ctx->g_units.ensure(dm::group_units_max(T, L.K, L.E, dm::kUnitSmall))) != hipSuccess)
+    return e;
   if ((e = ctx->g_xhi.ensure(TH)) != hipSuccess) return e;
   if ((e = ctx->g_xlo.ensure(TH)) != hipSuccess) return e;
   if ((e = ctx->g_hr.ensure(2 * TK * L.I)) != hipSuccess) return e;
@@ -779,7 +782,9 @@ hipError_t run_gguf_block(dmh_ctx* c, GgufLayer* G, unsigned long long* status, 
       if ((e = c->g_off.ensure(L.E + 1)) != hipSuccess) return e;
       if ((e = c->g_perm.ensure(TK)) != hipSuccess) return e;
       if ((e = c->g_meta.ensure(2)) != hipSuccess) return e;
-      if ((e = c->g_units.ensure(nu)) != hipSuccess) return e;
+      // (for the smallest units: see ctx_scratch)
+      if ((e = c->g_units.ensure(dm::group_units_max(T, L.K, L.E, dm::kGgufUnitLeast))) != hipSuccess)
+        return e;
       if ((e = c->g_r.ensure((size_t)T * (L.K + 1) * L.H)) != hipSuccess) return e;
       if (!rec.p) return hipSuccess;
       if ((e = c->g_xhi.ensure(3 * TH)) != hipSuccess) return e;

@@ -61,7 +61,8 @@ hipError_t launch_gguf_down_combine(const GgufMoeDev& L, const float* h, int ldh
 // Whether T tokens of L run faster grouped (launch_gguf_units) than token by
 // token (launch_gguf_gateup, launch_gguf_down_combine).
 bool gguf_units_pay(const GgufMoeDev& L, int T);
-// Tokens per unit of launch_gguf_units.
+// Tokens per unit of launch_gguf_units, at least kGgufUnitLeast.
+constexpr int kGgufUnitLeast = 4;
 int gguf_unit_tokens(const GgufMoeDev& L, int T);
 // The same outputs for T tokens grouped by expert (off, perm, units, meta
 // of launch_group_build on ids with tok = gguf_unit_tokens; nunits =

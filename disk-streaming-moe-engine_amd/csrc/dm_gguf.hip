@@ -1765,7 +1765,7 @@ bool gguf_units_pay(const GgufMoeDev& L, int T) {
 // Eight once the experts hold four or more each; four before, so that more
 // workgroups share a CU.
 int gguf_unit_tokens(const GgufMoeDev& L, int T) {
-  return (int64_t)T * L.K > 4 * (int64_t)L.E ? 8 : 4;
+  return (int64_t)T * L.K > 4 * (int64_t)L.E ? 8 : kGgufUnitLeast;
 }
 
 hipError_t launch_gguf_units(const GgufMoeDev& L, const float* x, int T, const int32_t* off,
