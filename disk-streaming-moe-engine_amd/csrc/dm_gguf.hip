@@ -1747,18 +1747,25 @@ static bool gguf_blk_down(const GgufMoeDev& L) {  // as launch_gguf_down_combine
 // what it saves grows with the row chunks (a row's share of one wave pass: 1024
 // weights of a gate or up row, 512 of a down row) that the token-by-token form
 // decodes again for every token, and with the cost of a type's decode there.
-// Measured over 2 .. 200 tokens at hidden / inter 2048 / 512, 1024 / 256 and
-// 256 / 128 (us per call, token by token against grouped, 2048 / 512: Q4_K 59 /
-// 46 at 2 tokens, 470 / 136 at 24, 2826 / 330 at 128; Q3_K 46 / 48 at 4, 74 / 66
-// at 8, 177 / 121 at 24; Q8_0 53 / 45 at 3, 319 / 163 at 24; 256 / 128: Q4_K 29 /
-// 30 at 12, Q3_K 37 / 36 at 48, Q8_0 30 / 31 at 32; 1280 / 128, Q8_0 at 10 tokens:
-// 37 / 40), the limits lie where the grouped form was the faster in all of them.
+// Measured over 2 .. 64 tokens of 9 shapes (hidden 256 .. 2048, inter 128 .. 512,
+// top 1 .. 8) and every type, both forms (us per call, token by token / grouped, on
+// either side of a type's line, hidden / inter / top):
+//   Q4_K   56000  1280 / 128 / 8: 32.8 / 34.9 at 3 tokens, 38.1 / 37.2 at 4
+//   Q8_0  120000  1280 / 128 / 8: 36.4 / 38.2 at 6 tokens, 44.1 / 40.1 at 8
+//   F32   120000  the same shape: 38.5 / 41.0 at 6 tokens, 46.2 / 42.4 at 8
+//   BF16  135000  640 / 256 / 4: 36.9 / 38.3 at 20 tokens, 41.4 / 38.8 at 24
+//   Q3_K  200000  640 / 256 / 4: 51.8 / 52.9 at 32 tokens, 69.3 / 62.5 at 48
+// From these lines on the grouped form was the faster one at every point; below,
+// other shapes would gain from it earlier (768 / 384 / 2 from 12 tokens of Q8_0).
 // Shapes without the blocked kernels: from 128 tokens.
 bool gguf_units_pay(const GgufMoeDev& L, int T) {
   if (!gguf_blk_gateup(L) || !gguf_blk_down(L)) return T >= 128;
   const int64_t gu = 2 * ((int64_t)L.K * L.I + L.Ish) * ((L.H + 1023) / 1024);
   const int64_t dn = (int64_t)L.H * ((int64_t)L.K * ((L.I + 511) / 512) + (L.Ish + 511) / 512);
-  const int64_t least = L.type == kGgmlQ4_K ? 56000 : L.type == kGgmlQ3_K ? 200000 : 120000;
+  const int64_t least = L.type == kGgmlQ4_K   ? 56000
+                        : L.type == kGgmlQ3_K ? 200000
+                        : L.type == kGgmlBF16 ? 135000
+                                              : 120000;
   return T * (gu + dn) >= least;
 }
 
