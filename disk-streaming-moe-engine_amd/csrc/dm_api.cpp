@@ -726,10 +726,7 @@ GgufLayer* get_glayer(dmh_ctx* c, int layer) {
 // and combine launches (dm::launch_gguf_units; from kGgufMmMinT tokens on
 // dm::launch_gguf_mm on layers with matrix-core records), below it gate/up of
 // every (token, slot) and the down projections with moe_aggregate_forward.
-// The grouped forms take at most 4096 experts (the grouping's LDS holds two
-// ints per expert).
-constexpr int kGgufGroupMaxE = 4096;
-
+// (The grouping's LDS holds two ints per expert; uploads take up to 2048.)
 hipError_t run_gguf_block(dmh_ctx* c, GgufLayer* G, unsigned long long* status, const float* dx,
                           const float* dres, int T, float* dy, int32_t* dids, float* dprobs,
                           float* dshg, bool allow_one = true) {
@@ -768,7 +765,7 @@ hipError_t run_gguf_block(dmh_ctx* c, GgufLayer* G, unsigned long long* status, 
   if ((e = dm::launch_router_select(c->z.p, L.E + 1, T, L.E, L.K, 1, dids, dprobs, dshg, status,
                                     st)) != hipSuccess)
     return e;
-  if (T > 1 && L.E <= kGgufGroupMaxE) {
+  if (T > 1) {
     // several tokens: grouped by expert, each expert row read once per unit
     RecordHold rec(G);
     if (dm::gguf_mm_ok(L, T) && (e = rec.take(st)) != hipSuccess) return e;

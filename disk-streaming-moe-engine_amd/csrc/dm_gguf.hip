@@ -823,7 +823,7 @@ __device__ __forceinline__ void gu_rows(const GgufMoeDev& L, const uint8_t* wg, 
   }
 }
 
-// Workgroup (rb, u): 8 rpw rows of unit u0 + u.  Sixteen weights per lane
+// Workgroup (rb, u): 4 rpw rows of unit u0 + u.  Sixteen weights per lane
 // (gu_dot16), H <= 64 * 16 * kGgufBlkCh.
 template <int T, int TM>
 __global__ __launch_bounds__(kGgufBlkThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_gguf_gateup_units_blk(

@@ -79,9 +79,9 @@ def _check(block, oracle, g, slot, dims, x):
 
 @pytest.mark.parametrize("ty", [11, 12, 8])
 @pytest.mark.parametrize("slot,dims,T", [
-    (60, (128, 2, 1, 128, 128), 256),     # two stages a product; full 128-token units
+    (60, (128, 2, 1, 128, 128), 256),     # two stages a product; several full units of an expert
     (61, (640, 9, 3, 384, 128), 257),     # rows of broken 256-weight blocks; partial row blocks
-    (62, (256, 70, 5, 256, 384), 300),    # units of about 21 tokens: one or two small ones
+    (62, (256, 70, 5, 256, 384), 300),    # units of about 21 tokens: two column tiles
     (63, (2048, 16, 8, 512, 512), 333),   # the Qwen3.6 shape
 ])
 def test_against_float64(block, oracle, tmp_path, ty, slot, dims, T):
@@ -93,27 +93,30 @@ def test_against_float64(block, oracle, tmp_path, ty, slot, dims, T):
     block.free_layer_gguf(slot)
 
 
-def test_unit_sizes(block, oracle, tmp_path):
-    """Experts with 1, 15, 16, 17, 32, 33, 48, 65, 81, 97 and 128 + 1 tokens:
-    every number of column tiles and both sides of the small units."""
-    dims = (256, 11, 1, 128, 128)
-    sizes = [1, 15, 16, 17, 32, 33, 48, 65, 81, 97, 129]
+@pytest.mark.parametrize("ty", [11, 12, 8])
+def test_unit_sizes(block, oracle, tmp_path, ty):
+    """Experts with 1 to 129 tokens: every number of column tiles (one to three
+    and units of 48 for Q8_0, one, two and four and units of 64 else) and the
+    sizes on either side of each."""
+    sizes = [1, 15, 16, 17, 32, 33, 47, 48, 49, 63, 64, 65, 81, 97, 129]
+    n = len(sizes)
+    dims = (256, n, 1, 128, 128)
 
     def route(ts):  # expert e's logit is x[e]
-        blocks = np.zeros((11, 8, 34), np.uint8)
+        blocks = np.zeros((n, 8, 34), np.uint8)
         blocks[:, :, 0:2] = np.array([1.0], np.float16).view(np.uint8)
-        for e in range(11):
+        for e in range(n):
             blocks[e, 0, 2 + e] = 1
         return [(*ts[0][:3], blocks.tobytes())] + ts[1:]
 
-    g = _upload(block, tmp_path, 64, dims, 11, route)
+    g = _upload(block, tmp_path, 64, dims, ty, route)
     rng = np.random.default_rng(5)
-    owner = rng.permutation(np.repeat(np.arange(11), sizes))
+    owner = rng.permutation(np.repeat(np.arange(n), sizes))
     x = rng.standard_normal((owner.size, 256)).astype(np.float32)
     x[np.arange(owner.size), owner] = 6.0
-    x[:, :11] = np.minimum(x[:, :11], 6.0)
+    x[:, :n] = np.minimum(x[:, :n], 6.0)
     _, ids = _check(block, oracle, g, 64, dims, x)
-    assert np.array_equal(np.bincount(ids.reshape(-1), minlength=11), sizes)
+    assert np.array_equal(np.bincount(ids.reshape(-1), minlength=n), sizes)
     block.free_layer_gguf(64)
 
 

@@ -97,10 +97,9 @@ def test_qwen_shape_q3_k(block, oracle, qwen_gguf):
 
 
 def test_many_tokens_grouped_qwen_shape(block, oracle, qwen_gguf):
-    """130 tokens on 16 experts: the grouped form's big units (more than 32
-    of an expert's tokens, the shared expert's 128 + 2) and small units,
-    against the oracle, and rows equal to the same tokens computed alone,
-    bit for bit."""
+    """130 tokens on 16 experts: the grouped form's units of eight tokens and
+    their remainders (the shared expert's 16 x 8 + 2), against the oracle, and
+    rows equal to the same tokens computed alone, bit for bit."""
     dims = (2048, 16, 8, 512, 512)
     with gguf.parse_gguf_index(qwen_gguf) as g:
         block.upload_layer_gguf(22, dims, g, model_layer=3)

@@ -16,6 +16,11 @@ SHAPES = [
     ((1040, 64, 2, 48, 80), 60),     # units of four, most of one or two tokens
     ((2048, 9, 3, 640, 128), 9),     # two chunks in every row, a few tokens
     ((256, 16, 4, 128, 512), 130),   # a quarter of a wave's chunk per row
+    # without the blocked kernels: grouped from 128 tokens
+    ((264, 6, 2, 64, 96), 130),      # rows of eight weights per lane, units of eight
+    ((264, 80, 1, 64, 96), 130),     # and of four
+    ((2304, 6, 2, 64, 64), 130),     # hidden above 2048
+    ((256, 6, 2, 1088, 128), 130),   # inter above 1024: blocked gate/up, down not
 ]
 
 
