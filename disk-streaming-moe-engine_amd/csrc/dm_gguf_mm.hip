@@ -832,7 +832,7 @@ hipError_t launch_gguf_tiles(const GgufMoeDev& L, uint8_t* out, hipStream_t st) 
 int gguf_mm_tok(const GgufMoeDev& L) { return mm_tok(L.type); }
 
 bool gguf_mm_ok(const GgufMoeDev& L, int T) {
-  // (2^32 parts and more: not measured, the grouped form)
+  // (calls of 2^31 activations and more: not measured, the grouped form)
   const uint64_t n = L.I > L.Ish ? L.I : L.Ish;
   return gguf_tiles_bytes(L) && T >= kGgufMmMinT && 2ull * T * L.H < (1ull << 32) &&
          2ull * T * L.K * n < (1ull << 32);
